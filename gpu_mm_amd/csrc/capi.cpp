@@ -1052,7 +1052,7 @@ int gmm_unplanned_tod2map(float *local_map_gpu, int64_t local_map_size,
         OpArgs a{lpix, tod_nsamp, partial_pixelization != 0};
         launch_unplanned_tod2map(local_map_gpu, tod_gpu, xpointing_gpu, a, errflags_gpu, nerrflags, stream);
         if (check_errors)
-            check_unplanned_errflags(errflags_gpu, unplanned_nblocks(tod_nsamp, nerrflags), where, stream);
+            check_unplanned_errflags(errflags_gpu, unplanned_tod2map_nblocks(tod_nsamp, nerrflags), where, stream);
     });
 }
 

@@ -189,6 +189,17 @@ __device__ inline void sincos_angle(float x, float &s, float &c)
     sincos_reduced(float(rd), int(jd - 4.0 * floor(jd * 0.25)), s, c);
 }
 
+// sin and cos of x0 + d from s0 = sin x0, c0 = cos x0 for |d| <= 0.0185, where cos d = 1 - d^2/2
+// and sin d = d (1 - d^2/6) are exact to float rounding (the bound of the table's reduction).
+__device__ inline void angle_step(float s0, float c0, float d, float &sn, float &cs)
+{
+    const float z = d * d;
+    const float cd = fmaf(z, -0.5f, 1.0f);
+    const float sd = d * fmaf(z, -0.16666667f, 1.0f);
+    sn = fmaf(s0, cd, c0 * sd);
+    cs = fmaf(c0, cd, -(s0 * sd));
+}
+
 // The (up to four) distinct cells touched by the bilinear footprint of one sample, as
 // cell keys; duplicates within the sample are replaced by NO_CELL.
 constexpr uint32_t NO_CELL = 0xffffffffu;

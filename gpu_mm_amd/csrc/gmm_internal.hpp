@@ -283,7 +283,9 @@ void launch_tod16_encode(void *out, int tod_type, float *scale, const float *tod
                          int64_t row_len, int error_feedback, hipStream_t stream);
 // Words of tod2map scratch kept in the plan buffer.
 
+// Blocks (error words written) of the plan-free launches.
 int64_t unplanned_nblocks(int64_t nsamp, int64_t max_blocks);
+int64_t unplanned_tod2map_nblocks(int64_t nsamp, int64_t max_blocks);
 void launch_unplanned_map2tod(float *tod, const float *lmap, const float *xp, const OpArgs &a,
                               uint32_t *errflags, int64_t nblocks, bool accum, hipStream_t stream);
 void launch_unplanned_tod2map(float *lmap, const float *tod, const float *xp, const OpArgs &a,

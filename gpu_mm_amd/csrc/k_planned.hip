@@ -803,17 +803,6 @@ __device__ inline void angle_step_tiny(float s0, float c0, float d, float &sn, f
     cs = fmaf(-d, s0, c0);
 }
 
-// sin and cos of x0 + d from s0 = sin x0, c0 = cos x0 for |d| <= 0.0185, where cos d = 1 - d^2/2
-// and sin d = d (1 - d^2/6) are exact to float rounding (the bound of the table's reduction).
-__device__ inline void angle_step(float s0, float c0, float d, float &sn, float &cs)
-{
-    const float z = d * d;
-    const float cd = fmaf(z, -0.5f, 1.0f);
-    const float sd = d * fmaf(z, -0.16666667f, 1.0f);
-    sn = fmaf(s0, cd, c0 * sd);
-    cs = fmaf(c0, cd, -(s0 * sd));
-}
-
 // Per-sample state of a 4-sample group in fixed-point tod2map: tile-local corner (ly, lx), offsets
 // (dy, dx), whether the block evaluates the sample (own), its T value and its polarized value
 // before the angle factor (ts, ps: zero when not evaluated), and its angle.
