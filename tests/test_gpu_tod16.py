@@ -1,0 +1,61 @@
+"""The 16-bit encoder, bit for bit against its definition in numpy float32: row scale, 256 error-feedback
+runs per row, and the row lengths, row counts and alignments at which its staging changes form.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+F32 = np.float32
+HALF_MAX = {torch.float16: 32752.0, torch.bfloat16: float.fromhex("0x1.fep126")}
+
+
+def round16(v, dtype):
+    return torch.from_numpy(np.ascontiguousarray(v)).to(dtype)
+
+
+def encode(tod, dtype, order):
+    nrows, n = tod.shape
+    scale = np.maximum(np.abs(tod).max(axis=1) / F32(HALF_MAX[dtype]), np.finfo(F32).tiny).astype(F32)
+    with np.errstate(over="ignore"):
+        x = tod / scale[:, None]
+    if order == 0:
+        return round16(x, dtype), scale
+    run = -(-n // 256)
+    pad = np.zeros((nrows, 256 * run), F32)
+    pad[:, :n] = x
+    x = pad.reshape(nrows * 256, run)
+    out = torch.empty(x.shape, dtype=dtype)
+    e1 = np.zeros(x.shape[0], F32)
+    e2 = e1.copy()
+    for i in range(run):
+        v = x[:, i] + (e1 if order == 1 else F32(2) * e1 - e2)
+        out[:, i] = round16(v, dtype)
+        e2, e1 = e1, v - out[:, i].float().numpy()
+    return out.reshape(nrows, 256 * run)[:, :n].contiguous(), scale
+
+
+# One block per row (short rows, or at least 256 rows) and several; runs of one sample, of whole tiles
+# of 32, of tiles and a rest; lengths that are no multiple of 4; a last group of runs that is cut short.
+SHAPES = [(1, 1), (3, 5), (2, 255), (2, 257), (1, 8192), (2, 8448), (300, 421), (257, 1024), (1, 16384), (1, 16388),
+          (3, 20000), (2, 33001), (5, 65536)]
+
+
+@pytest.mark.parametrize("order", [0, 1, 2])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: f"{s[0]}x{s[1]}")
+def test_encode_bits(gmm, dev, shape, dtype, order):
+    rng = np.random.default_rng(shape[0] * 7 + shape[1])
+    tod = (rng.standard_normal(shape) * np.exp(rng.uniform(-12, 12, (shape[0], 1)))).astype(F32)
+    tod[0, ::5] = 0.0
+    tod[-1, ::3] *= F32(1e-30)               # quotients that a reciprocal may not give exactly
+    ref, scale = encode(tod, dtype, order)
+    for offset in (0, 1):                    # 16-byte aligned input or not
+        buf = torch.empty(tod.size + offset, dtype=torch.float32, device=dev)
+        src = buf[offset:].view(shape)
+        src.copy_(torch.from_numpy(tod))
+        got, sc = gmm.encode_tod16(src, dtype, error_feedback=order)
+        assert np.array_equal(sc.cpu().numpy(), scale)
+        assert torch.equal(got.cpu().view(torch.int16), ref.view(torch.int16))
