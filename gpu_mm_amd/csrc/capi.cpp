@@ -582,19 +582,19 @@ int gmm_plan_create(gmm_plan **out, const gmm_preplan *pp, const float *xpointin
             const int64_t scratch_nbytes = pp->sort_nbytes - 128;
             uint32_t *counts = reinterpret_cast<uint32_t *>(scratch + scratch_nbytes);
 
-            launch_fill_u32(plan->err, pp->n_err, 0u, stream);
+            uint32_t *err_word = plan->err + (pp->n_err - 1);
             launch_plan_emit(xpointing_gpu, *pp, a, plan->err, stream);
-            launch_reduce_or(plan->err, pp->pparams.planner_nblocks, plan->err + (pp->n_err - 1), stream);
-            plan_sort(*pp, a, b, plan->plan_mt, scratch, scratch_nbytes, stream);
+            launch_plan_errors(plan->err, pp->pparams.planner_nblocks, err_word, counts, stream);
+            plan_sort(*pp, a, b, plan->plan_mt, plan->qmask, scratch, scratch_nbytes, stream);
             plan_schedule(*pp, plan->plan_mt, xpointing_gpu, plan->chunks, plan->qmask, counts, scratch, scratch_nbytes,
                           stream);
 
-            uint32_t h[2];
+            uint32_t h[3];                                  // chunks, multi-cell lines, error bits
             GMM_HIP(hipMemcpyAsync(h, counts, sizeof(h), hipMemcpyDeviceToHost, stream));
-            uint32_t e = read_word(plan->err + (pp->n_err - 1), stream);
-            if (e) {
-                clear_word(plan->err + (pp->n_err - 1), stream);
-                throw_errflags(e, where);
+            GMM_HIP(hipStreamSynchronize(stream));
+            if (h[2]) {
+                clear_word(err_word, stream);
+                throw_errflags(h[2], where);
             }
             plan->nchunks = h[0];
             plan->nmlines = h[1];

@@ -127,15 +127,21 @@ void launch_preplan_count(const float *xp, int64_t nsamp, const gmm_preplan &pp,
 void launch_preplan_finish(uint32_t *nmt, const uint32_t *err, int64_t nblocks,
                            uint32_t *summary_gpu, hipStream_t stream);
 
+// Entries in line order, with their owned-quad masks in bits 48..63; err_out[b]: error bits of planner
+// block b and, above them, its number of lines that touch several cells.
 void launch_plan_emit(const float *xp, const gmm_preplan &pp, uint64_t *out_mt,
                       uint32_t *err_out, hipStream_t stream);
 
-// Sorts plan entries by cell (stable), ping-ponging between a and b, result in 'out'.
-void plan_sort(const gmm_preplan &pp, uint64_t *a, uint64_t *b, uint64_t *out,
+// Gathers these words: error bits to *err_word and counts[2], multi-cell lines to counts[1].
+void launch_plan_errors(const uint32_t *in, int64_t nblocks, uint32_t *err_word, uint32_t *counts, hipStream_t stream);
+
+// Sorts plan entries by cell (stable), ping-ponging between a and b; the entries go to 'out', their
+// masks to 'qmask'.
+void plan_sort(const gmm_preplan &pp, uint64_t *a, uint64_t *b, uint64_t *out, uint16_t *qmask,
                void *scratch, int64_t scratch_nbytes, hipStream_t stream);
 
-// Builds the chunk list and the multi-cell line list from the sorted plan. Writes the
-// two counts to counts_gpu[0], counts_gpu[1].
+// Builds the chunk list from the sorted plan (their number goes to counts_gpu[0]) and the masks that
+// the emit pass left pending.
 void plan_schedule(const gmm_preplan &pp, const uint64_t *sorted_mt, const float *xp, Chunk *chunks,
                    uint16_t *qmask, uint32_t *counts_gpu, void *scratch,
                    int64_t scratch_nbytes, hipStream_t stream);
@@ -150,9 +156,6 @@ int64_t plan_scratch_nbytes(const gmm_preplan &pp);
 
 // Fills n words with v (a kernel, so it is safe inside captured graphs).
 void launch_fill_u32(uint32_t *p, int64_t n, uint32_t v, hipStream_t stream);
-
-// OR-reduce n words into out[0].
-void launch_reduce_or(const uint32_t *in, int64_t n, uint32_t *out, hipStream_t stream);
 
 // Quantize kernel for the plan tester (src_lib/PointingPlanTester.cu:23-63).
 void launch_quantize(const float *xp, int64_t nsamp, int ny, int nx, bool periodic,

@@ -7,6 +7,7 @@
 
 #include "gmm_internal.hpp"
 #include "gmm_locate.hpp"
+#include "gmm_wave.hpp"
 
 namespace gmm {
 
@@ -17,18 +18,6 @@ constexpr int WAVE = 64;
 __device__ inline int lane_id() { return threadIdx.x & 63; }
 
 __device__ inline uint64_t lanemask_lt() { return (1ull << lane_id()) - 1ull; }
-
-// Inclusive scan across a wave.
-__device__ inline uint32_t wave_inclusive_scan(uint32_t v)
-{
-    const int lane = lane_id();
-#pragma unroll
-    for (int off = 1; off < WAVE; off <<= 1) {
-        uint32_t t = __shfl_up(v, off, WAVE);
-        v += (lane >= off) ? t : 0u;
-    }
-    return v;
-}
 
 __device__ inline uint32_t wave_reduce_or(uint32_t v)
 {
@@ -52,7 +41,7 @@ __device__ inline uint32_t block_exclusive_scan(uint32_t v, uint32_t *s_wave, ui
 {
     constexpr int NW = NT / WAVE;
     const int lane = lane_id(), wave = threadIdx.x / WAVE;
-    uint32_t inc = wave_inclusive_scan(v);
+    uint32_t inc = wave_inclusive_sum(v);
     if (lane == WAVE - 1)
         s_wave[wave] = inc;
     __syncthreads();
@@ -93,22 +82,6 @@ __device__ inline bool extract_one(uint32_t k[4], uint32_t &c, bool &lo_hit, boo
     return true;
 }
 
-// Fast path of the extraction (the usual case, a line inside one cell): true (wave-uniform) when
-// in both halves every sample's footprint is the one cell of the half's first sample, k[0] of
-// lane 0 or 32. Then that cell, in 'c', is the half's only cell, the one extract_one() would
-// return first, and nlo / nhi count the halves whose line exists (first sample active).
-__device__ inline bool single_cell_halves(const uint32_t k[4], uint32_t &c, uint32_t &nlo, uint32_t &nhi)
-{
-    const uint32_t lo = __builtin_amdgcn_readlane(k[0], 0), hi = __builtin_amdgcn_readlane(k[0], 32);
-    c = (lane_id() < 32) ? lo : hi;
-    nlo = (lo != NO_CELL);
-    nhi = (hi != NO_CELL);
-    // Inactive lanes (past the end of a partial line, or of a line that does not exist) hold
-    // NO_CELL in every slot.
-    const bool one = ((k[1] & k[2] & k[3]) == NO_CELL) && (k[0] == c || k[0] == NO_CELL);
-    return __ballot(!one) == 0;
-}
-
 // The four corner indices of a sample's bilinear footprint (locate_pixel's,
 // include/gpu_mm_internals.hpp:124-164), located by locate_op with its range checks deferred to
 // 'chk'.
@@ -134,55 +107,220 @@ __device__ inline void sample_cells(float y, float x, const Geom &g, Checks &chk
 }
 
 // ------------------------------------------------------------------------------------------
+// Both passes over the pointing (count and emit) read a 32-sample line with eight lanes, four samples
+// each, a wave eight lines at a time. The cells of a line come from the range of its coordinates: trunc
+// and the shift to cells are monotonic, so the lowest corner's cell and the highest one's bound the
+// line, and when they are the same or neighbours along one axis, the line's cells are exactly these
+// (the lowest sample touches the one, the highest the other). A line that spans two cells along both
+// axes takes the union of its samples' corners in these 2 x 2 cells. Anything else (longer lines, the
+// wrap of periodic x) is found sample by sample, by repeated extraction.
+// Working through every sample's four corners, with ballots over them, took 68 and 101 instructions
+// per sample, 0.93 and 1.38 ms of VALU issue in the 1.01 and 1.62 ms of the passes on 2048x262144
+// samples. By ranges the count takes 0.63 ms (6.8 TB/s: the 4.3 GB it reads) and the emit 0.87 ms (at
+// most 50 instructions per sample, 0.68 ms; loading a step ahead spills and takes 0.98).
+
+constexpr int SCAN_LINES = 8;                 // lines per wave and load
+
+// One lane's four samples: the range of their coordinates as bit patterns of c + 0 (as in Checks: those
+// of valid coordinates are in the order of the numbers).
+struct QuadRange
+{
+    uint32_t ylo, yhi, xlo, xhi;
+};
+
+// y and x of the lane's samples: n (0..4) of them from p = the first one's y on (the first one's values
+// beyond n, zeros when n == 0). Non-temporal: each pass reads its pointing once (count 757 -> 635 us).
+template<bool Vec>
+__device__ inline void load_quad(const float *__restrict__ p, int64_t nsamp, int n, float (&y)[4], float (&x)[4])
+{
+    if (Vec) {
+        typedef float f4v __attribute__((ext_vector_type(4)));
+        f4v a = { 0.0f, 0.0f, 0.0f, 0.0f }, b = a;
+        if (n > 0) {
+            a = __builtin_nontemporal_load(reinterpret_cast<const f4v *>(p));
+            b = __builtin_nontemporal_load(reinterpret_cast<const f4v *>(p + nsamp));
+        }
+        y[0] = a.x; y[1] = a.y; y[2] = a.z; y[3] = a.w;
+        x[0] = b.x; x[1] = b.y; x[2] = b.z; x[3] = b.w;
+    }
+    else {
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int j = (k < n) ? k : 0;
+            y[k] = (n > 0) ? p[j] : 0.0f;
+            x[k] = (n > 0) ? p[nsamp + j] : 0.0f;
+        }
+    }
+}
+
+// Samples of lines [line, l1) that exist (the last line may be partial), at most 'cap': wave-uniform, so
+// that a lane's count is one clamp of the difference to its place.
+__device__ inline int samples_left(int64_t line, int64_t l1, int64_t nsamp, int cap)
+{
+    return int(max<int64_t>(0, min<int64_t>(cap, min(nsamp, l1 * LINE) - line * LINE)));
+}
+
+// x after the wrap of locate_op: in [0, nx] for every valid x.
+template<bool Periodic>
+__device__ inline float wrap_x(float x, const Geom &g)
+{
+    if (Periodic) {
+        x = (x >= 0.0f) ? x : (x + g.fnx);
+        x = (x <= g.fnx) ? x : (x - g.fnx);
+    }
+    return x;
+}
+
+__device__ inline void range4(const float (&v)[4], uint32_t &lo, uint32_t &hi)
+{
+    uint32_t b[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+        b[k] = __float_as_uint(v[k] + 0.0f);
+    lo = min(min(b[0], b[1]), min(b[2], b[3]));
+    hi = max(max(b[0], b[1]), max(b[2], b[3]));
+}
+
+// Range of a lane's samples, the checks of locate_op added to chk. x is left wrapped.
+template<bool Periodic>
+__device__ inline QuadRange quad_range(const float (&y)[4], float (&x)[4], bool on, const Geom &g, Checks &chk)
+{
+    if (Periodic) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            chk.px = fmaxf(chk.px, fmaxf(g.xlo - x[k], x[k] - g.xhi));
+            chk.pn += x[k];
+            x[k] = wrap_x<true>(x[k], g);
+        }
+    }
+    QuadRange r;
+    range4(y, r.ylo, r.yhi);
+    range4(x, r.xlo, r.xhi);
+    chk.uy = max(chk.uy, r.yhi);
+    if (!Periodic)
+        chk.ux = max(chk.ux, r.xhi);
+    if (!on) {
+        r.ylo = r.xlo = 0xffffffffu;
+        r.yhi = r.xhi = 0;
+    }
+    return r;
+}
+
+template<bool Periodic>
+__device__ inline int pixel_x(float x, const Geom &g) { return int(clamp0(x, Periodic ? g.fnx : g.fnx2)); }
+template<bool Periodic>
+__device__ inline int pixel_x(uint32_t bits, const Geom &g) { return pixel_x<Periodic>(__uint_as_float(bits), g); }
+__device__ inline int pixel_y(float y, const Geom &g) { return int(clamp0(y, g.fny2)); }
+__device__ inline int pixel_y(uint32_t bits, const Geom &g) { return pixel_y(__uint_as_float(bits), g); }
+
+// Cells of one line, the same in its eight lanes: bit 2 * r + c of 'at' stands for cell (cy + r,
+// cx + c). slow: found sample by sample instead (at = 0).
+struct LineCells
+{
+    int cy, cx;
+    int xhi;               // largest ix0 of the line
+    uint32_t at;
+    bool slow;
+};
+
+template<bool Periodic>
+__device__ inline LineCells line_cells(const QuadRange &q, const float (&y)[4], const float (&x)[4], bool on,
+                                       const Geom &g)
+{
+    auto umin = [](uint32_t a, uint32_t b) { return min(a, b); };
+    auto umax = [](uint32_t a, uint32_t b) { return max(a, b); };
+    const uint32_t ylo = group8_reduce(q.ylo, umin), yhi = group8_reduce(q.yhi, umax);
+    const uint32_t xlo = group8_reduce(q.xlo, umin), xhi = group8_reduce(q.xhi, umax);
+    LineCells l;
+    l.xhi = pixel_x<Periodic>(xhi, g);
+    l.cy = pixel_y(ylo, g) >> 6;
+    l.cx = pixel_x<Periodic>(xlo, g) >> 6;
+    const int dy = ((pixel_y(yhi, g) + 1) >> 6) - l.cy, dx = ((l.xhi + 1) >> 6) - l.cx;
+    // Periodic x: ix0 = nx - 1 (and x = nx, which is pixel 0) have a corner at ix = 0.
+    l.slow = (unsigned(dy) > 1u) || (unsigned(dx) > 1u) || (Periodic && l.xhi + 1 >= g.nx);
+    l.at = l.slow ? 0u : 1u | (uint32_t(dx) << 1) | (uint32_t(dy) << 2);
+    const bool both = !l.slow && dx + dy == 2;
+    if (__any(both)) {
+        uint32_t m = 0;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int iy = pixel_y(y[k], g), ix = pixel_x<Periodic>(x[k], g);
+            const int r0 = (iy >> 6) - l.cy, r1 = ((iy + 1) >> 6) - l.cy, c0 = (ix >> 6) - l.cx, c1 = ((ix + 1) >> 6) - l.cx;
+            const uint32_t cols = (1u << (c0 & 1)) | (1u << (c1 & 1));
+            m |= (cols << (2 * (r0 & 1))) | (cols << (2 * (r1 & 1)));
+        }
+        m = group8_reduce(on ? m : 0u, [](uint32_t a, uint32_t b) { return a | b; });
+        l.at = both ? m : l.at;
+    }
+    return l;
+}
+
+// Number of cells of a slow line of n samples from s0, by the whole wave: one sample per lane.
+template<bool Periodic, typename F>
+__device__ inline uint32_t slow_line(const float *__restrict__ xp, int64_t nsamp, int64_t s0, const Geom &g, F &&each)
+{
+    const int lane = lane_id();
+    const bool act = lane < 32 && s0 + lane < nsamp;
+    uint32_t k[4];
+    Checks unchecked;                          // the line's ranges were checked already
+    sample_cells<Periodic>(act ? xp[s0 + lane] : 0.0f, act ? xp[nsamp + s0 + lane] : 0.0f, g, unchecked, act, k);
+    uint32_t c, n = 0;
+    bool lo, hi;
+    while (extract_one(k, c, lo, hi)) {
+        each(n, __builtin_amdgcn_readfirstlane(c));
+        n++;
+    }
+    return n;
+}
+
+// ------------------------------------------------------------------------------------------
 // Preplan: number of distinct (line, cell) pairs per planner block
 // (src_lib/PointingPrePlan.cu:37-108 computes the same per-block counts).
 
 constexpr int PP_THREADS = 512;
-constexpr int PP_UNROLL = 4;
+constexpr int PP_UNROLL = 2;
 
-template<bool Periodic>
-__global__ void __launch_bounds__(PP_THREADS)
+template<bool Periodic, bool Vec>
+__global__ void __launch_bounds__(PP_THREADS) __attribute__((amdgpu_waves_per_eu(8)))
 preplan_count_kernel(const float *__restrict__ xp, int64_t nsamp, int64_t ncl, int64_t ncl_per_block,
                      int ny, int nx, uint32_t *__restrict__ nmt_out, uint32_t *__restrict__ err_out)
 {
     __shared__ uint32_t s_cnt[PP_THREADS / WAVE], s_err[PP_THREADS / WAVE];
-    const int lane = lane_id(), wave = threadIdx.x / WAVE;
+    const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     constexpr int NW = PP_THREADS / WAVE;
-    const int half = lane >> 5, sub = lane & 31;
+    const int q = lane & 7;
 
     const int64_t l0 = int64_t(blockIdx.x) * ncl_per_block;
     const int64_t l1 = min(ncl, l0 + ncl_per_block);
-    uint32_t cnt = 0;   // wave-uniform
+    uint32_t cnt = 0;                          // lanes q == 0: cells of the lane's lines
+    uint32_t slow_cnt = 0;                     // wave-uniform
     const Geom g = make_geom(ny, nx, Periodic);
     Checks chk;
 
-    for (int64_t lb = l0 + 2 * wave; lb < l1; lb += 2 * NW * PP_UNROLL) {
-        float y[PP_UNROLL], x[PP_UNROLL];
-        bool act[PP_UNROLL];
+    for (int64_t lb = l0 + SCAN_LINES * wave; lb < l1; lb += SCAN_LINES * NW * PP_UNROLL) {
+        float y[PP_UNROLL][4], x[PP_UNROLL][4];
+        int n[PP_UNROLL];
 #pragma unroll
         for (int u = 0; u < PP_UNROLL; u++) {
-            int64_t line = lb + 2 * NW * u + half;
-            int64_t s = line * LINE + sub;
-            act[u] = (line < l1) && (s < nsamp);        // the last line may be partial
-            y[u] = act[u] ? xp[s] : 0.0f;
-            x[u] = act[u] ? xp[s + nsamp] : 0.0f;
+            const int64_t line = lb + SCAN_LINES * NW * u;         // the wave's first line of the group
+            n[u] = min(max(samples_left(line, l1, nsamp, SCAN_LINES * LINE) - 4 * lane, 0), 4);
+            load_quad<Vec>(xp + line * LINE + 4 * lane, nsamp, n[u], y[u], x[u]);
         }
 #pragma unroll
         for (int u = 0; u < PP_UNROLL; u++) {
-            uint32_t k[4];
-            sample_cells<Periodic>(y[u], x[u], g, chk, act[u], k);
-            uint32_t c, nlo, nhi;
-            if (single_cell_halves(k, c, nlo, nhi)) {
-                cnt += nlo + nhi;
-                continue;
+            const QuadRange r = quad_range<Periodic>(y[u], x[u], n[u] > 0, g, chk);
+            const LineCells l = line_cells<Periodic>(r, y[u], x[u], n[u] > 0, g);
+            const bool lead = (q == 0) && n[u] > 0;
+            cnt += lead ? uint32_t(__popc(l.at)) : 0u;
+            for (uint64_t m = __ballot(lead && l.slow); m; m &= m - 1) {
+                const int64_t line = lb + SCAN_LINES * NW * u + (__builtin_ctzll(m) >> 3);
+                slow_cnt += slow_line<Periodic>(xp, nsamp, line * LINE, g, [](uint32_t, uint32_t) {});
             }
-            bool lo, hi;
-            while (extract_one(k, c, lo, hi))
-                cnt += uint32_t(lo) + uint32_t(hi);
         }
     }
 
-    uint32_t err = wave_reduce_or(chk.bits(g));
+    const uint32_t err = wave_reduce_or(chk.bits(g));
+    cnt = wave_reduce_add(cnt) + slow_cnt;
     if (lane == 0) {
         s_cnt[wave] = cnt;
         s_err[wave] = err;
@@ -231,27 +369,31 @@ preplan_finish_kernel(uint32_t *nmt, uint32_t *err, int nblocks)
 
 // ------------------------------------------------------------------------------------------
 // Emit: writes the plan entries of each planner block into its window
-// [nmt_cumsum[b-1], nmt_cumsum[b]) in line order; inside a line, cells come in extraction order
-// (lowest lane first), which makes the output deterministic. The entry layout and the
-// consistency check against the preplan count follow src_lib/PointingPlan.cu:75-89, 116, 227.
+// [nmt_cumsum[b-1], nmt_cumsum[b]) in line order; inside a line in an order that the sort by cell
+// replaces. The entry layout and the consistency check against the preplan count follow
+// src_lib/PointingPlan.cu:75-89, 116, 227. Bits 48..63 carry the entry's owned-quad mask through the
+// sort (its last pass stores it apart): the ranges give it for lines of one or two cells, others are
+// marked QM_PENDING and done by qmask_kernel afterwards.
 
 constexpr int EM_THREADS = 512;
 constexpr int EM_NW = EM_THREADS / WAVE;
-constexpr int EM_U = 2;                       // line pairs per wave per step
-constexpr int EM_LINES = 2 * EM_NW * EM_U;    // lines per block step (32)
+constexpr int EM_LINES = SCAN_LINES * EM_NW;           // lines per block step (64; 128 measure the same)
+constexpr uint16_t QM_PENDING = 0x8000;
+constexpr int QM_SHIFT = 48;
+constexpr int NML_SHIFT = 8;
 
 // At most 64 VGPRs (8 waves per SIMD, 4 blocks per CU): the planner grid (1024 blocks at most)
 // is then resident at once on 256 CUs instead of leaving a tail.
-template<bool Periodic>
+template<bool Periodic, bool Vec>
 __global__ void __launch_bounds__(EM_THREADS) __attribute__((amdgpu_waves_per_eu(8)))
 plan_emit_kernel(const float *__restrict__ xp, int64_t nsamp, int64_t ncl, int64_t ncl_per_block,
                  int ny, int nx, const uint32_t *__restrict__ nmt_cumsum,
                  uint64_t *__restrict__ out, uint32_t *__restrict__ err_out)
 {
-    __shared__ uint32_t s_counts[2][EM_LINES];
-    __shared__ uint32_t s_err[EM_NW];
-    const int lane = lane_id(), wave = threadIdx.x / WAVE;
-    const int half = lane >> 5, sub = lane & 31;
+    __shared__ uint32_t s_total[2][EM_NW];
+    __shared__ uint32_t s_err[EM_NW], s_nml[EM_NW];
+    const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const int li = lane >> 3, q = lane & 7;
     const int b = blockIdx.x;
 
     const int64_t l0 = int64_t(b) * ncl_per_block;
@@ -262,92 +404,97 @@ plan_emit_kernel(const float *__restrict__ xp, int64_t nsamp, int64_t ncl, int64
 
     uint32_t err = 0;
     uint32_t running = 0;   // entries written by earlier steps (block-uniform)
+    uint32_t nml = 0;       // multi-cell lines (wave-uniform)
     const Geom g = make_geom(ny, nx, Periodic);
     Checks chk;
     int parity = 0;
 
     for (int64_t ls = l0; ls < l1; ls += EM_LINES) {
-        float y[EM_U], x[EM_U];
-        bool act[EM_U];
-        int64_t line[EM_U];
-#pragma unroll
-        for (int u = 0; u < EM_U; u++) {
-            line[u] = ls + 2 * (wave * EM_U + u) + half;
-            int64_t s = line[u] * LINE + sub;
-            act[u] = (line[u] < l1) && (s < nsamp);     // the last line may be partial
-            y[u] = act[u] ? xp[s] : 0.0f;
-            x[u] = act[u] ? xp[s + nsamp] : 0.0f;
+        const int64_t lw = ls + SCAN_LINES * wave;         // the wave's first line
+        const int n = min(max(samples_left(lw, l1, nsamp, SCAN_LINES * LINE) - 4 * lane, 0), 4);
+        float y[4], x[4];
+        load_quad<Vec>(xp + lw * LINE + 4 * lane, nsamp, n, y, x);
+
+        const bool on = n > 0, lead = (q == 0) && on;
+        const QuadRange r = quad_range<Periodic>(y, x, on, g, chk);
+        const LineCells l = line_cells<Periodic>(r, y, x, on, g);
+        const uint64_t slow = __ballot(lead && l.slow);
+        const uint64_t present = __ballot(on);
+        const int shift = lane & ~7;
+        const uint32_t quads = uint32_t(present >> shift) & 0xffu;
+        // Lanes q < 4 write the line's cell number q, if it is one; its first sample's cell carries the
+        // zflag.
+        const uint32_t at = (quads & 1u) ? l.at : 0u;
+        uint32_t cnt = lead ? uint32_t(__popc(at)) : 0u;
+        uint32_t m = quads, z = 0;                          // owned quads of the lane's entry, its flags
+        if (__any(at > 1u)) {
+            // Two cells side by side: the left one evaluates all when the right one's samples (if it
+            // owns any) lie in its halo; else, and for two cells in a column, each its own (the rule of
+            // qmask_kernel).
+            const bool xpair = at == 3u, ypair = at == 5u;
+            const bool owns = (l.xhi >> 6) == l.cx + 1, takes = xpair && owns && (l.xhi & 63) <= HALO_X - 2;
+            const bool each = ypair || (xpair && owns && !takes);
+            if (at > 1u)
+                m = (xpair && q == 0) ? (quads | (takes ? QM_TAKES_RIGHT : 0u)) : (xpair ? 0u : QM_PENDING);
+            if (__any(each)) {
+                const int ixlo = pixel_x<Periodic>(r.xlo, g), ixhi = pixel_x<Periodic>(r.xhi, g);
+                const int iylo = pixel_y(r.ylo, g), iyhi = pixel_y(r.yhi, g);
+                const bool first = on && (xpair ? (ixlo >> 6) == l.cx : (iylo >> 6) == l.cy);
+                const bool second = on && (xpair ? (ixhi >> 6) == l.cx + 1 : (iyhi >> 6) == l.cy + 1);
+                const uint32_t qa = uint32_t(__ballot(first) >> shift) & 0xffu, qb = uint32_t(__ballot(second) >> shift) & 0xffu;
+                m = each ? ((q == 0) ? qa : qb) : m;
+            }
+            const uint32_t zc = uint32_t(2 * ((pixel_y(y[0], g) >> 6) - l.cy) + ((pixel_x<Periodic>(x[0], g) >> 6) - l.cx));
+            const bool zf = dpp<DPP_QUAD0>(zc) == uint32_t(q);
+            z = (at > 1u) ? (uint32_t(MFLAG >> 32) | (zf ? uint32_t(ZFLAG >> 32) : 0u)) : 0u;
+            nml += uint32_t(__popcll(__ballot(lead && at > 1u)));
+        }
+        for (uint64_t sm = slow; sm; sm &= sm - 1) {
+            const int src = __builtin_ctzll(sm);
+            const uint32_t c = slow_line<Periodic>(xp, nsamp, (lw + (src >> 3)) * LINE, g, [](uint32_t, uint32_t) {});
+            cnt = (lane == src) ? c : cnt;
+            nml += (c > 1) ? 1u : 0u;
         }
 
-        uint32_t mycell[EM_U], nmy[EM_U];
-#pragma unroll
-        for (int u = 0; u < EM_U; u++) {
-            uint32_t k[4];
-            sample_cells<Periodic>(y[u], x[u], g, chk, act[u], k);
-            uint32_t c, nlo, nhi;
-            mycell[u] = NO_CELL;
-            if (single_cell_halves(k, c, nlo, nhi)) {
-                mycell[u] = (sub == 0) ? c : NO_CELL;
-            }
-            else {
-                nlo = nhi = 0;
-                bool lo, hi;
-                while (extract_one(k, c, lo, hi)) {
-                    uint32_t j = half ? nhi : nlo;
-                    mycell[u] = (uint32_t(sub) == j) ? c : mycell[u];
-                    nlo += lo;
-                    nhi += hi;
-                }
-            }
-            nmy[u] = half ? nhi : nlo;
-            if (sub == 0)
-                s_counts[parity][2 * (wave * EM_U + u) + half] = nmy[u];
-        }
+        // Offsets of the wave's lines, then of the step's waves, in line order.
+        const uint32_t inc = wave_inclusive_sum(cnt);
+        if (lane == WAVE - 1)
+            s_total[parity][wave] = inc;
         __syncthreads();
-
-        // Exclusive offsets of this step's lines, in line order.
-        uint32_t cv = (lane < EM_LINES) ? s_counts[parity][lane] : 0u;
-        uint32_t inc = wave_inclusive_scan(cv);
-        uint32_t step_total = __shfl(inc, EM_LINES - 1, WAVE);
-        uint32_t excl = inc - cv;
-
+        uint32_t before = running, step_total = 0;
 #pragma unroll
-        for (int u = 0; u < EM_U; u++) {
-            int idx = 2 * (wave * EM_U + u) + half;
-            uint32_t off = running + __shfl(excl, idx, WAVE);
-            uint32_t n = nmy[u];
-            bool mflag = (n > 1);
-            if (act[u] && uint32_t(sub) < n) {
-                uint32_t pos = off + sub;
-                uint64_t mt = uint64_t(mycell[u]) | (uint64_t(line[u]) << ICL_SHIFT)
-                            | (mflag ? MFLAG : 0ull) | ((mflag && sub == 0) ? ZFLAG : 0ull);
-                if (pos < limit)
-                    out[pos] = mt;
-                else
-                    err |= ERR_INCONSISTENT_NMT;
-            }
-            // Lines touching more than 32 cells (not reachable by ordinary scans): the extra
-            // cells are re-extracted and written one at a time by the half's first lane.
-            uint64_t big = __ballot(n > 32);
-            if (big) {
-                uint32_t k[4];
-                sample_cells<Periodic>(y[u], x[u], g, chk, act[u], k);
-                uint32_t c, nlo = 0, nhi = 0;
-                bool lo, hi;
-                while (extract_one(k, c, lo, hi)) {
-                    uint32_t j = half ? nhi : nlo;
-                    if (sub == 0 && j >= 32 && c != NO_CELL) {
-                        uint32_t pos = off + j;
-                        uint64_t mt = uint64_t(c) | (uint64_t(line[u]) << ICL_SHIFT) | MFLAG;
-                        if (pos < limit)
-                            out[pos] = mt;
-                        else
-                            err |= ERR_INCONSISTENT_NMT;
-                    }
-                    nlo += lo;
-                    nhi += hi;
+        for (int w = 0; w < EM_NW; w++) {
+            const uint32_t t = s_total[parity][w];
+            before += (w < wave) ? t : 0u;
+            step_total += t;
+        }
+        // The line's offset: the sum up to its first lane less its own count.
+        const uint32_t off = before + __shfl(inc - cnt, lane & ~7, WAVE);
+
+        if (q < 4 && ((at >> q) & 1u)) {
+            const uint32_t pos = off + uint32_t(__popc(at & ((1u << q) - 1u)));
+            const uint64_t mt = (uint64_t((m << (QM_SHIFT - 32)) | z) << 32) | (uint64_t(lw + li) << ICL_SHIFT)
+                              | cell_key(l.cy + (q >> 1), l.cx + (q & 1));
+            if (pos < limit)
+                out[pos] = mt;
+            else
+                err |= ERR_INCONSISTENT_NMT;
+        }
+        for (uint64_t sm = slow; sm; sm &= sm - 1) {
+            const int src = __builtin_ctzll(sm);
+            const int64_t line = lw + (src >> 3);
+            const uint32_t soff = __builtin_amdgcn_readlane(off, src), c = __builtin_amdgcn_readlane(cnt, src);
+            slow_line<Periodic>(xp, nsamp, line * LINE, g, [&](uint32_t i, uint32_t key) {
+                // The first cell extracted is the first sample's.
+                const uint64_t mt = uint64_t(key) | (uint64_t(line) << ICL_SHIFT) | (uint64_t(QM_PENDING) << QM_SHIFT)
+                                  | ((c > 1) ? MFLAG : 0ull) | ((c > 1 && i == 0) ? ZFLAG : 0ull);
+                if (lane == 0) {
+                    if (soff + i < limit)
+                        out[soff + i] = mt;
+                    else
+                        err |= ERR_INCONSISTENT_NMT;
                 }
-            }
+            });
         }
 
         running += step_total;
@@ -358,14 +505,20 @@ plan_emit_kernel(const float *__restrict__ xp, int64_t nsamp, int64_t ncl, int64
         err |= ERR_INCONSISTENT_NMT;
 
     err = wave_reduce_or(err | chk.bits(g));
-    if (lane == 0)
+    if (lane == 0) {
         s_err[wave] = err;
+        s_nml[wave] = nml;
+    }
     __syncthreads();
     if (threadIdx.x == 0) {
-        uint32_t e = 0;
-        for (int w = 0; w < EM_NW; w++)
+        uint32_t e = 0, m = 0;
+        for (int w = 0; w < EM_NW; w++) {
             e |= s_err[w];
-        err_out[b] = e;
+            m += s_nml[w];
+        }
+        // The block's multi-cell lines above its error bits (at most 2^16 lines per block; a count that all
+        // blocks add to takes 10 us).
+        err_out[b] = e | (m << NML_SHIFT);
     }
 }
 
@@ -444,6 +597,16 @@ __device__ inline uint32_t dense_key(uint64_t mt, uint32_t kx)
     return (c >> 10) * kx + (c & 1023u);
 }
 
+__device__ inline void store_item(uint64_t *__restrict__ out, uint16_t *__restrict__ qmask, int64_t i, uint64_t item)
+{
+    if (qmask) {
+        out[i] = item & ((1ull << QM_SHIFT) - 1ull);
+        qmask[i] = uint16_t(item >> QM_SHIFT);
+    }
+    else
+        out[i] = item;
+}
+
 __global__ void __launch_bounds__(RS_THREADS)
 radix_hist_kernel(const uint64_t *__restrict__ in, int64_t n, uint32_t kx, int shift, uint32_t dmask,
                   uint32_t *__restrict__ hist, int64_t ntiles)
@@ -464,8 +627,9 @@ radix_hist_kernel(const uint64_t *__restrict__ in, int64_t n, uint32_t kx, int s
     hist[int64_t(threadIdx.x) * ntiles + blockIdx.x] = s_hist[threadIdx.x];
 }
 
+// With 'qmask' (the plan's last pass) the items are stored apart: the entry and its mask (bits 48..63).
 __global__ void __launch_bounds__(RS_THREADS)
-radix_scatter_kernel(const uint64_t *__restrict__ in, uint64_t *__restrict__ out, int64_t n,
+radix_scatter_kernel(const uint64_t *__restrict__ in, uint64_t *__restrict__ out, uint16_t *__restrict__ qmask, int64_t n,
                      uint32_t kx, int shift, int nbits, const uint32_t *__restrict__ hist_scanned,
                      int64_t ntiles)
 {
@@ -518,8 +682,16 @@ radix_scatter_kernel(const uint64_t *__restrict__ in, uint64_t *__restrict__ out
     for (int r = 0; r < RS_ROUNDS; r++) {
         int64_t j = w0 + int64_t(r) * WAVE + lane;
         if (j < n)
-            out[s_cnt[wave][dig[r]] + rank[r]] = item[r];
+            store_item(out, qmask, s_cnt[wave][dig[r]] + rank[r], item[r]);
     }
+}
+
+// One cell only: nothing to sort.
+__global__ void split_items_kernel(const uint64_t *__restrict__ in, uint64_t *__restrict__ out,
+                                   uint16_t *__restrict__ qmask, int64_t n)
+{
+    for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += int64_t(gridDim.x) * blockDim.x)
+        store_item(out, qmask, i, in[i]);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -589,21 +761,18 @@ __global__ void chunk_fill_kernel(const uint32_t *__restrict__ begin, const uint
 // X's own samples go left, so no block both gives and takes, and each sample has exactly one
 // evaluator; every entry of l computes these from the same 32 samples, so they agree. Bit q of
 // qmask[e] is set iff quad q (samples 4q..4q+3) holds a sample that Y evaluates; QM_TAKES_RIGHT
-// is R(l, Y). A line that lies in one cell gives all quads that hold a sample to it. Also counts
-// the multi-cell lines (one zflag entry each).
+// is R(l, Y). A line that lies in one cell gives all quads that hold a sample to it. Works on the
+// entries that plan_emit_kernel marked QM_PENDING (97 us on the 2048x262144 raster; 461 when it did all
+// of them, from 1.65 GB of pointing read again).
 template<bool Periodic>
 __global__ void __launch_bounds__(256)
 qmask_kernel(const uint64_t *__restrict__ mt, int64_t n, const float *__restrict__ xp, int64_t nsamp, int ny,
-             int nx, uint16_t *__restrict__ qmask, uint32_t *__restrict__ nmlines)
+             int nx, uint16_t *__restrict__ qmask)
 {
     // Each wave takes 64 entries at a time, one per lane. An entry of a single-cell line owns
     // every quad of its line that holds a sample: written directly. The entries of multi-cell
     // lines are listed in LDS and handled eight at a time, eight lanes each (one quad per lane).
-    __shared__ uint32_t s_nml;
     __shared__ uint32_t s_list[256 / WAVE][WAVE];
-    if (threadIdx.x == 0)
-        s_nml = 0;
-    __syncthreads();
     const int lane = lane_id(), wave = threadIdx.x / WAVE;
     const int g = lane >> 3, q = lane & 7;
     // The planner's passes have checked the pointing's range already.
@@ -616,12 +785,12 @@ qmask_kernel(const uint64_t *__restrict__ mt, int64_t n, const float *__restrict
     const int64_t nwaves = int64_t(gridDim.x) * (256 / WAVE);
     for (int64_t base = (int64_t(blockIdx.x) * (256 / WAVE) + wave) * WAVE; base < n; base += nwaves * WAVE) {
         const int64_t e = base + lane;
-        const uint64_t m = (e < n) ? mt[e] : 0ull;
-        const bool multi = (e < n) && (m & MFLAG);
-        const uint64_t z = __ballot((e < n) && (m & ZFLAG));
-        if (lane == 0 && z)
-            atomicAdd(&s_nml, uint32_t(__popcll(z)));
-        if (e < n && !multi) {
+        const bool pending = (e < n) && (qmask[e] & QM_PENDING);
+        if (!__any(pending))
+            continue;
+        const uint64_t m = pending ? mt[e] : 0ull;
+        const bool multi = pending && (m & MFLAG);
+        if (pending && !multi) {
             // Samples past the end of a partial last line do not exist.
             const int64_t s0 = int64_t(uint32_t(m >> ICL_SHIFT) & ICL_MASK) * LINE;
             const int64_t nv = max<int64_t>(0, min<int64_t>(LINE, nsamp - s0));
@@ -693,29 +862,33 @@ qmask_kernel(const uint64_t *__restrict__ mt, int64_t n, const float *__restrict
         // in issue order; the fence keeps the compiler from reordering them).
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
-    __syncthreads();
-    if (threadIdx.x == 0 && s_nml)
-        atomicAdd(nmlines, s_nml);
 }
 
 __global__ void copy_word_kernel(const uint32_t *src, uint32_t *dst) { *dst = *src; }
 
-__global__ void __launch_bounds__(1024)
-reduce_or_kernel(const uint32_t *__restrict__ in, int64_t n, uint32_t *__restrict__ out)
+// Error bits and multi-cell lines of the emit pass's blocks: the bits go to *err_word and counts[2],
+// the number of lines to counts[1]. One block.
+__global__ void __launch_bounds__(PREPLAN_SIZE)
+plan_errors_kernel(const uint32_t *__restrict__ in, int n, uint32_t *__restrict__ err_word, uint32_t *__restrict__ counts)
 {
-    __shared__ uint32_t s;
-    if (threadIdx.x == 0)
-        s = 0;
+    __shared__ uint32_t s_err[PREPLAN_SIZE / WAVE], s_nml[PREPLAN_SIZE / WAVE];
+    const uint32_t v = (int(threadIdx.x) < n) ? in[threadIdx.x] : 0u;
+    const uint32_t e = wave_reduce_or(v & ((1u << NML_SHIFT) - 1u)), m = wave_reduce_add(v >> NML_SHIFT);
+    if (lane_id() == 0) {
+        s_err[threadIdx.x / WAVE] = e;
+        s_nml[threadIdx.x / WAVE] = m;
+    }
     __syncthreads();
-    uint32_t v = 0;
-    for (int64_t i = threadIdx.x; i < n; i += blockDim.x)
-        v |= in[i];
-    v = wave_reduce_or(v);
-    if (lane_id() == 0 && v)
-        atomicOr(&s, v);
-    __syncthreads();
-    if (threadIdx.x == 0)
-        *out = s;
+    if (threadIdx.x == 0) {
+        uint32_t err = 0, nml = 0;
+        for (int w = 0; w < PREPLAN_SIZE / WAVE; w++) {
+            err |= s_err[w];
+            nml += s_nml[w];
+        }
+        *err_word = err;
+        counts[1] = nml;
+        counts[2] = err;
+    }
 }
 
 // ------------------------------------------------------------------------------------------
@@ -811,17 +984,21 @@ inline int grid_for(int64_t n, int threads, int64_t cap = 65536)
 // ==========================================================================================
 // Host launchers.
 
+// float4 access to every line's groups of four samples.
+static bool vec_pointing(const float *xp, int64_t nsamp)
+{
+    return (reinterpret_cast<uintptr_t>(xp) & 15) == 0 && nsamp % 4 == 0;
+}
+
 void launch_preplan_count(const float *xp, int64_t nsamp, const gmm_preplan &pp,
                           uint32_t *nmt_out, uint32_t *err_out, hipStream_t stream)
 {
     const auto &p = pp.pparams;
-    dim3 grid(unsigned(p.planner_nblocks)), block(PP_THREADS);
-    if (pp.periodic_xcoord)
-        preplan_count_kernel<true><<<grid, block, 0, stream>>>(xp, nsamp, p.ncl, p.ncl_per_threadblock,
-            int(pp.nypix_global), int(pp.nxpix_global), nmt_out, err_out);
-    else
-        preplan_count_kernel<false><<<grid, block, 0, stream>>>(xp, nsamp, p.ncl, p.ncl_per_threadblock,
-            int(pp.nypix_global), int(pp.nxpix_global), nmt_out, err_out);
+    const bool vec = vec_pointing(xp, nsamp);
+    auto k = pp.periodic_xcoord ? (vec ? preplan_count_kernel<true, true> : preplan_count_kernel<true, false>)
+                                : (vec ? preplan_count_kernel<false, true> : preplan_count_kernel<false, false>);
+    k<<<unsigned(p.planner_nblocks), PP_THREADS, 0, stream>>>(xp, nsamp, p.ncl, p.ncl_per_threadblock,
+        int(pp.nypix_global), int(pp.nxpix_global), nmt_out, err_out);
     GMM_HIP(hipGetLastError());
 }
 
@@ -836,13 +1013,11 @@ void launch_plan_emit(const float *xp, const gmm_preplan &pp, uint64_t *out_mt,
                       uint32_t *err_out, hipStream_t stream)
 {
     const auto &p = pp.pparams;
-    dim3 grid(unsigned(p.planner_nblocks)), block(EM_THREADS);
-    if (pp.periodic_xcoord)
-        plan_emit_kernel<true><<<grid, block, 0, stream>>>(xp, pp.nsamp, p.ncl, p.ncl_per_threadblock,
-            int(pp.nypix_global), int(pp.nxpix_global), pp.nmt_cumsum_gpu, out_mt, err_out);
-    else
-        plan_emit_kernel<false><<<grid, block, 0, stream>>>(xp, pp.nsamp, p.ncl, p.ncl_per_threadblock,
-            int(pp.nypix_global), int(pp.nxpix_global), pp.nmt_cumsum_gpu, out_mt, err_out);
+    const bool vec = vec_pointing(xp, pp.nsamp);
+    auto k = pp.periodic_xcoord ? (vec ? plan_emit_kernel<true, true> : plan_emit_kernel<true, false>)
+                                : (vec ? plan_emit_kernel<false, true> : plan_emit_kernel<false, false>);
+    k<<<unsigned(p.planner_nblocks), EM_THREADS, 0, stream>>>(xp, pp.nsamp, p.ncl, p.ncl_per_threadblock,
+        int(pp.nypix_global), int(pp.nxpix_global), pp.nmt_cumsum_gpu, out_mt, err_out);
     GMM_HIP(hipGetLastError());
 }
 
@@ -927,7 +1102,7 @@ void order_chunks(const gmm_preplan &pp, Chunk *chunks, int64_t nch, uint64_t *a
                                                                           L.ntiles);
         GMM_HIP(hipGetLastError());
         exclusive_scan_u32(hist, int64_t(1 << nb) * L.ntiles, sc + L.hist_scan_off, stream);
-        radix_scatter_kernel<<<unsigned(L.ntiles), RS_THREADS, 0, stream>>>(src, dst, nch, 1024u, shift, nb, hist,
+        radix_scatter_kernel<<<unsigned(L.ntiles), RS_THREADS, 0, stream>>>(src, dst, nullptr, nch, 1024u, shift, nb, hist,
                                                                              L.ntiles);
         GMM_HIP(hipGetLastError());
         std::swap(src, dst);
@@ -944,7 +1119,7 @@ int64_t plan_scratch_nbytes(const gmm_preplan &pp)
     return sort_layout(pp.plan_nmt, pp.nycells_g * pp.nxcells_g).total;
 }
 
-void plan_sort(const gmm_preplan &pp, uint64_t *a, uint64_t *b, uint64_t *out,
+void plan_sort(const gmm_preplan &pp, uint64_t *a, uint64_t *b, uint64_t *out, uint16_t *qmask,
                void *scratch, int64_t scratch_nbytes, hipStream_t stream)
 {
     const int64_t n = pp.plan_nmt;
@@ -956,7 +1131,8 @@ void plan_sort(const gmm_preplan &pp, uint64_t *a, uint64_t *b, uint64_t *out,
 
     const int bits = pp.key_bits;
     if (bits == 0) {
-        GMM_HIP(hipMemcpyAsync(out, a, size_t(n) * 8, hipMemcpyDeviceToDevice, stream));
+        split_items_kernel<<<grid_for(n, 256, 4096), 256, 0, stream>>>(a, out, qmask, n);
+        GMM_HIP(hipGetLastError());
         return;
     }
     const int npasses = (bits + RS_MAXBITS - 1) / RS_MAXBITS;
@@ -969,7 +1145,8 @@ void plan_sort(const gmm_preplan &pp, uint64_t *a, uint64_t *b, uint64_t *out,
         radix_hist_kernel<<<unsigned(L.ntiles), RS_THREADS, 0, stream>>>(src, n, kx, shift, (1u << nb) - 1u, hist, L.ntiles);
         GMM_HIP(hipGetLastError());
         exclusive_scan_u32(hist, int64_t(1 << nb) * L.ntiles, sc + L.hist_scan_off, stream);
-        radix_scatter_kernel<<<unsigned(L.ntiles), RS_THREADS, 0, stream>>>(src, dst, n, kx, shift, nb, hist, L.ntiles);
+        radix_scatter_kernel<<<unsigned(L.ntiles), RS_THREADS, 0, stream>>>(src, dst, (dst == out) ? qmask : nullptr, n,
+                                                                             kx, shift, nb, hist, L.ntiles);
         GMM_HIP(hipGetLastError());
         src = dst;
     }
@@ -1013,15 +1190,14 @@ void plan_schedule(const gmm_preplan &pp, const uint64_t *sorted_mt, const float
     build_chunks(sorted_mt, n, nkeys, uint32_t(pp.nxcells_g), uint32_t(pp.chunk_cap), chunks,
                  pp.max_nchunks, counts_gpu, sc, L, stream);
 
-    // Owned-quad masks and the multi-cell line count.
-    fill_u32_kernel<<<1, 64, 0, stream>>>(counts_gpu + 1, 1, 0u);
+    // The owned-quad masks that the emit pass left.
     const int grid = int(std::min<int64_t>((n + 255) / 256, 2048));
     if (pp.periodic_xcoord)
         qmask_kernel<true><<<grid, 256, 0, stream>>>(sorted_mt, n, xp, pp.nsamp, int(pp.nypix_global),
-                                                     int(pp.nxpix_global), qmask, counts_gpu + 1);
+                                                     int(pp.nxpix_global), qmask);
     else
         qmask_kernel<false><<<grid, 256, 0, stream>>>(sorted_mt, n, xp, pp.nsamp, int(pp.nypix_global),
-                                                      int(pp.nxpix_global), qmask, counts_gpu + 1);
+                                                      int(pp.nxpix_global), qmask);
     GMM_HIP(hipGetLastError());
 }
 
@@ -1054,9 +1230,9 @@ void launch_fill_u32(uint32_t *p, int64_t n, uint32_t v, hipStream_t stream)
     GMM_HIP(hipGetLastError());
 }
 
-void launch_reduce_or(const uint32_t *in, int64_t n, uint32_t *out, hipStream_t stream)
+void launch_plan_errors(const uint32_t *in, int64_t nblocks, uint32_t *err_word, uint32_t *counts, hipStream_t stream)
 {
-    reduce_or_kernel<<<1, 1024, 0, stream>>>(in, n, out);
+    plan_errors_kernel<<<1, PREPLAN_SIZE, 0, stream>>>(in, int(nblocks), err_word, counts);
     GMM_HIP(hipGetLastError());
 }
 
