@@ -480,14 +480,21 @@ int gmm_preplan_create(gmm_preplan **out, const float *xpointing_gpu, int64_t ns
         pp.nxcells_g = (nxpix_global + 63) / 64;
         const int64_t nkeys = pp.nycells_g * pp.nxcells_g;
         pp.key_bits = bits_for(nkeys);
-        int64_t cap = (nmt + 3071) / 3072;
-        pp.chunk_cap = std::min<int64_t>(8192, std::max<int64_t>(512, cap));
+        // Entries per work unit. map2tod: a block costs little (it stages its cell), and many small ones
+        // balance well. tod2map: every block clears and flushes a 116 KiB tile, atomically when its cell
+        // is split, and runs alone on its CU: about two blocks per CU at the least 1024 entries each
+        // (times with its own list against map2tod's: 299 / 480 us on 1.8e6 entries, 38 / 52 us on 1.4e5;
+        // map2tod takes 285 and 33 us with tod2map's list, 263 and 27 us with its own).
+        pp.chunk_cap = std::min<int64_t>(8192, std::max<int64_t>(512, (nmt + 3071) / 3072));
+        pp.chunk_cap_t2m = std::min<int64_t>(8192, std::max<int64_t>(1024, (nmt + 511) / 512));
         pp.max_nchunks = (nmt + pp.chunk_cap - 1) / pp.chunk_cap + std::min(nmt, nkeys);
-        pp.n_err = std::max<int64_t>(pp.pparams.planner_nblocks, pp.max_nchunks) + 1;
+        pp.max_nchunks_t2m = (nmt + pp.chunk_cap_t2m - 1) / pp.chunk_cap_t2m + std::min(nmt, nkeys);
+        pp.n_err = pp.pparams.planner_nblocks + 1;
 
         pp.off_err = align128(8 * nmt);
         pp.off_chunks = pp.off_err + align128(4 * pp.n_err);
-        pp.off_qmask = pp.off_chunks + align128(int64_t(sizeof(Chunk)) * pp.max_nchunks);
+        pp.off_chunks_t2m = pp.off_chunks + align128(int64_t(sizeof(Chunk)) * pp.max_nchunks);
+        pp.off_qmask = pp.off_chunks_t2m + align128(int64_t(sizeof(Chunk)) * pp.max_nchunks_t2m);
         pp.plan_nbytes = pp.off_qmask + align128(2 * nmt);
 
         pp.sort_nbytes = plan_scratch_nbytes(pp) + 128;
@@ -571,6 +578,7 @@ int gmm_plan_create(gmm_plan **out, const gmm_preplan *pp, const float *xpointin
         plan->plan_mt = reinterpret_cast<uint64_t *>(plan->buf);
         plan->err = reinterpret_cast<uint32_t *>(plan->buf + pp->off_err);
         plan->chunks = reinterpret_cast<Chunk *>(plan->buf + pp->off_chunks);
+        plan->chunks_t2m = reinterpret_cast<Chunk *>(plan->buf + pp->off_chunks_t2m);
         plan->qmask = reinterpret_cast<uint16_t *>(plan->buf + pp->off_qmask);
 
         try {
@@ -586,21 +594,22 @@ int gmm_plan_create(gmm_plan **out, const gmm_preplan *pp, const float *xpointin
             launch_plan_emit(xpointing_gpu, *pp, a, plan->err, stream);
             launch_plan_errors(plan->err, pp->pparams.planner_nblocks, err_word, counts, stream);
             plan_sort(*pp, a, b, plan->plan_mt, plan->qmask, scratch, scratch_nbytes, stream);
-            plan_schedule(*pp, plan->plan_mt, xpointing_gpu, plan->chunks, plan->qmask, counts, scratch, scratch_nbytes,
-                          stream);
+            const PlanLists lists = plan_lists(*pp, plan->chunks, plan->chunks_t2m, scratch);
+            plan_schedule(*pp, plan->plan_mt, xpointing_gpu, lists, plan->qmask, counts, stream);
 
-            uint32_t h[3];                                  // chunks, multi-cell lines, error bits
+            uint32_t h[PC_WORDS];
             GMM_HIP(hipMemcpyAsync(h, counts, sizeof(h), hipMemcpyDeviceToHost, stream));
             GMM_HIP(hipStreamSynchronize(stream));
-            if (h[2]) {
+            if (h[PC_ERROR]) {
                 clear_word(err_word, stream);
-                throw_errflags(h[2], where);
+                throw_errflags(h[PC_ERROR], where);
             }
-            plan->nchunks = h[0];
-            plan->nmlines = h[1];
-            GMM_REQUIRE(plan->nchunks <= pp->max_nchunks,
+            plan->nchunks = h[PC_CHUNKS_M2T];
+            plan->nchunks_t2m = h[PC_CHUNKS_T2M];
+            plan->nmlines = h[PC_NMLINES];
+            GMM_REQUIRE(plan->nchunks <= pp->max_nchunks && plan->nchunks_t2m <= pp->max_nchunks_t2m,
                         "PointingPlan constructor: work list larger than its bound (internal error)");
-            order_chunks(*pp, plan->chunks, plan->nchunks, a, b, scratch, scratch_nbytes, stream);
+            order_long_lists(*pp, lists, plan->nchunks, plan->nchunks_t2m, counts, a, b, scratch, stream);
             if (debug)
                 check_plan_invariants(*plan, where, stream);
         }
@@ -1167,9 +1176,8 @@ int gmm_test_plan_iterator(const uint64_t *plan_mt_cpu, int64_t nmt, int64_t nmt
                 fail(std::string(where) + ": plan_mt is not sorted by cell");
 
         const int64_t max_chunks = (nmt + nmt_per_block - 1) / nmt_per_block + std::min<int64_t>(nmt, int64_t(1) << 20);
-        const int64_t scratch = build_chunks_generic_scratch(nmt);
         const int64_t bytes = align128(8 * nmt) + align128(int64_t(sizeof(Chunk)) * max_chunks)
-                            + align128(4 * nmt) + 128 + scratch;
+                            + align128(4 * nmt) + 128;
         void *mem = nullptr;
         GMM_HIP(hipMalloc(&mem, size_t(bytes)));
         std::string failure;
@@ -1179,10 +1187,11 @@ int gmm_test_plan_iterator(const uint64_t *plan_mt_cpu, int64_t nmt, int64_t nmt
             Chunk *d_ch = reinterpret_cast<Chunk *>(m + align128(8 * nmt));
             uint32_t *d_vis = reinterpret_cast<uint32_t *>(m + align128(8 * nmt) + align128(int64_t(sizeof(Chunk)) * max_chunks));
             uint32_t *d_err = d_vis + nmt;
-            uint8_t *d_scr = m + align128(8 * nmt) + align128(int64_t(sizeof(Chunk)) * max_chunks) + align128(4 * nmt) + 128;
+            uint32_t *d_cnt = reinterpret_cast<uint32_t *>(m + align128(8 * nmt) + align128(int64_t(sizeof(Chunk)) * max_chunks)
+                                                           + align128(4 * nmt)) + 16;
             GMM_HIP(hipMemcpy(d_mt, plan_mt_cpu, size_t(nmt) * 8, hipMemcpyHostToDevice));
             GMM_HIP(hipMemset(d_vis, 0, size_t(nmt) * 4));
-            int64_t nch = build_chunks_generic(d_mt, nmt, nmt_per_block, d_ch, max_chunks, d_scr, scratch, nullptr);
+            int64_t nch = build_chunks_generic(d_mt, nmt, nmt_per_block, d_ch, max_chunks, d_cnt, nullptr);
             GMM_REQUIRE(nch <= max_chunks, "test_plan_iterator: chunk count exceeds bound");
             launch_iterator_test(d_mt, d_ch, nch, waves_per_block, d_vis, d_err, nullptr);
             std::vector<uint32_t> vis(static_cast<size_t>(nmt), 0u);

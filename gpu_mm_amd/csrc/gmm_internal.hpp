@@ -38,12 +38,13 @@ struct gmm_preplan
     // Derived sizes (computed once in the constructor).
     int64_t nycells_g = 0, nxcells_g = 0;  // cells of the global map
     int key_bits = 0;                      // bits of the dense cell key iycell*nxcells_g + ixcell
-    int64_t chunk_cap = 0;                 // max plan entries per operator work unit
-    int64_t max_nchunks = 0;
+    int64_t chunk_cap = 0;                 // max plan entries per map2tod work unit
+    int64_t chunk_cap_t2m = 0;             // ... per tod2map work unit
+    int64_t max_nchunks = 0, max_nchunks_t2m = 0;
     int64_t plan_nbytes = 0, tmp_nbytes = 0, sort_nbytes = 0;
 
     // Offsets inside the plan buffer.
-    int64_t off_err = 0, off_chunks = 0, off_qmask = 0, n_err = 0;
+    int64_t off_err = 0, off_chunks = 0, off_chunks_t2m = 0, off_qmask = 0, n_err = 0;
 };
 
 struct gmm_plan
@@ -52,9 +53,10 @@ struct gmm_plan
     uint8_t *buf = nullptr;         // caller-owned device buffer, >= pp.plan_nbytes
     uint64_t *plan_mt = nullptr;    // sorted plan entries
     uint32_t *err = nullptr;        // per-block error words (n_err of them)
-    gmm::Chunk *chunks = nullptr;   // operator work list
+    gmm::Chunk *chunks = nullptr;       // map2tod's work list
+    gmm::Chunk *chunks_t2m = nullptr;   // tod2map's
     uint16_t *qmask = nullptr;      // per entry: the quads of its line it evaluates (+ QM_TAKES_RIGHT)
-    int64_t nchunks = 0;
+    int64_t nchunks = 0, nchunks_t2m = 0;
     int64_t nmlines = 0;
 };
 
@@ -132,7 +134,8 @@ void launch_preplan_finish(uint32_t *nmt, const uint32_t *err, int64_t nblocks,
 void launch_plan_emit(const float *xp, const gmm_preplan &pp, uint64_t *out_mt,
                       uint32_t *err_out, hipStream_t stream);
 
-// Gathers these words: error bits to *err_word and counts[2], multi-cell lines to counts[1].
+// Gathers these words: error bits to *err_word and counts[PC_ERROR], multi-cell lines to
+// counts[PC_NMLINES]; clears the other counts.
 void launch_plan_errors(const uint32_t *in, int64_t nblocks, uint32_t *err_word, uint32_t *counts, hipStream_t stream);
 
 // Sorts plan entries by cell (stable), ping-ponging between a and b; the entries go to 'out', their
@@ -140,16 +143,25 @@ void launch_plan_errors(const uint32_t *in, int64_t nblocks, uint32_t *err_word,
 void plan_sort(const gmm_preplan &pp, uint64_t *a, uint64_t *b, uint64_t *out, uint16_t *qmask,
                void *scratch, int64_t scratch_nbytes, hipStream_t stream);
 
-// Builds the chunk list from the sorted plan (their number goes to counts_gpu[0]) and the masks that
-// the emit pass left pending.
-void plan_schedule(const gmm_preplan &pp, const uint64_t *sorted_mt, const float *xp, Chunk *chunks,
-                   uint16_t *qmask, uint32_t *counts_gpu, void *scratch,
-                   int64_t scratch_nbytes, hipStream_t stream);
+// Counts that plan construction brings back to the host.
+enum PlanCount { PC_CHUNKS_M2T = 0, PC_NMLINES = 1, PC_ERROR = 2, PC_CHUNKS_T2M = 3, PC_WORDS = 4 };
 
-// Reorders the work list (nch chunks, count known on the host) largest first; a and b are the
-// plan sort's ping-pong buffers, free after plan_sort().
-void order_chunks(const gmm_preplan &pp, Chunk *chunks, int64_t nch, uint64_t *a, uint64_t *b, void *scratch,
-                  int64_t scratch_nbytes, hipStream_t stream);
+// The operators' work lists: where they go, and the scratch in which they are made.
+struct PlanLists
+{
+    Chunk *m2t, *t2m;
+    Chunk *tmp_m2t, *tmp_t2m;
+    int64_t max_m2t, max_t2m;
+};
+PlanLists plan_lists(const gmm_preplan &pp, Chunk *m2t, Chunk *t2m, void *scratch);
+
+// Work lists of the sorted plan (their lengths go to counts_gpu) and the masks that the emit pass left
+// pending. Lists that may be longer than a ranking handles are left in the scratch for
+// order_long_lists(), which needs their lengths on the host.
+void plan_schedule(const gmm_preplan &pp, const uint64_t *sorted_mt, const float *xp, const PlanLists &l,
+                   uint16_t *qmask, uint32_t *counts_gpu, hipStream_t stream);
+void order_long_lists(const gmm_preplan &pp, const PlanLists &l, int64_t n_m2t, int64_t n_t2m, const uint32_t *counts_gpu,
+                      uint64_t *a, uint64_t *b, void *scratch, hipStream_t stream);
 
 // Size of the scratch used by plan_sort() + plan_schedule().
 int64_t plan_scratch_nbytes(const gmm_preplan &pp);
@@ -166,11 +178,9 @@ void launch_iterator_test(const uint64_t *plan_mt, const Chunk *chunks, int64_t 
                           int waves_per_block, uint32_t *visit_counts, uint32_t *err_word,
                           hipStream_t stream);
 
-// Builds chunks from an arbitrary cell-sorted plan (used by the iterator test).
+// Builds chunks from an arbitrary cell-sorted plan (used by the iterator test); counts: two words.
 int64_t build_chunks_generic(const uint64_t *plan_mt_gpu, int64_t nmt, int64_t chunk_cap,
-                             Chunk *chunks_gpu, int64_t max_chunks, void *scratch,
-                             int64_t scratch_nbytes, hipStream_t stream);
-int64_t build_chunks_generic_scratch(int64_t nmt);
+                             Chunk *chunks_gpu, int64_t max_chunks, uint32_t *counts, hipStream_t stream);
 
 // ------------------------------------------------------------------------------------------
 // Operator launchers (k_planned.hip, k_unplanned.hip).

@@ -9,7 +9,7 @@
 //   - entries sorted by cell, and inside a cell by line, each (cell, line) once;
 //   - every line index below ceil(nsamp/32); every line has an entry; mflag set on all entries of
 //     a multi-cell line and on none of a single-cell line; exactly one zflag per multi-cell line;
-//   - the operator work list covers every entry exactly once, each chunk within one cell.
+//   - each operator's work list covers every entry exactly once, each chunk within one cell.
 // Operator invariants (the planned operators' debug instantiations count into DebugBuffers):
 //   - each plan entry is walked by exactly one wave;
 //   - each sample is evaluated by exactly one block (sample ownership and the halo rule);
@@ -123,10 +123,10 @@ void check_plan_invariants(const gmm_plan &plan, const char *where, hipStream_t 
 {
     const int64_t nmt = plan.pp.plan_nmt;
     const uint32_t ncl = uint32_t((plan.pp.nsamp + 31) / 32);
-    DevBuf viol(8 * 4), lines(3 * int64_t(ncl) * 4), cover(nmt * 4);
+    DevBuf viol(8 * 4), lines(3 * int64_t(ncl) * 4), cover(2 * nmt * 4);
     GMM_HIP(hipMemsetAsync(viol.p, 0, 8 * 4, stream));
     GMM_HIP(hipMemsetAsync(lines.p, 0, size_t(3 * int64_t(ncl) * 4), stream));
-    GMM_HIP(hipMemsetAsync(cover.p, 0, size_t(std::max<int64_t>(nmt * 4, 4)), stream));
+    GMM_HIP(hipMemsetAsync(cover.p, 0, size_t(std::max<int64_t>(2 * nmt * 4, 4)), stream));
     uint32_t *n_ent = lines.u32(), *n_z = lines.u32(ncl), *n_m = lines.u32(2 * int64_t(ncl));
     if (nmt > 0)
         plan_entries_kernel<<<db_grid(nmt), DB_THREADS, 0, stream>>>(plan.plan_mt, nmt, ncl, n_ent, n_z, n_m, viol.u32());
@@ -136,9 +136,12 @@ void check_plan_invariants(const gmm_plan &plan, const char *where, hipStream_t 
     if (plan.nchunks > 0)
         chunk_cover_kernel<<<int(std::min<int64_t>(plan.nchunks, 8192)), DB_THREADS, 0, stream>>>(
             plan.chunks, plan.nchunks, plan.plan_mt, nmt, cover.u32(), viol.u32());
+    if (plan.nchunks_t2m > 0)
+        chunk_cover_kernel<<<int(std::min<int64_t>(plan.nchunks_t2m, 8192)), DB_THREADS, 0, stream>>>(
+            plan.chunks_t2m, plan.nchunks_t2m, plan.plan_mt, nmt, cover.u32(nmt), viol.u32());
     GMM_HIP(hipGetLastError());
     if (nmt > 0)
-        count_ne_kernel<<<db_grid(nmt), DB_THREADS, 0, stream>>>(cover.u32(), nmt, 1u, viol.u32(5));
+        count_ne_kernel<<<db_grid(2 * nmt), DB_THREADS, 0, stream>>>(cover.u32(), 2 * nmt, 1u, viol.u32(5));
     GMM_HIP(hipGetLastError());
     uint32_t v[8];
     GMM_HIP(hipMemcpyAsync(v, viol.p, sizeof(v), hipMemcpyDeviceToHost, stream));

@@ -695,7 +695,8 @@ __global__ void split_items_kernel(const uint64_t *__restrict__ in, uint64_t *__
 }
 
 // ------------------------------------------------------------------------------------------
-// Work list: per-cell [begin, end) in the sorted plan, cut into chunks of <= chunk_cap entries.
+// Work lists: per-cell [begin, end) in the sorted plan, cut into chunks of <= cap entries, one list per
+// operator. The chunks of a list come in no fixed order; rank_chunks_kernel puts them in theirs.
 
 __global__ void fill_u32_kernel(uint32_t *p, int64_t n, uint32_t v)
 {
@@ -703,52 +704,119 @@ __global__ void fill_u32_kernel(uint32_t *p, int64_t n, uint32_t v)
         p[i] = v;
 }
 
-// Entries whose cell lies outside the global map (only possible in a plan whose emit step
-// already reported an error) are skipped, so the tables are never indexed out of range.
-__global__ void cell_bounds_kernel(const uint64_t *__restrict__ mt, int64_t n, uint32_t kx, int64_t nkeys,
-                                   uint32_t *__restrict__ begin, uint32_t *__restrict__ end)
+// First entry of the sorted plan whose cell key is at least k.
+__device__ inline uint32_t key_lower_bound(const uint64_t *__restrict__ mt, int64_t n, uint32_t kx, uint32_t k)
 {
-    for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += int64_t(gridDim.x) * blockDim.x) {
-        uint32_t k = dense_key(mt[i], kx);
-        if (((uint32_t(mt[i]) & 1023u) >= kx) || int64_t(k) >= nkeys)
-            continue;
-        if (i == 0 || dense_key(mt[i - 1], kx) != k)
-            begin[k] = uint32_t(i);
-        if (i == n - 1 || dense_key(mt[i + 1], kx) != k)
-            end[k] = uint32_t(i + 1);
+    uint32_t lo = 0, hi = uint32_t(n);
+    while (lo < hi) {
+        const uint32_t mid = lo + (hi - lo) / 2;
+        if (dense_key(mt[mid], kx) < k)
+            lo = mid + 1;
+        else
+            hi = mid;
     }
+    return lo;
 }
 
 __device__ inline uint32_t nchunks_for(uint32_t cnt, uint32_t cap) { return (cnt + cap - 1) / cap; }
 
-__global__ void chunk_count_kernel(const uint32_t *__restrict__ begin, const uint32_t *__restrict__ end,
-                                   int64_t nkeys, uint32_t cap, uint32_t *__restrict__ nch)
+// Chunks of a cell's entries [b, b + cnt), stored from position 'at' of the list on.
+__device__ inline void store_chunks(uint32_t icell, uint32_t b, uint32_t cnt, uint32_t cap, uint32_t at,
+                                    Chunk *__restrict__ list, int64_t max_chunks)
 {
-    for (int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; k <= nkeys; k += int64_t(gridDim.x) * blockDim.x)
-        nch[k] = (k < nkeys && end[k] > begin[k]) ? nchunks_for(end[k] - begin[k], cap) : 0u;
+    const uint32_t nc = nchunks_for(cnt, cap);
+    for (uint32_t j = 0; j < nc; j++) {
+        Chunk c;
+        c.icell = icell;
+        c.begin = b + uint32_t((uint64_t(cnt) * j) / nc);
+        c.end = b + uint32_t((uint64_t(cnt) * (j + 1)) / nc);
+        c.flags = (nc > 1) ? CHUNK_SHARED : 0u;
+        if (int64_t(at) + j < max_chunks)
+            list[at + j] = c;
+    }
 }
 
-__global__ void chunk_fill_kernel(const uint32_t *__restrict__ begin, const uint32_t *__restrict__ end,
-                                  int64_t nkeys, uint32_t kx, uint32_t cap,
-                                  const uint32_t *__restrict__ choff, Chunk *__restrict__ chunks,
-                                  int64_t max_chunks)
+// One list as the kernels see it: chunks of at most 'cap' entries, their number in *count.
+struct WorkListOut
 {
-    for (int64_t k = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; k < nkeys; k += int64_t(gridDim.x) * blockDim.x) {
-        if (end[k] <= begin[k])
-            continue;
-        uint32_t b = begin[k], cnt = end[k] - begin[k];
-        uint32_t nc = nchunks_for(cnt, cap);
-        uint32_t icell = cell_key(int(k / kx), int(k % kx));
-        for (uint32_t j = 0; j < nc; j++) {
-            Chunk c;
-            c.icell = icell;
-            c.begin = b + uint32_t((uint64_t(cnt) * j) / nc);
-            c.end = b + uint32_t((uint64_t(cnt) * (j + 1)) / nc);
-            c.flags = (nc > 1) ? CHUNK_SHARED : 0u;
-            if (int64_t(choff[k]) + j < max_chunks)
-                chunks[choff[k] + j] = c;
+    Chunk *list;
+    int64_t max_chunks;
+    uint32_t cap;
+    uint32_t *count;
+};
+
+constexpr int WL_THREADS = 256;
+
+// One thread per cell of the global map: its entries by two binary searches (25 dependent loads, 10 us;
+// marking the ends of the runs in a pass over the plan took 59 us on the 2048x262144 raster).
+__global__ void __launch_bounds__(WL_THREADS)
+work_list_kernel(const uint64_t *__restrict__ mt, int64_t n, uint32_t kx, int64_t nkeys, WorkListOut a, WorkListOut b)
+{
+    __shared__ uint32_t s_begin[WL_THREADS + 1], s_wave[WL_THREADS / WAVE], s_base[2];
+    const int64_t k0 = int64_t(blockIdx.x) * WL_THREADS, k = k0 + threadIdx.x;
+    s_begin[threadIdx.x] = key_lower_bound(mt, n, kx, uint32_t(min(k, nkeys)));
+    if (threadIdx.x == 0)
+        s_begin[WL_THREADS] = key_lower_bound(mt, n, kx, uint32_t(min(k0 + WL_THREADS, nkeys)));
+    __syncthreads();
+    const uint32_t begin = s_begin[threadIdx.x], cnt = max(s_begin[threadIdx.x + 1], begin) - begin;
+    const uint32_t na = nchunks_for(cnt, a.cap), nb = nchunks_for(cnt, b.cap);
+    uint32_t ta, tb;
+    const uint32_t xa = block_exclusive_scan<WL_THREADS>(na, s_wave, ta);
+    const uint32_t xb = block_exclusive_scan<WL_THREADS>(nb, s_wave, tb);
+    if (threadIdx.x == 0) {
+        s_base[0] = ta ? atomicAdd(a.count, ta) : 0u;
+        s_base[1] = tb ? atomicAdd(b.count, tb) : 0u;
+    }
+    __syncthreads();
+    if (cnt > 0) {
+        const uint32_t icell = cell_key(int(k / kx), int(k % kx));
+        store_chunks(icell, begin, cnt, a.cap, s_base[0] + xa, a.list, a.max_chunks);
+        store_chunks(icell, begin, cnt, b.cap, s_base[1] + xb, b.list, b.max_chunks);
+    }
+}
+
+// Largest-first order of a list (entries equal in size in plan order), so that the operators' last
+// blocks are short ones (tod2map 1.4% faster on the 2048x262144 raster): each wave counts the chunks
+// that go before its four. blockIdx.y tells the list.
+constexpr int RK_PER_WAVE = 4;
+constexpr int RK_PER_BLOCK = RK_PER_WAVE * (WL_THREADS / WAVE);
+
+struct RankList
+{
+    const Chunk *src;
+    Chunk *dst;
+    const uint32_t *count;
+    int64_t max_chunks;
+};
+
+__global__ void __launch_bounds__(WL_THREADS)
+rank_chunks_kernel(RankList a, RankList b)
+{
+    const RankList l = blockIdx.y ? b : a;
+    const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+    const uint32_t n = uint32_t(min<int64_t>(*l.count, l.max_chunks));
+    const uint32_t i0 = blockIdx.x * RK_PER_BLOCK + wave * RK_PER_WAVE;
+    if (i0 >= n)
+        return;
+    Chunk own[RK_PER_WAVE];
+    uint32_t rank[RK_PER_WAVE] = {};
+#pragma unroll
+    for (int i = 0; i < RK_PER_WAVE; i++)
+        own[i] = l.src[min(i0 + i, n - 1)];
+    for (uint32_t j0 = 0; j0 < n; j0 += WAVE) {
+        const bool in = j0 + lane < n;
+        const Chunk c = in ? l.src[j0 + lane] : Chunk{};
+        const uint32_t len = c.end - c.begin;
+#pragma unroll
+        for (int i = 0; i < RK_PER_WAVE; i++) {
+            const uint32_t mine = own[i].end - own[i].begin;
+            rank[i] += uint32_t(__popcll(__ballot(in && (len > mine || (len == mine && c.begin < own[i].begin)))));
         }
     }
+#pragma unroll
+    for (int i = 0; i < RK_PER_WAVE; i++)
+        if (lane == 0 && i0 + i < n)
+            l.dst[rank[i]] = own[i];
 }
 
 // Owned-quad masks for the operators (ownership rule at HALO_X in gmm_common.hpp). For entry e
@@ -864,10 +932,9 @@ qmask_kernel(const uint64_t *__restrict__ mt, int64_t n, const float *__restrict
     }
 }
 
-__global__ void copy_word_kernel(const uint32_t *src, uint32_t *dst) { *dst = *src; }
-
-// Error bits and multi-cell lines of the emit pass's blocks: the bits go to *err_word and counts[2],
-// the number of lines to counts[1]. One block.
+// Error bits and multi-cell lines of the emit pass's blocks: the bits go to *err_word and
+// counts[PC_ERROR], the number of lines to counts[PC_NMLINES]; the other counts start from zero. One
+// block.
 __global__ void __launch_bounds__(PREPLAN_SIZE)
 plan_errors_kernel(const uint32_t *__restrict__ in, int n, uint32_t *__restrict__ err_word, uint32_t *__restrict__ counts)
 {
@@ -886,8 +953,9 @@ plan_errors_kernel(const uint32_t *__restrict__ in, int n, uint32_t *__restrict_
             nml += s_nml[w];
         }
         *err_word = err;
-        counts[1] = nml;
-        counts[2] = err;
+        counts[PC_CHUNKS_M2T] = counts[PC_CHUNKS_T2M] = 0;
+        counts[PC_NMLINES] = nml;
+        counts[PC_ERROR] = err;
     }
 }
 
@@ -948,8 +1016,8 @@ __global__ void iterator_test_kernel(const uint64_t *__restrict__ plan_mt, const
         atomicOr(err_word, err);
 }
 
-// Largest-first order of the operator work list (below): sort items (index << 20 | key) with
-// key = 8192 - entries, then gather the chunks in item order.
+// Long lists are put largest first by the radix sort: items (index << 20 | key) with key = 8192 -
+// entries, then the chunks gathered in item order.
 __global__ void chunk_key_kernel(const Chunk *__restrict__ chunks, int64_t n, uint64_t *__restrict__ items)
 {
     for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += int64_t(gridDim.x) * blockDim.x) {
@@ -957,12 +1025,6 @@ __global__ void chunk_key_kernel(const Chunk *__restrict__ chunks, int64_t n, ui
         const uint32_t key = 8192u - min(len, 8192u);
         items[i] = (uint64_t(i) << 20) | key;
     }
-}
-
-__global__ void chunk_copy_kernel(const Chunk *__restrict__ src, int64_t n, Chunk *__restrict__ dst)
-{
-    for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += int64_t(gridDim.x) * blockDim.x)
-        dst[i] = src[i];
 }
 
 __global__ void chunk_gather_kernel(const uint64_t *__restrict__ items, const Chunk *__restrict__ src, int64_t n,
@@ -1053,70 +1115,50 @@ struct SortLayout
 {
     int64_t ntiles;
     int64_t hist_off, hist_scan_off;   // histogram, scan scratch
-    int64_t begin_off, end_off, nch_off, nch_scan_off;
-    int64_t zc_off, zc_scan_off;
     int64_t total;
 };
 
-SortLayout sort_layout(int64_t nmt, int64_t nkeys)
+SortLayout sort_layout(int64_t nmt)
 {
     SortLayout L;
     L.ntiles = (nmt + RS_TILE - 1) / RS_TILE;
     int64_t o = 0;
     L.hist_off = o;      o += align128(4 * RS_RADIX * L.ntiles);
     L.hist_scan_off = o; o += align128(scan_scratch_nbytes(RS_RADIX * L.ntiles));
-    L.begin_off = o;     o += align128(4 * nkeys);
-    L.end_off = o;       o += align128(4 * nkeys);
-    L.nch_off = o;       o += align128(4 * (nkeys + 1));
-    L.nch_scan_off = o;  o += align128(scan_scratch_nbytes(nkeys + 1));
-    int64_t zt = (nmt + SC_TILE - 1) / SC_TILE;
-    L.zc_off = o;        o += align128(4 * (zt + 1));
-    L.zc_scan_off = o;   o += align128(scan_scratch_nbytes(zt + 1));
     L.total = o;
     return L;
 }
 
-}  // namespace
+// Lists of up to this many chunks are ordered by rank (n^2 comparisons: 16384 take about 40 us).
+constexpr int64_t RANK_MAX = 16384;
 
-// Reorders the work list of nch chunks largest first (stable: equal sizes stay in cell order),
-// so that the operators' last blocks are short ones (measured: tod2map 1.4% faster on the
-// 2048x262144 raster). Chunk sizes are at most chunk_cap <= 8192 entries: 13-bit keys, sorted
-// with the plan's radix sort (kx = 1024 makes its key the item's low 20 bits). Uses a and b
-// (>= 8 * nmt bytes each) and the plan scratch; skipped when 16 * nch bytes do not fit in b.
-void order_chunks(const gmm_preplan &pp, Chunk *chunks, int64_t nch, uint64_t *a, uint64_t *b, void *scratch,
-                  int64_t scratch_nbytes, hipStream_t stream)
+void launch_rank(const PlanLists &l, const uint32_t *counts, int64_t max_m2t, int64_t max_t2m, hipStream_t stream)
 {
-    if (nch < 2 || 2 * nch > pp.plan_nmt)
+    const RankList a{l.tmp_m2t, l.m2t, counts + PC_CHUNKS_M2T, l.max_m2t}, b{l.tmp_t2m, l.t2m, counts + PC_CHUNKS_T2M, l.max_t2m};
+    const int64_t n = std::max(max_m2t, max_t2m);
+    if (n <= 0)
         return;
-    SortLayout L = sort_layout(nch, 1);
-    GMM_REQUIRE(scratch_nbytes >= L.total, "order_chunks: scratch too small");
-    uint8_t *sc = reinterpret_cast<uint8_t *>(scratch);
-    uint32_t *hist = reinterpret_cast<uint32_t *>(sc + L.hist_off);
-    chunk_key_kernel<<<grid_for(nch, 256), 256, 0, stream>>>(chunks, nch, a);
-    GMM_HIP(hipGetLastError());
-    const int bits = 13, npasses = 2, per = 7;
-    uint64_t *src = a, *dst = b;
-    for (int pass = 0, shift = 0; pass < npasses; pass++, shift += per) {
-        const int nb = (bits - shift < per) ? (bits - shift) : per;
-        radix_hist_kernel<<<unsigned(L.ntiles), RS_THREADS, 0, stream>>>(src, nch, 1024u, shift, (1u << nb) - 1u, hist,
-                                                                          L.ntiles);
-        GMM_HIP(hipGetLastError());
-        exclusive_scan_u32(hist, int64_t(1 << nb) * L.ntiles, sc + L.hist_scan_off, stream);
-        radix_scatter_kernel<<<unsigned(L.ntiles), RS_THREADS, 0, stream>>>(src, dst, nullptr, nch, 1024u, shift, nb, hist,
-                                                                             L.ntiles);
-        GMM_HIP(hipGetLastError());
-        std::swap(src, dst);
-    }
-    // The sorted items are in src (= a after two passes); copy the chunks into b, gather back.
-    Chunk *copy = reinterpret_cast<Chunk *>(dst);
-    chunk_copy_kernel<<<grid_for(nch, 256), 256, 0, stream>>>(chunks, nch, copy);
-    chunk_gather_kernel<<<grid_for(nch, 256), 256, 0, stream>>>(src, copy, nch, chunks);
+    rank_chunks_kernel<<<dim3(unsigned((n + RK_PER_BLOCK - 1) / RK_PER_BLOCK), 2), WL_THREADS, 0, stream>>>(a, b);
     GMM_HIP(hipGetLastError());
 }
 
+}  // namespace
+
 int64_t plan_scratch_nbytes(const gmm_preplan &pp)
 {
-    return sort_layout(pp.plan_nmt, pp.nycells_g * pp.nxcells_g).total;
+    return sort_layout(pp.plan_nmt).total + align128(int64_t(sizeof(Chunk)) * (pp.max_nchunks + pp.max_nchunks_t2m));
+}
+
+PlanLists plan_lists(const gmm_preplan &pp, Chunk *m2t, Chunk *t2m, void *scratch)
+{
+    PlanLists l;
+    l.m2t = m2t;
+    l.t2m = t2m;
+    l.max_m2t = pp.max_nchunks;
+    l.max_t2m = pp.max_nchunks_t2m;
+    l.tmp_m2t = reinterpret_cast<Chunk *>(static_cast<uint8_t *>(scratch) + sort_layout(pp.plan_nmt).total);
+    l.tmp_t2m = l.tmp_m2t + pp.max_nchunks;
+    return l;
 }
 
 void plan_sort(const gmm_preplan &pp, uint64_t *a, uint64_t *b, uint64_t *out, uint16_t *qmask,
@@ -1124,7 +1166,7 @@ void plan_sort(const gmm_preplan &pp, uint64_t *a, uint64_t *b, uint64_t *out, u
 {
     const int64_t n = pp.plan_nmt;
     const uint32_t kx = uint32_t(pp.nxcells_g);
-    SortLayout L = sort_layout(n, pp.nycells_g * pp.nxcells_g);
+    SortLayout L = sort_layout(n);
     GMM_REQUIRE(scratch_nbytes >= L.total, "plan_sort: scratch too small");
     uint8_t *sc = reinterpret_cast<uint8_t *>(scratch);
     uint32_t *hist = reinterpret_cast<uint32_t *>(sc + L.hist_off);
@@ -1152,46 +1194,21 @@ void plan_sort(const gmm_preplan &pp, uint64_t *a, uint64_t *b, uint64_t *out, u
     }
 }
 
-namespace {
-
-// Shared by plan_schedule() and the iterator test: chunk list from a cell-sorted plan.
-// counts_gpu[0] <- number of chunks.
-void build_chunks(const uint64_t *mt, int64_t n, int64_t nkeys, uint32_t kx, uint32_t cap,
-                  Chunk *chunks, int64_t max_chunks, uint32_t *count_gpu, uint8_t *sc, const SortLayout &L,
-                  hipStream_t stream)
-{
-    uint32_t *begin = reinterpret_cast<uint32_t *>(sc + L.begin_off);
-    uint32_t *end = reinterpret_cast<uint32_t *>(sc + L.end_off);
-    uint32_t *nch = reinterpret_cast<uint32_t *>(sc + L.nch_off);
-
-    fill_u32_kernel<<<grid_for(nkeys, 256, 4096), 256, 0, stream>>>(begin, nkeys, 0u);
-    fill_u32_kernel<<<grid_for(nkeys, 256, 4096), 256, 0, stream>>>(end, nkeys, 0u);
-    cell_bounds_kernel<<<grid_for(n, 256), 256, 0, stream>>>(mt, n, kx, nkeys, begin, end);
-    chunk_count_kernel<<<grid_for(nkeys + 1, 256, 4096), 256, 0, stream>>>(begin, end, nkeys, cap, nch);
-    GMM_HIP(hipGetLastError());
-    exclusive_scan_u32(nch, nkeys + 1, sc + L.nch_scan_off, stream);
-    chunk_fill_kernel<<<grid_for(nkeys, 256, 4096), 256, 0, stream>>>(begin, end, nkeys, kx, cap, nch, chunks, max_chunks);
-    copy_word_kernel<<<1, 1, 0, stream>>>(nch + nkeys, count_gpu);
-    GMM_HIP(hipGetLastError());
-}
-
-}  // namespace
-
-void plan_schedule(const gmm_preplan &pp, const uint64_t *sorted_mt, const float *xp, Chunk *chunks,
-                   uint16_t *qmask, uint32_t *counts_gpu, void *scratch,
-                   int64_t scratch_nbytes, hipStream_t stream)
+void plan_schedule(const gmm_preplan &pp, const uint64_t *sorted_mt, const float *xp, const PlanLists &l,
+                   uint16_t *qmask, uint32_t *counts_gpu, hipStream_t stream)
 {
     const int64_t n = pp.plan_nmt;
     const int64_t nkeys = pp.nycells_g * pp.nxcells_g;
-    SortLayout L = sort_layout(n, nkeys);
-    GMM_REQUIRE(scratch_nbytes >= L.total, "plan_schedule: scratch too small");
-    uint8_t *sc = reinterpret_cast<uint8_t *>(scratch);
-
-    build_chunks(sorted_mt, n, nkeys, uint32_t(pp.nxcells_g), uint32_t(pp.chunk_cap), chunks,
-                 pp.max_nchunks, counts_gpu, sc, L, stream);
+    const WorkListOut a{l.tmp_m2t, l.max_m2t, uint32_t(pp.chunk_cap), counts_gpu + PC_CHUNKS_M2T};
+    const WorkListOut b{l.tmp_t2m, l.max_t2m, uint32_t(pp.chunk_cap_t2m), counts_gpu + PC_CHUNKS_T2M};
+    work_list_kernel<<<unsigned((nkeys + WL_THREADS - 1) / WL_THREADS), WL_THREADS, 0, stream>>>(
+        sorted_mt, n, uint32_t(pp.nxcells_g), nkeys, a, b);
+    GMM_HIP(hipGetLastError());
+    if (l.max_m2t <= RANK_MAX && l.max_t2m <= RANK_MAX)
+        launch_rank(l, counts_gpu, l.max_m2t, l.max_t2m, stream);
 
     // The owned-quad masks that the emit pass left.
-    const int grid = int(std::min<int64_t>((n + 255) / 256, 2048));
+    const int grid = int(std::min<int64_t>((n + 255) / 256, 8192));
     if (pp.periodic_xcoord)
         qmask_kernel<true><<<grid, 256, 0, stream>>>(sorted_mt, n, xp, pp.nsamp, int(pp.nypix_global),
                                                      int(pp.nxpix_global), qmask);
@@ -1201,23 +1218,55 @@ void plan_schedule(const gmm_preplan &pp, const uint64_t *sorted_mt, const float
     GMM_HIP(hipGetLastError());
 }
 
-int64_t build_chunks_generic_scratch(int64_t nmt)
+void order_long_lists(const gmm_preplan &pp, const PlanLists &l, int64_t n_m2t, int64_t n_t2m, const uint32_t *counts_gpu,
+                      uint64_t *a, uint64_t *b, void *scratch, hipStream_t stream)
 {
-    return sort_layout(nmt, int64_t(1) << 20).total;
+    if (l.max_m2t <= RANK_MAX && l.max_t2m <= RANK_MAX)
+        return;                                                      // plan_schedule() did it
+    if (n_m2t <= RANK_MAX && n_t2m <= RANK_MAX) {
+        launch_rank(l, counts_gpu, n_m2t, n_t2m, stream);
+        return;
+    }
+    // a and b hold plan_nmt items each, a list at most as many. 13-bit keys: kx = 1024 makes the sort's
+    // key the item's low 20 bits.
+    uint8_t *sc = reinterpret_cast<uint8_t *>(scratch);
+    auto order = [&](const Chunk *src, Chunk *dst, int64_t nch) {
+        if (nch <= 0)
+            return;
+        SortLayout L = sort_layout(nch);
+        uint32_t *hist = reinterpret_cast<uint32_t *>(sc + L.hist_off);
+        chunk_key_kernel<<<grid_for(nch, 256), 256, 0, stream>>>(src, nch, a);
+        GMM_HIP(hipGetLastError());
+        const int bits = 13, npasses = 2, per = 7;
+        uint64_t *from = a, *to = b;
+        for (int pass = 0, shift = 0; pass < npasses; pass++, shift += per) {
+            const int nb = (bits - shift < per) ? (bits - shift) : per;
+            radix_hist_kernel<<<unsigned(L.ntiles), RS_THREADS, 0, stream>>>(from, nch, 1024u, shift, (1u << nb) - 1u, hist,
+                                                                              L.ntiles);
+            GMM_HIP(hipGetLastError());
+            exclusive_scan_u32(hist, int64_t(1 << nb) * L.ntiles, sc + L.hist_scan_off, stream);
+            radix_scatter_kernel<<<unsigned(L.ntiles), RS_THREADS, 0, stream>>>(from, to, nullptr, nch, 1024u, shift, nb,
+                                                                                 hist, L.ntiles);
+            GMM_HIP(hipGetLastError());
+            std::swap(from, to);
+        }
+        chunk_gather_kernel<<<grid_for(nch, 256), 256, 0, stream>>>(from, src, nch, dst);
+        GMM_HIP(hipGetLastError());
+    };
+    order(l.tmp_m2t, l.m2t, n_m2t);
+    order(l.tmp_t2m, l.t2m, n_t2m);
 }
 
 int64_t build_chunks_generic(const uint64_t *plan_mt_gpu, int64_t nmt, int64_t chunk_cap,
-                             Chunk *chunks_gpu, int64_t max_chunks, void *scratch,
-                             int64_t scratch_nbytes, hipStream_t stream)
+                             Chunk *chunks_gpu, int64_t max_chunks, uint32_t *counts, hipStream_t stream)
 {
     const int64_t nkeys = int64_t(1) << 20;
-    SortLayout L = sort_layout(nmt, nkeys);
-    GMM_REQUIRE(scratch_nbytes >= L.total, "build_chunks_generic: scratch too small");
-    uint8_t *sc = reinterpret_cast<uint8_t *>(scratch);
-    uint32_t *count = reinterpret_cast<uint32_t *>(sc + L.zc_off);
-    build_chunks(plan_mt_gpu, nmt, nkeys, 1024u, uint32_t(chunk_cap), chunks_gpu, max_chunks, count, sc, L, stream);
+    fill_u32_kernel<<<1, 64, 0, stream>>>(counts, 2, 0u);
+    const WorkListOut a{chunks_gpu, max_chunks, uint32_t(chunk_cap), counts}, b{chunks_gpu, 0, uint32_t(nmt), counts + 1};
+    work_list_kernel<<<unsigned(nkeys / WL_THREADS), WL_THREADS, 0, stream>>>(plan_mt_gpu, nmt, 1024u, nkeys, a, b);
+    GMM_HIP(hipGetLastError());
     uint32_t h = 0;
-    GMM_HIP(hipMemcpyAsync(&h, count, 4, hipMemcpyDeviceToHost, stream));
+    GMM_HIP(hipMemcpyAsync(&h, counts, 4, hipMemcpyDeviceToHost, stream));
     GMM_HIP(hipStreamSynchronize(stream));
     return int64_t(h);
 }
