@@ -35,6 +35,7 @@ LIB_SOURCES = [
     ("capi.cpp", ["-x", "hip"]),
     ("capi_batch.cpp", ["-x", "hip"]),
     ("host_ref.cpp", ["-x", "hip", "-ffp-contract=off"]),
+    ("host_words.hip", []),
     ("k_planner.hip", []),
     ("k_planned.hip", []),
     ("k_unplanned.hip", []),

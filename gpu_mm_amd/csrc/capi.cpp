@@ -116,14 +116,6 @@ void require_ptr(const void *p, const char *where, const char *name)
         fail(std::string(where) + ": '" + name + "' is a null pointer");
 }
 
-uint32_t read_word(const uint32_t *p, hipStream_t stream)
-{
-    uint32_t h = 0;
-    GMM_HIP(hipMemcpyAsync(&h, p, 4, hipMemcpyDeviceToHost, stream));
-    GMM_HIP(hipStreamSynchronize(stream));
-    return h;
-}
-
 void clear_word(uint32_t *p, hipStream_t stream)
 {
     static const uint32_t zero = 0;
@@ -266,8 +258,7 @@ void with_bad_word(const char *where, hipStream_t stream, F f)
     try {
         launch_fill_u32(bad, 1, 0u, stream);
         f(bad);
-        GMM_HIP(hipMemcpyAsync(&h, bad, 4, hipMemcpyDeviceToHost, stream));
-        GMM_HIP(hipStreamSynchronize(stream));
+        h = read_word(bad, stream);
     }
     catch (...) {
         (void) hipFree(bad);
@@ -460,8 +451,7 @@ int gmm_preplan_create(gmm_preplan **out, const float *xpointing_gpu, int64_t ns
         launch_preplan_finish(nmt_gpu, err_gpu, pp.pparams.planner_nblocks, nullptr, stream);
 
         uint32_t h[3];
-        GMM_HIP(hipMemcpyAsync(h, err_gpu, sizeof(h), hipMemcpyDeviceToHost, stream));
-        GMM_HIP(hipStreamSynchronize(stream));
+        read_words(h, err_gpu, 3, stream);
         throw_errflags(h[0], where);
 
         const int64_t nmt = int64_t(h[1]) | (int64_t(h[2]) << 32);
@@ -598,8 +588,7 @@ int gmm_plan_create(gmm_plan **out, const gmm_preplan *pp, const float *xpointin
             plan_schedule(*pp, plan->plan_mt, xpointing_gpu, lists, plan->qmask, counts, stream);
 
             uint32_t h[PC_WORDS];
-            GMM_HIP(hipMemcpyAsync(h, counts, sizeof(h), hipMemcpyDeviceToHost, stream));
-            GMM_HIP(hipStreamSynchronize(stream));
+            read_words(h, counts, PC_WORDS, stream);
             if (h[PC_ERROR]) {
                 clear_word(err_word, stream);
                 throw_errflags(h[PC_ERROR], where);
@@ -796,9 +785,7 @@ void expand_dynamic(uint32_t *global_ncells_gpu, int64_t *cell_offsets_gpu, int6
     GMM_HIP(hipMalloc(&scratch, size_t(nb)));
     try {
         launch_expand_dynamic(global_ncells_gpu, cell_offsets_gpu, nycells, nxcells, plan_mt_gpu, nmt, scratch, stream);
-        uint32_t n = 0;
-        GMM_HIP(hipMemcpyAsync(&n, global_ncells_gpu, 4, hipMemcpyDeviceToHost, stream));
-        GMM_HIP(hipStreamSynchronize(stream));
+        const uint32_t n = read_word(global_ncells_gpu, stream);
         if (new_ncells)
             *new_ncells = n;
     }
@@ -848,10 +835,7 @@ int gmm_expand_dynamic_map_noalloc(uint32_t *global_ncells_gpu, int64_t *cell_of
         hipStream_t stream = as_stream(stream_);
         launch_expand_dynamic_noalloc(global_ncells_gpu, cell_offsets_gpu, nycells, nxcells, plan_mt_gpu, nmt, stream);
         if (new_ncells) {
-            uint32_t n = 0;
-            GMM_HIP(hipMemcpyAsync(&n, global_ncells_gpu, 4, hipMemcpyDeviceToHost, stream));
-            GMM_HIP(hipStreamSynchronize(stream));
-            *new_ncells = n;
+            *new_ncells = read_word(global_ncells_gpu, stream);
         }
     });
 }
@@ -1007,13 +991,7 @@ namespace {
 void check_unplanned_errflags(const uint32_t *errflags, int64_t nblocks, const char *where,
                               hipStream_t stream)
 {
-    std::vector<uint32_t> h(static_cast<size_t>(nblocks), 0u);
-    GMM_HIP(hipMemcpyAsync(h.data(), errflags, size_t(nblocks) * 4, hipMemcpyDeviceToHost, stream));
-    GMM_HIP(hipStreamSynchronize(stream));
-    uint32_t e = 0;
-    for (uint32_t v : h)
-        e |= v;
-    throw_errflags(e, where);
+    throw_errflags(read_word_or(errflags, nblocks, stream), where);
 }
 }  // namespace
 

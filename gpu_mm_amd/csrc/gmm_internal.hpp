@@ -97,7 +97,11 @@ int guarded(F &&f)
 inline hipStream_t as_stream(void *s) { return reinterpret_cast<hipStream_t>(s); }
 void require_ptr(const void *p, const char *where, const char *name);
 // Synchronous read / clear of one device word on 'stream'.
+// Device words as they are after the work enqueued on 'stream' so far, for which they wait: one, n (a few,
+// below 16), or the OR of n.
 uint32_t read_word(const uint32_t *p, hipStream_t stream);
+void read_words(uint32_t *out, const uint32_t *src, int n, hipStream_t stream);
+uint32_t read_word_or(const uint32_t *p, int64_t n, hipStream_t stream);
 void clear_word(uint32_t *p, hipStream_t stream);
 
 // Converts a set of error bits into the exception the reference raises

@@ -1,0 +1,73 @@
+"""Error flags and counts that a call waits for: after work that is still running on the call's stream,
+from several threads on streams of their own, and with errors in some of the calls."""
+
+import threading
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+NY, NX = 100, 130
+
+
+def make_pointing(n, seed, dev):
+    rng = np.random.default_rng(seed)
+    xp = np.stack([rng.uniform(0, NY - 1.5, n), rng.uniform(0, NX - 2.5, n), rng.uniform(0, 3, n)])
+    return torch.from_numpy(xp.astype(np.float32)).to(dev)
+
+
+@pytest.mark.parametrize("cycles", [0, 10000, 4000000])     # the last far longer than the polled wait
+def test_waits_for_the_stream(gmm, dev, cycles):
+    xg = make_pointing(4096, 1, dev)
+    plan = gmm.PointingPlan(gmm.PointingPrePlan(xg, NY, NX, periodic_xcoord=False), xg)
+    lp = gmm.LocalPixelization.make_rectangle(NY, NX, periodic_xcoord=False)
+    m = gmm.LocalMap(lp, torch.ones(3 * lp.npix, dtype=torch.float32, device=dev))
+    tod = torch.zeros(4096, dtype=torch.float32, device=dev)
+    good = xg.clone()
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        torch.cuda._sleep(cycles) if cycles else None
+        xg[0, 7] = -3.0                                     # bad by the time the operator runs
+        with pytest.raises(RuntimeError, match="y-value"):
+            gmm.map2tod(tod, m, xg, plan)
+        torch.cuda._sleep(cycles) if cycles else None
+        xg.copy_(good)
+        assert gmm.PointingPrePlan(xg, NY, NX, periodic_xcoord=False).plan_nmt == plan.plan_nmt
+        gmm.map2tod(tod, m, xg, plan)                       # flags were cleared
+    torch.cuda.current_stream().wait_stream(s)
+    want = 1 + torch.cos(2 * good[2]) + torch.sin(2 * good[2])
+    assert torch.allclose(tod, want, atol=1e-5)             # unit map: weights sum to 1
+
+
+def test_threads(gmm, dev):
+    """More calls at once than one thread's, each with its own outcome."""
+    nthreads, ncalls = 12, 40
+    xgs = [make_pointing(1000 + 37 * i, i, dev) for i in range(nthreads)]
+    bad = [x.clone() for x in xgs]
+    for i, b in enumerate(bad):
+        b[0, 5 * i] = NY + 1.0
+    nmt = [gmm.PointingPrePlan(x, NY, NX, periodic_xcoord=False).plan_nmt for x in xgs]
+    torch.cuda.synchronize()
+    failures = []
+
+    def work(i):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for k in range(ncalls):
+                    if (i + k) % 3:
+                        assert gmm.PointingPrePlan(xgs[i], NY, NX, periodic_xcoord=False).plan_nmt == nmt[i]
+                    else:
+                        with pytest.raises(RuntimeError, match="y-value"):
+                            gmm.PointingPrePlan(bad[i], NY, NX, periodic_xcoord=False)
+        except BaseException as e:                          # an assertion in a thread fails the test
+            failures.append((i, repr(e)))
+
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(nthreads)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join(60)
+    assert not failures and not any(t.is_alive() for t in ts)
