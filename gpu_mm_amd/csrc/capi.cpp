@@ -855,8 +855,17 @@ int gmm_lpix_expand_dynamic(gmm_lpix *lpix, const gmm_plan *plan, uint32_t *glob
             fail(std::string(where) + ": LocalPixelization and PointingPlan disagree on (nypix_global, nxpix_global, periodic_xcoord)");
         if (lpix->nycells != (pp.nypix_global + 63) / 64 || lpix->nxcells != (pp.nxpix_global + 63) / 64)
             fail(std::string(where) + ": a dynamic map needs the full (nycells, nxcells) cell table");
-        expand_dynamic(global_ncells_gpu, const_cast<int64_t *>(lpix->offsets_gpu), lpix->nycells, lpix->nxcells,
-                       plan->plan_mt, pp.plan_nmt, new_ncells, as_stream(stream_));
+        hipStream_t stream = as_stream(stream_);
+        int64_t *offsets = const_cast<int64_t *>(lpix->offsets_gpu);
+        if (!launch_expand_dynamic_chunks(global_ncells_gpu, offsets, lpix->nycells, lpix->nxcells, plan->chunks_t2m,
+                                          plan->nchunks_t2m, stream)) {
+            expand_dynamic(global_ncells_gpu, offsets, lpix->nycells, lpix->nxcells, plan->plan_mt, pp.plan_nmt,
+                           new_ncells, stream);
+            return;
+        }
+        const uint32_t n = read_word(global_ncells_gpu, stream);
+        if (new_ncells)
+            *new_ncells = n;
     });
 }
 

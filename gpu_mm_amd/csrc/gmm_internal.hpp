@@ -273,6 +273,9 @@ void launch_batched_tod2map(const BatchLaunch &bl, float *lmap, const gmm_lpix &
 // Dynamic map expansion (cells of a cell-sorted plan_mt into cell_offsets, new indices in
 // cell-key order); scratch of expand_dynamic_scratch_nbytes(nmt) bytes.
 int64_t expand_dynamic_scratch_nbytes(int64_t nmt);
+// The same for a plan's work list; false (nothing launched) when it is too long for one block.
+bool launch_expand_dynamic_chunks(uint32_t *global_ncells, int64_t *cell_offsets, int64_t nycells, int64_t nxcells,
+                                  const Chunk *chunks, int64_t nchunks, hipStream_t stream);
 void launch_expand_dynamic(uint32_t *global_ncells, int64_t *cell_offsets, int64_t nycells, int64_t nxcells,
                            const uint64_t *plan_mt, int64_t nmt, void *work, hipStream_t stream);
 // The same result without allocating: per-cell flags over the cell grid in a static device

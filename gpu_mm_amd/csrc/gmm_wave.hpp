@@ -73,4 +73,27 @@ __device__ inline uint32_t group8_reduce(uint32_t v, Op op)
     return v;
 }
 
+// Exclusive scan over a block of NT threads (NT/64 waves), returns the block total too;
+// s_wave: a word per wave.
+template<int NT>
+__device__ inline uint32_t block_exclusive_scan(uint32_t v, uint32_t *s_wave, uint32_t &total)
+{
+    constexpr int NW = NT / 64;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x / 64;
+    uint32_t inc = wave_inclusive_sum(v);
+    if (lane == 63)
+        s_wave[wave] = inc;
+    __syncthreads();
+    uint32_t before = 0, tot = 0;
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+        uint32_t t = s_wave[w];
+        before += (w < wave) ? t : 0u;
+        tot += t;
+    }
+    __syncthreads();
+    total = tot;
+    return before + inc - v;
+}
+
 }  // namespace gmm

@@ -10,6 +10,7 @@
 #include <mutex>
 
 #include "gmm_internal.hpp"
+#include "gmm_wave.hpp"
 
 namespace gmm {
 
@@ -57,6 +58,47 @@ dyn_assign_kernel(const uint64_t *__restrict__ mt, int64_t n, int64_t *__restric
 __global__ void dyn_count_kernel(const uint32_t *__restrict__ pos, int64_t n, uint32_t *__restrict__ global_ncells)
 {
     *global_ncells += pos[n];
+}
+
+// The same from a plan's work list, which names every cell of the plan at least once, in no matter what
+// order: one block marks the new cells in a bitmap of the grid in LDS (1024 x 1024 bits fit), numbers
+// them in row-major order, which is cell-key order, and stores their offsets. One launch without scratch
+// in place of a pass over the plan's entries with a scan of as many words, in memory allocated for the
+// call: three timestreams of 300 x 16421 samples into a map that grows 441 -> 261 us.
+constexpr int DC_THREADS = 1024;
+constexpr int DC_MAX_WORDS = 1024 * 1024 / 32;
+constexpr int64_t DC_MAX_CHUNKS = 32768;      // half a MiB for the one block to read, a few us
+
+__global__ void __launch_bounds__(DC_THREADS)
+dyn_chunks_kernel(const Chunk *__restrict__ chunks, int nchunks, int64_t *__restrict__ cell_offsets, uint32_t nycells,
+                  uint32_t nxcells, uint32_t *__restrict__ global_ncells)
+{
+    __shared__ uint32_t s_bits[DC_MAX_WORDS], s_wave[DC_THREADS / 64];
+    const int t = threadIdx.x;
+    const int nwords = int((nycells * nxcells + 31) / 32), per = (nwords + DC_THREADS - 1) / DC_THREADS;
+    const uint32_t base = *global_ncells;
+    for (int i = t; i < nwords; i += DC_THREADS)
+        s_bits[i] = 0;
+    __syncthreads();
+    for (int i = t; i < nchunks; i += DC_THREADS) {
+        const uint32_t icell = chunks[i].icell, cy = icell >> 10, cx = icell & 1023u;
+        const uint32_t ioff = cy * nxcells + cx;
+        if (cy < nycells && cx < nxcells && cell_offsets[ioff] == -1)
+            atomicOr(&s_bits[ioff >> 5], 1u << (ioff & 31));
+    }
+    __syncthreads();
+    // Thread t numbers the cells of words [per * t, per * t + per).
+    const int w0 = per * t, w1 = min(w0 + per, nwords);
+    uint32_t n = 0, total;
+    for (int w = w0; w < w1; w++)
+        n += uint32_t(__popc(s_bits[w]));
+    uint32_t at = base + block_exclusive_scan<DC_THREADS>(n, s_wave, total);
+    for (int w = w0; w < w1; w++)
+        for (uint32_t m = s_bits[w]; m; m &= m - 1)
+            cell_offsets[32 * w + __builtin_ctz(m)] = int64_t(at++) * int64_t(3 * CELL_NPIX);
+    __syncthreads();
+    if (t == 0)
+        *global_ncells = base + total;
 }
 
 // Allocation-free variant: per-cell flags over the (nycells, nxcells) grid instead of per-entry
@@ -155,6 +197,17 @@ void launch_expand_dynamic_noalloc(uint32_t *global_ncells, int64_t *cell_offset
     GMM_HIP(hipGetLastError());
     dyn_count_kernel<<<1, 1, 0, stream>>>(flags, ncg, global_ncells);
     GMM_HIP(hipGetLastError());
+}
+
+bool launch_expand_dynamic_chunks(uint32_t *global_ncells, int64_t *cell_offsets, int64_t nycells, int64_t nxcells,
+                                  const Chunk *chunks, int64_t nchunks, hipStream_t stream)
+{
+    if (nchunks > DC_MAX_CHUNKS || nycells * nxcells > 32 * int64_t(DC_MAX_WORDS))
+        return false;
+    dyn_chunks_kernel<<<1, DC_THREADS, 0, stream>>>(chunks, int(nchunks), cell_offsets, uint32_t(nycells),
+                                                    uint32_t(nxcells), global_ncells);
+    GMM_HIP(hipGetLastError());
+    return true;
 }
 
 int64_t expand_dynamic_scratch_nbytes(int64_t nmt)

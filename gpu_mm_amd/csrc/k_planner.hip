@@ -35,28 +35,6 @@ __device__ inline uint32_t wave_reduce_add(uint32_t v)
     return v;
 }
 
-// Exclusive scan over a block of NT threads (NT/64 waves), returns the block total too.
-template<int NT>
-__device__ inline uint32_t block_exclusive_scan(uint32_t v, uint32_t *s_wave, uint32_t &total)
-{
-    constexpr int NW = NT / WAVE;
-    const int lane = lane_id(), wave = threadIdx.x / WAVE;
-    uint32_t inc = wave_inclusive_sum(v);
-    if (lane == WAVE - 1)
-        s_wave[wave] = inc;
-    __syncthreads();
-    uint32_t before = 0, tot = 0;
-#pragma unroll
-    for (int w = 0; w < NW; w++) {
-        uint32_t t = s_wave[w];
-        before += (w < wave) ? t : 0u;
-        tot += t;
-    }
-    __syncthreads();
-    total = tot;
-    return before + inc - v;
-}
-
 // One extraction round over the remaining candidate cells of the two half-waves.
 // 'k' holds up to four distinct candidate keys per lane (NO_CELL = none). Returns false when
 // both halves are exhausted; otherwise removes one cell per non-empty half from every lane of
