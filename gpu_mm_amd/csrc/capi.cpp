@@ -582,10 +582,15 @@ int gmm_plan_create(gmm_plan **out, const gmm_preplan *pp, const float *xpointin
 
             uint32_t *err_word = plan->err + (pp->n_err - 1);
             launch_plan_emit(xpointing_gpu, *pp, a, plan->err, stream);
-            launch_plan_errors(plan->err, pp->pparams.planner_nblocks, err_word, counts, stream);
-            plan_sort(*pp, a, b, plan->plan_mt, plan->qmask, scratch, scratch_nbytes, stream);
             const PlanLists lists = plan_lists(*pp, plan->chunks, plan->chunks_t2m, scratch);
-            plan_schedule(*pp, plan->plan_mt, xpointing_gpu, lists, plan->qmask, counts, stream);
+            if (pp->plan_nmt <= SP_MAX)
+                plan_small(*pp, a, plan->plan_mt, plan->qmask, lists, plan->err, err_word, counts, stream);
+            else {
+                launch_plan_errors(plan->err, pp->pparams.planner_nblocks, err_word, counts, stream);
+                plan_sort(*pp, a, b, plan->plan_mt, plan->qmask, scratch, scratch_nbytes, stream);
+                plan_schedule(*pp, plan->plan_mt, lists, counts, stream);
+            }
+            plan_masks(*pp, plan->plan_mt, xpointing_gpu, plan->qmask, stream);
 
             uint32_t h[PC_WORDS];
             read_words(h, counts, PC_WORDS, stream);

@@ -159,11 +159,20 @@ struct PlanLists
 };
 PlanLists plan_lists(const gmm_preplan &pp, Chunk *m2t, Chunk *t2m, void *scratch);
 
-// Work lists of the sorted plan (their lengths go to counts_gpu) and the masks that the emit pass left
-// pending. Lists that may be longer than a ranking handles are left in the scratch for
-// order_long_lists(), which needs their lengths on the host.
-void plan_schedule(const gmm_preplan &pp, const uint64_t *sorted_mt, const float *xp, const PlanLists &l,
-                   uint16_t *qmask, uint32_t *counts_gpu, hipStream_t stream);
+// Work lists of the sorted plan; their lengths go to counts_gpu.
+void plan_schedule(const gmm_preplan &pp, const uint64_t *sorted_mt, const PlanLists &l, uint32_t *counts_gpu,
+                   hipStream_t stream);
+
+// Plans of at most SP_MAX entries: launch_plan_errors(), plan_sort() and plan_schedule() in one launch.
+constexpr int64_t SP_MAX = 8192;
+void plan_small(const gmm_preplan &pp, const uint64_t *items, uint64_t *out, uint16_t *qmask, const PlanLists &l,
+                const uint32_t *err_in, uint32_t *err_word, uint32_t *counts_gpu, hipStream_t stream);
+
+// The owned-quad masks that the emit pass left pending.
+void plan_masks(const gmm_preplan &pp, const uint64_t *sorted_mt, const float *xp, uint16_t *qmask, hipStream_t stream);
+
+// Lists that were too long to be put in order on the way are in the scratch; this orders them, their
+// lengths known on the host.
 void order_long_lists(const gmm_preplan &pp, const PlanLists &l, int64_t n_m2t, int64_t n_t2m, const uint32_t *counts_gpu,
                       uint64_t *a, uint64_t *b, void *scratch, hipStream_t stream);
 

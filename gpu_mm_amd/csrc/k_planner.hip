@@ -321,27 +321,31 @@ preplan_count_kernel(const float *__restrict__ xp, int64_t nsamp, int64_t ncl, i
 __global__ void __launch_bounds__(PREPLAN_SIZE)
 preplan_finish_kernel(uint32_t *nmt, uint32_t *err, int nblocks)
 {
-    __shared__ uint32_t s_wave[PREPLAN_SIZE / WAVE];
-    __shared__ unsigned long long s_tot64;
-    __shared__ uint32_t s_err;
+    constexpr int NW = PREPLAN_SIZE / WAVE;
+    __shared__ uint32_t s_wave[NW], s_lo[NW], s_hi[NW], s_err[NW];
     const int t = threadIdx.x;
     uint32_t v = (t < nblocks) ? nmt[t] : 0u;
-    uint32_t e = (t < nblocks) ? err[t] : 0u;
-    if (t == 0) {
-        s_tot64 = 0;
-        s_err = 0;
+    // The total in 64 bits from sums of 16-bit halves (all lanes adding to one word take 6 us).
+    const uint32_t lo = wave_reduce_add(v & 0xffffu), hi = wave_reduce_add(v >> 16);
+    const uint32_t e = wave_reduce_or((t < nblocks) ? err[t] : 0u);
+    if (lane_id() == 0) {
+        s_lo[t / WAVE] = lo;
+        s_hi[t / WAVE] = hi;
+        s_err[t / WAVE] = e;
     }
-    __syncthreads();
-    atomicAdd(&s_tot64, (unsigned long long)v);
-    atomicOr(&s_err, e);
     uint32_t total;
-    uint32_t excl = block_exclusive_scan<PREPLAN_SIZE>(v, s_wave, total);
+    uint32_t excl = block_exclusive_scan<PREPLAN_SIZE>(v, s_wave, total);   // synchronizes
     nmt[t] = (t < nblocks) ? (excl + v) : total;
-    __syncthreads();
     if (t == 0) {
-        err[0] = s_err;
-        err[1] = uint32_t(s_tot64);
-        err[2] = uint32_t(s_tot64 >> 32);
+        uint64_t sum = 0;
+        uint32_t flags = 0;
+        for (int w = 0; w < NW; w++) {
+            sum += uint64_t(s_lo[w]) + (uint64_t(s_hi[w]) << 16);
+            flags |= s_err[w];
+        }
+        err[0] = flags;
+        err[1] = uint32_t(sum);
+        err[2] = uint32_t(sum >> 32);
     }
 }
 
@@ -910,11 +914,10 @@ qmask_kernel(const uint64_t *__restrict__ mt, int64_t n, const float *__restrict
     }
 }
 
-// Error bits and multi-cell lines of the emit pass's blocks: the bits go to *err_word and
-// counts[PC_ERROR], the number of lines to counts[PC_NMLINES]; the other counts start from zero. One
-// block.
-__global__ void __launch_bounds__(PREPLAN_SIZE)
-plan_errors_kernel(const uint32_t *__restrict__ in, int n, uint32_t *__restrict__ err_word, uint32_t *__restrict__ counts)
+// Error bits and multi-cell lines of the emit pass's blocks, by a block of PREPLAN_SIZE threads: the bits go
+// to *err_word and counts[PC_ERROR], the number of lines to counts[PC_NMLINES].
+__device__ inline void gather_plan_errors(const uint32_t *__restrict__ in, int n, uint32_t *__restrict__ err_word,
+                                          uint32_t *__restrict__ counts)
 {
     __shared__ uint32_t s_err[PREPLAN_SIZE / WAVE], s_nml[PREPLAN_SIZE / WAVE];
     const uint32_t v = (int(threadIdx.x) < n) ? in[threadIdx.x] : 0u;
@@ -931,10 +934,178 @@ plan_errors_kernel(const uint32_t *__restrict__ in, int n, uint32_t *__restrict_
             nml += s_nml[w];
         }
         *err_word = err;
-        counts[PC_CHUNKS_M2T] = counts[PC_CHUNKS_T2M] = 0;
         counts[PC_NMLINES] = nml;
         counts[PC_ERROR] = err;
     }
+}
+
+__global__ void __launch_bounds__(PREPLAN_SIZE)
+plan_errors_kernel(const uint32_t *__restrict__ in, int n, uint32_t *__restrict__ err_word, uint32_t *__restrict__ counts)
+{
+    gather_plan_errors(in, n, err_word, counts);
+    if (threadIdx.x == 0)
+        counts[PC_CHUNKS_M2T] = counts[PC_CHUNKS_T2M] = 0;
+}
+
+// ------------------------------------------------------------------------------------------
+// Small plans, up to SP_MAX entries: what follows the emit pass (error words, sort, work lists) in one
+// launch of one block, the entries in LDS. Such a plan's time is launches: with one each for the error
+// words, the digit histograms, their scan, the scatter (per pass), the lists and their order, preplan and
+// plan of 1000 entries took 93 us, now 75; of 7900, where the one block takes 23 us, 100 and 91.
+
+constexpr int SP_THREADS = PREPLAN_SIZE;
+constexpr int SP_NW = SP_THREADS / WAVE;
+constexpr int SP_ROUNDS = 8;
+constexpr int SP_RANK = SP_THREADS;                      // longest list that is ordered here
+constexpr int SP_BEGIN_BITS = 13, SP_LEN_BITS = 11;      // a chunk has at most 1024 entries
+static_assert(SP_THREADS * SP_ROUNDS == SP_MAX && SP_MAX == 1 << SP_BEGIN_BITS, "one item per thread and round");
+
+// A list's chunks as words: ~length, begin, shared, so that they are in the list's order.
+__device__ inline uint32_t sp_pack(uint32_t begin, uint32_t end, bool shared)
+{
+    const uint32_t inv = (1u << SP_LEN_BITS) - 1u - (end - begin);
+    return (inv << (SP_BEGIN_BITS + 1)) | (begin << 1) | (shared ? CHUNK_SHARED : 0u);
+}
+
+__device__ inline Chunk sp_unpack(uint32_t v, const uint64_t *items)
+{
+    Chunk c;
+    c.begin = (v >> 1) & (SP_MAX - 1);
+    c.end = c.begin + (1u << SP_LEN_BITS) - 1u - (v >> (SP_BEGIN_BITS + 1));
+    c.flags = v & CHUNK_SHARED;
+    c.icell = uint32_t(items[c.begin]) & CELL_MASK;
+    return c;
+}
+
+// The list of chunks of at most 'cap' entries of the cells that start at start[0 .. ncells). In 'dst' in
+// order when there are at most SP_RANK, else in 'tmp' in any (the host then orders it).
+__device__ inline void sp_work_list(const uint64_t *items, const uint16_t *start, uint32_t ncells, const WorkListOut &l,
+                                    Chunk *__restrict__ dst, uint32_t *s_key, uint32_t *s_wave)
+{
+    const uint32_t t = threadIdx.x;
+    uint32_t mine = 0, total;
+    for (uint32_t c = t; c < ncells; c += SP_THREADS)
+        mine += nchunks_for(uint32_t(start[c + 1]) - start[c], l.cap);
+    uint32_t at = block_exclusive_scan<SP_THREADS>(mine, s_wave, total);
+    if (t == 0)
+        *l.count = total;
+    const bool ordered = total <= SP_RANK;
+    for (uint32_t c = t; c < ncells; c += SP_THREADS) {
+        const uint32_t b = start[c], cnt = uint32_t(start[c + 1]) - b, nc = nchunks_for(cnt, l.cap);
+        for (uint32_t j = 0; j < nc; j++, at++) {
+            const uint32_t v = sp_pack(b + cnt * j / nc, b + cnt * (j + 1) / nc, nc > 1);
+            if (ordered)
+                s_key[at] = v;
+            else if (int64_t(at) < l.max_chunks)
+                l.list[at] = sp_unpack(v, items);
+        }
+    }
+    __syncthreads();
+    if (ordered && t < total) {
+        const uint32_t v = s_key[t];
+        uint32_t rank = 0;
+        for (uint32_t j = 0; j < total; j++)
+            rank += (s_key[j] < v) ? 1u : 0u;
+        if (int64_t(rank) < l.max_chunks)
+            dst[rank] = sp_unpack(v, items);
+    }
+    __syncthreads();
+}
+
+__global__ void __launch_bounds__(SP_THREADS)
+small_plan_kernel(const uint64_t *__restrict__ in, uint32_t n, uint32_t kx, int bits, uint64_t *__restrict__ out,
+                  uint16_t *__restrict__ qmask, WorkListOut a, WorkListOut b, Chunk *__restrict__ dst_a,
+                  Chunk *__restrict__ dst_b, const uint32_t *__restrict__ err_in, int nblocks,
+                  uint32_t *__restrict__ err_word, uint32_t *__restrict__ counts)
+{
+    __shared__ uint64_t s_item[SP_MAX];
+    __shared__ uint32_t s_cnt[SP_NW][RS_RADIX];
+    __shared__ uint16_t s_start[SP_MAX + 1];
+    __shared__ uint32_t s_key[SP_RANK], s_wave[SP_NW];
+    const int t = threadIdx.x, lane = lane_id(), wave = t / WAVE;
+
+    gather_plan_errors(err_in, nblocks, err_word, counts);
+
+    // The stable radix sort of the tiles above, on one tile: wave w owns items [w * 64 * rounds, ...).
+    const int rounds = int((n + SP_THREADS - 1) / SP_THREADS);
+    const uint32_t w0 = uint32_t(wave * rounds * WAVE + lane);
+    for (int r = 0; r < rounds; r++) {
+        const uint32_t i = w0 + r * WAVE;
+        if (i < n)
+            s_item[i] = in[i];
+    }
+    const int npasses = (bits + RS_MAXBITS - 1) / RS_MAXBITS;
+    const int per = npasses ? (bits + npasses - 1) / npasses : 0;
+    for (int pass = 0, shift = 0; pass < npasses; pass++, shift += per) {
+        const int nb = min(bits - shift, per);
+        const uint32_t dmask = (1u << nb) - 1u;
+        for (int i = t; i < SP_NW * RS_RADIX; i += SP_THREADS)
+            (&s_cnt[0][0])[i] = 0;
+        __syncthreads();
+        uint64_t item[SP_ROUNDS];
+        uint32_t dig[SP_ROUNDS], rank[SP_ROUNDS];
+#pragma unroll
+        for (int r = 0; r < SP_ROUNDS; r++) {
+            if (r >= rounds)
+                break;
+            const uint32_t i = w0 + r * WAVE;
+            const bool valid = i < n;
+            item[r] = valid ? s_item[i] : 0ull;
+            const uint32_t d = valid ? ((dense_key(item[r], kx) >> shift) & dmask) : 0u;
+            dig[r] = d;
+            uint64_t peers = __ballot(valid);
+            for (int bit = 0; bit < nb; bit++) {
+                const uint64_t bb = __ballot((d >> bit) & 1u);
+                peers &= ((d >> bit) & 1u) ? bb : ~bb;
+            }
+            const uint32_t below = uint32_t(__popcll(peers & lanemask_lt()));
+            const uint32_t old = valid ? s_cnt[wave][d] : 0u;
+            if (valid && below == 0)
+                s_cnt[wave][d] = old + uint32_t(__popcll(peers));
+            rank[r] = old + below;
+        }
+        __syncthreads();
+        uint32_t sum = 0, total;
+        if (t < RS_RADIX)
+            for (int w = 0; w < SP_NW; w++)
+                sum += s_cnt[w][t];
+        uint32_t at = block_exclusive_scan<SP_THREADS>(sum, s_wave, total);
+        if (t < RS_RADIX)
+            for (int w = 0; w < SP_NW; w++) {
+                const uint32_t c = s_cnt[w][t];
+                s_cnt[w][t] = at;
+                at += c;
+            }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < SP_ROUNDS; r++) {
+            if (r >= rounds)
+                break;
+            if (w0 + r * WAVE < n)
+                s_item[s_cnt[wave][dig[r]] + rank[r]] = item[r];
+        }
+        __syncthreads();
+    }
+    __syncthreads();
+    for (uint32_t i = t; i < n; i += SP_THREADS)
+        store_item(out, qmask, i, s_item[i]);
+
+    // First entries of the cells, in order: thread t looks at entries [t * rounds, ...).
+    auto starts = [&](uint32_t i) {
+        return i < n && (i == 0 || ((uint32_t(s_item[i]) ^ uint32_t(s_item[i - 1])) & CELL_MASK));
+    };
+    uint32_t mine = 0, ncells;
+    for (int r = 0; r < rounds; r++)
+        mine += starts(uint32_t(t * rounds + r)) ? 1u : 0u;
+    uint32_t at = block_exclusive_scan<SP_THREADS>(mine, s_wave, ncells);
+    for (int r = 0; r < rounds; r++)
+        if (starts(uint32_t(t * rounds + r)))
+            s_start[at++] = uint16_t(t * rounds + r);
+    if (t == 0)
+        s_start[ncells] = uint16_t(n);
+    __syncthreads();
+    sp_work_list(s_item, s_start, ncells, a, dst_a, s_key, s_wave);
+    sp_work_list(s_item, s_start, ncells, b, dst_b, s_key, s_wave);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1110,9 +1281,20 @@ SortLayout sort_layout(int64_t nmt)
 // Lists of up to this many chunks are ordered by rank (n^2 comparisons: 16384 take about 40 us).
 constexpr int64_t RANK_MAX = 16384;
 
+WorkListOut m2t_out(const gmm_preplan &pp, const PlanLists &l, uint32_t *counts)
+{
+    return WorkListOut{l.tmp_m2t, l.max_m2t, uint32_t(pp.chunk_cap), counts + PC_CHUNKS_M2T};
+}
+
+WorkListOut t2m_out(const gmm_preplan &pp, const PlanLists &l, uint32_t *counts)
+{
+    return WorkListOut{l.tmp_t2m, l.max_t2m, uint32_t(pp.chunk_cap_t2m), counts + PC_CHUNKS_T2M};
+}
+
+// Orders the lists, of at most max_m2t and max_t2m chunks (0: leaves that one alone).
 void launch_rank(const PlanLists &l, const uint32_t *counts, int64_t max_m2t, int64_t max_t2m, hipStream_t stream)
 {
-    const RankList a{l.tmp_m2t, l.m2t, counts + PC_CHUNKS_M2T, l.max_m2t}, b{l.tmp_t2m, l.t2m, counts + PC_CHUNKS_T2M, l.max_t2m};
+    const RankList a{l.tmp_m2t, l.m2t, counts + PC_CHUNKS_M2T, max_m2t}, b{l.tmp_t2m, l.t2m, counts + PC_CHUNKS_T2M, max_t2m};
     const int64_t n = std::max(max_m2t, max_t2m);
     if (n <= 0)
         return;
@@ -1172,20 +1354,32 @@ void plan_sort(const gmm_preplan &pp, uint64_t *a, uint64_t *b, uint64_t *out, u
     }
 }
 
-void plan_schedule(const gmm_preplan &pp, const uint64_t *sorted_mt, const float *xp, const PlanLists &l,
-                   uint16_t *qmask, uint32_t *counts_gpu, hipStream_t stream)
+void plan_schedule(const gmm_preplan &pp, const uint64_t *sorted_mt, const PlanLists &l, uint32_t *counts_gpu,
+                   hipStream_t stream)
 {
     const int64_t n = pp.plan_nmt;
     const int64_t nkeys = pp.nycells_g * pp.nxcells_g;
-    const WorkListOut a{l.tmp_m2t, l.max_m2t, uint32_t(pp.chunk_cap), counts_gpu + PC_CHUNKS_M2T};
-    const WorkListOut b{l.tmp_t2m, l.max_t2m, uint32_t(pp.chunk_cap_t2m), counts_gpu + PC_CHUNKS_T2M};
     work_list_kernel<<<unsigned((nkeys + WL_THREADS - 1) / WL_THREADS), WL_THREADS, 0, stream>>>(
-        sorted_mt, n, uint32_t(pp.nxcells_g), nkeys, a, b);
+        sorted_mt, n, uint32_t(pp.nxcells_g), nkeys, m2t_out(pp, l, counts_gpu), t2m_out(pp, l, counts_gpu));
     GMM_HIP(hipGetLastError());
     if (l.max_m2t <= RANK_MAX && l.max_t2m <= RANK_MAX)
         launch_rank(l, counts_gpu, l.max_m2t, l.max_t2m, stream);
+}
 
-    // The owned-quad masks that the emit pass left.
+void plan_small(const gmm_preplan &pp, const uint64_t *items, uint64_t *out, uint16_t *qmask, const PlanLists &l,
+                const uint32_t *err_in, uint32_t *err_word, uint32_t *counts_gpu, hipStream_t stream)
+{
+    GMM_REQUIRE(pp.plan_nmt <= SP_MAX && pp.chunk_cap < (1 << SP_LEN_BITS) && pp.chunk_cap_t2m < (1 << SP_LEN_BITS),
+                "plan_small: plan too large");
+    small_plan_kernel<<<1, SP_THREADS, 0, stream>>>(items, uint32_t(pp.plan_nmt), uint32_t(pp.nxcells_g), pp.key_bits, out,
+                                                    qmask, m2t_out(pp, l, counts_gpu), t2m_out(pp, l, counts_gpu), l.m2t,
+                                                    l.t2m, err_in, int(pp.pparams.planner_nblocks), err_word, counts_gpu);
+    GMM_HIP(hipGetLastError());
+}
+
+void plan_masks(const gmm_preplan &pp, const uint64_t *sorted_mt, const float *xp, uint16_t *qmask, hipStream_t stream)
+{
+    const int64_t n = pp.plan_nmt;
     const int grid = int(std::min<int64_t>((n + 255) / 256, 8192));
     if (pp.periodic_xcoord)
         qmask_kernel<true><<<grid, 256, 0, stream>>>(sorted_mt, n, xp, pp.nsamp, int(pp.nypix_global),
@@ -1199,6 +1393,10 @@ void plan_schedule(const gmm_preplan &pp, const uint64_t *sorted_mt, const float
 void order_long_lists(const gmm_preplan &pp, const PlanLists &l, int64_t n_m2t, int64_t n_t2m, const uint32_t *counts_gpu,
                       uint64_t *a, uint64_t *b, void *scratch, hipStream_t stream)
 {
+    if (pp.plan_nmt <= SP_MAX) {                                     // plan_small() did the short ones
+        launch_rank(l, counts_gpu, (n_m2t > SP_RANK) ? n_m2t : 0, (n_t2m > SP_RANK) ? n_t2m : 0, stream);
+        return;
+    }
     if (l.max_m2t <= RANK_MAX && l.max_t2m <= RANK_MAX)
         return;                                                      // plan_schedule() did it
     if (n_m2t <= RANK_MAX && n_t2m <= RANK_MAX) {
