@@ -470,15 +470,7 @@ int gmm_preplan_create(gmm_preplan **out, const float *xpointing_gpu, int64_t ns
         pp.nxcells_g = (nxpix_global + 63) / 64;
         const int64_t nkeys = pp.nycells_g * pp.nxcells_g;
         pp.key_bits = bits_for(nkeys);
-        // Entries per work unit. map2tod: a block costs little (it stages its cell), and many small ones
-        // balance well. tod2map: every block clears and flushes a 116 KiB tile, atomically when its cell
-        // is split, and runs alone on its CU: about two blocks per CU at the least 1024 entries each
-        // (times with its own list against map2tod's: 299 / 480 us on 1.8e6 entries, 38 / 52 us on 1.4e5;
-        // map2tod takes 285 and 33 us with tod2map's list, 263 and 27 us with its own).
-        pp.chunk_cap = std::min<int64_t>(8192, std::max<int64_t>(512, (nmt + 3071) / 3072));
-        pp.chunk_cap_t2m = std::min<int64_t>(8192, std::max<int64_t>(1024, (nmt + 511) / 512));
-        pp.max_nchunks = (nmt + pp.chunk_cap - 1) / pp.chunk_cap + std::min(nmt, nkeys);
-        pp.max_nchunks_t2m = (nmt + pp.chunk_cap_t2m - 1) / pp.chunk_cap_t2m + std::min(nmt, nkeys);
+        plan_chunk_caps(pp);
         pp.n_err = pp.pparams.planner_nblocks + 1;
 
         pp.off_err = align128(8 * nmt);
@@ -1169,7 +1161,7 @@ int gmm_test_plan_iterator(const uint64_t *plan_mt_cpu, int64_t nmt, int64_t nmt
 
         const int64_t max_chunks = (nmt + nmt_per_block - 1) / nmt_per_block + std::min<int64_t>(nmt, int64_t(1) << 20);
         const int64_t bytes = align128(8 * nmt) + align128(int64_t(sizeof(Chunk)) * max_chunks)
-                            + align128(4 * nmt) + 128;
+                            + align128(4 * nmt) + 128 + build_chunks_generic_scratch_nbytes();
         void *mem = nullptr;
         GMM_HIP(hipMalloc(&mem, size_t(bytes)));
         std::string failure;
@@ -1179,11 +1171,10 @@ int gmm_test_plan_iterator(const uint64_t *plan_mt_cpu, int64_t nmt, int64_t nmt
             Chunk *d_ch = reinterpret_cast<Chunk *>(m + align128(8 * nmt));
             uint32_t *d_vis = reinterpret_cast<uint32_t *>(m + align128(8 * nmt) + align128(int64_t(sizeof(Chunk)) * max_chunks));
             uint32_t *d_err = d_vis + nmt;
-            uint32_t *d_cnt = reinterpret_cast<uint32_t *>(m + align128(8 * nmt) + align128(int64_t(sizeof(Chunk)) * max_chunks)
-                                                           + align128(4 * nmt)) + 16;
+            uint8_t *d_scr = m + align128(8 * nmt) + align128(int64_t(sizeof(Chunk)) * max_chunks) + align128(4 * nmt) + 128;
             GMM_HIP(hipMemcpy(d_mt, plan_mt_cpu, size_t(nmt) * 8, hipMemcpyHostToDevice));
             GMM_HIP(hipMemset(d_vis, 0, size_t(nmt) * 4));
-            int64_t nch = build_chunks_generic(d_mt, nmt, nmt_per_block, d_ch, max_chunks, d_cnt, nullptr);
+            int64_t nch = build_chunks_generic(d_mt, nmt, nmt_per_block, d_ch, max_chunks, d_scr, nullptr);
             GMM_REQUIRE(nch <= max_chunks, "test_plan_iterator: chunk count exceeds bound");
             launch_iterator_test(d_mt, d_ch, nch, waves_per_block, d_vis, d_err, nullptr);
             std::vector<uint32_t> vis(static_cast<size_t>(nmt), 0u);

@@ -254,6 +254,15 @@ struct Chunk
 
 constexpr uint32_t CHUNK_SHARED = 1u;
 
+// Sizes that a work list may be cut by, the best first: the list takes the first 'cap' (most entries of a
+// chunk) that makes at most 'limit' chunks. The last has no limit.
+constexpr int NCAPS = 12;
+struct ChunkCaps
+{
+    uint32_t n;
+    uint32_t cap[NCAPS], limit[NCAPS];
+};
+
 // Entries [wb, we) of a chunk handled by wave 'wave' of 'nw' in the planned operators: the chunk
 // split into nw contiguous, near-equal slices. Each wave then walks its slice in batches of 64
 // entries (one plan entry per lane, one vector load) and steps of 8 entries (lane 8*li + q takes

@@ -38,8 +38,7 @@ struct gmm_preplan
     // Derived sizes (computed once in the constructor).
     int64_t nycells_g = 0, nxcells_g = 0;  // cells of the global map
     int key_bits = 0;                      // bits of the dense cell key iycell*nxcells_g + ixcell
-    int64_t chunk_cap = 0;                 // max plan entries per map2tod work unit
-    int64_t chunk_cap_t2m = 0;             // ... per tod2map work unit
+    gmm::ChunkCaps caps_m2t = {}, caps_t2m = {};   // sizes of the operators' work units
     int64_t max_nchunks = 0, max_nchunks_t2m = 0;
     int64_t plan_nbytes = 0, tmp_nbytes = 0, sort_nbytes = 0;
 
@@ -147,14 +146,20 @@ void launch_plan_errors(const uint32_t *in, int64_t nblocks, uint32_t *err_word,
 void plan_sort(const gmm_preplan &pp, uint64_t *a, uint64_t *b, uint64_t *out, uint16_t *qmask,
                void *scratch, int64_t scratch_nbytes, hipStream_t stream);
 
-// Counts that plan construction brings back to the host.
-enum PlanCount { PC_CHUNKS_M2T = 0, PC_NMLINES = 1, PC_ERROR = 2, PC_CHUNKS_T2M = 3, PC_WORDS = 4 };
+// Counts that plan construction keeps on the device; the first PC_WORDS are brought back to the host.
+enum PlanCount { PC_CHUNKS_M2T = 0, PC_NMLINES = 1, PC_ERROR = 2, PC_CHUNKS_T2M = 3, PC_WORDS = 4,
+                 PC_CAPS_M2T = PC_WORDS, PC_CAPS_T2M = PC_CAPS_M2T + NCAPS, PC_TOTAL = PC_CAPS_T2M + NCAPS };
+
+// The sizes that the operators' work lists of a plan of pp.plan_nmt entries may be cut by, and the bounds
+// on the lists' lengths.
+void plan_chunk_caps(gmm_preplan &pp);
 
 // The operators' work lists: where they go, and the scratch in which they are made.
 struct PlanLists
 {
     Chunk *m2t, *t2m;
     Chunk *tmp_m2t, *tmp_t2m;
+    uint32_t *begin;                       // first entry of each cell of the global map
     int64_t max_m2t, max_t2m;
 };
 PlanLists plan_lists(const gmm_preplan &pp, Chunk *m2t, Chunk *t2m, void *scratch);
@@ -191,9 +196,10 @@ void launch_iterator_test(const uint64_t *plan_mt, const Chunk *chunks, int64_t 
                           int waves_per_block, uint32_t *visit_counts, uint32_t *err_word,
                           hipStream_t stream);
 
-// Builds chunks from an arbitrary cell-sorted plan (used by the iterator test); counts: two words.
+// Builds chunks from an arbitrary cell-sorted plan (used by the iterator test).
+int64_t build_chunks_generic_scratch_nbytes();
 int64_t build_chunks_generic(const uint64_t *plan_mt_gpu, int64_t nmt, int64_t chunk_cap,
-                             Chunk *chunks_gpu, int64_t max_chunks, uint32_t *counts, hipStream_t stream);
+                             Chunk *chunks_gpu, int64_t max_chunks, void *scratch, hipStream_t stream);
 
 // ------------------------------------------------------------------------------------------
 // Operator launchers (k_planned.hip, k_unplanned.hip).

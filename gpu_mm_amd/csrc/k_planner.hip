@@ -1,9 +1,5 @@
 // Plan construction on gfx950: preplan count, deterministic emit, device scan, stable LSD
-// radix sort in LDS, and the operator work list (chunks + multi-cell line list).
-//
-// All kernels assume 64-lane waves. A 32-sample TOD line maps onto one half-wave, so each wave
-// handles two lines at a time; the set of cells touched by a line is found by repeated
-// ballot/readlane extraction instead of warp32 match-any.
+// radix sort in LDS, and the operators' work lists. All kernels assume 64-lane waves.
 
 #include "gmm_internal.hpp"
 #include "gmm_locate.hpp"
@@ -718,30 +714,68 @@ __device__ inline void store_chunks(uint32_t icell, uint32_t b, uint32_t cnt, ui
     }
 }
 
-// One list as the kernels see it: chunks of at most 'cap' entries, their number in *count.
+// One list as the kernels see it: the sizes to choose from, how many chunks each of them makes, and the
+// number of chunks of the list.
 struct WorkListOut
 {
     Chunk *list;
     int64_t max_chunks;
-    uint32_t cap;
+    ChunkCaps caps;
+    uint32_t *cap_counts;
     uint32_t *count;
 };
 
 constexpr int WL_THREADS = 256;
 
-// One thread per cell of the global map: its entries by two binary searches (25 dependent loads, 10 us;
-// marking the ends of the runs in a pass over the plan took 59 us on the 2048x262144 raster).
+// First entry of each cell of the global map, one cell a thread, by binary search (25 dependent loads,
+// 10 us; marking the ends of the runs in a pass over the plan took 59 us on the 2048x262144 raster); and
+// the number of chunks that each size of the two lists would make.
 __global__ void __launch_bounds__(WL_THREADS)
-work_list_kernel(const uint64_t *__restrict__ mt, int64_t n, uint32_t kx, int64_t nkeys, WorkListOut a, WorkListOut b)
+cell_runs_kernel(const uint64_t *__restrict__ mt, int64_t n, uint32_t kx, int64_t nkeys, uint32_t *__restrict__ begin,
+                 WorkListOut a, WorkListOut b)
 {
-    __shared__ uint32_t s_begin[WL_THREADS + 1], s_wave[WL_THREADS / WAVE], s_base[2];
+    __shared__ uint32_t s_begin[WL_THREADS + 1], s_counts[2 * NCAPS];
     const int64_t k0 = int64_t(blockIdx.x) * WL_THREADS, k = k0 + threadIdx.x;
-    s_begin[threadIdx.x] = key_lower_bound(mt, n, kx, uint32_t(min(k, nkeys)));
+    const uint32_t b0 = key_lower_bound(mt, n, kx, uint32_t(min(k, nkeys)));
+    s_begin[threadIdx.x] = b0;
     if (threadIdx.x == 0)
         s_begin[WL_THREADS] = key_lower_bound(mt, n, kx, uint32_t(min(k0 + WL_THREADS, nkeys)));
+    if (threadIdx.x < 2 * NCAPS)
+        s_counts[threadIdx.x] = 0;
+    if (k <= nkeys)
+        begin[k] = b0;
     __syncthreads();
-    const uint32_t begin = s_begin[threadIdx.x], cnt = max(s_begin[threadIdx.x + 1], begin) - begin;
-    const uint32_t na = nchunks_for(cnt, a.cap), nb = nchunks_for(cnt, b.cap);
+    const uint32_t cnt = max(s_begin[threadIdx.x + 1], b0) - b0;
+    if (__any(cnt)) {
+        for (uint32_t j = 0; j < a.caps.n + b.caps.n; j++) {
+            const bool ina = j < a.caps.n;
+            const uint32_t sum = wave_reduce_add(nchunks_for(cnt, ina ? a.caps.cap[j] : b.caps.cap[j - a.caps.n]));
+            if (lane_id() == 0)
+                atomicAdd(&s_counts[ina ? j : NCAPS + j - a.caps.n], sum);
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < 2 * NCAPS && s_counts[threadIdx.x])
+        atomicAdd((threadIdx.x < NCAPS) ? a.cap_counts + threadIdx.x : b.cap_counts + threadIdx.x - NCAPS,
+                  s_counts[threadIdx.x]);
+}
+
+__device__ inline uint32_t chosen_cap(const WorkListOut &l)
+{
+    for (uint32_t j = 0; j + 1 < l.caps.n; j++)
+        if (l.cap_counts[j] <= l.caps.limit[j])
+            return l.caps.cap[j];
+    return l.caps.cap[l.caps.n - 1];
+}
+
+__global__ void __launch_bounds__(WL_THREADS)
+work_list_kernel(const uint32_t *__restrict__ begin, uint32_t kx, int64_t nkeys, WorkListOut a, WorkListOut b)
+{
+    __shared__ uint32_t s_wave[WL_THREADS / WAVE], s_base[2];
+    const int64_t k = int64_t(blockIdx.x) * WL_THREADS + threadIdx.x;
+    const uint32_t b0 = (k < nkeys) ? begin[k] : 0u, cnt = (k < nkeys) ? max(begin[k + 1], b0) - b0 : 0u;
+    const uint32_t cap_a = chosen_cap(a), cap_b = chosen_cap(b);
+    const uint32_t na = nchunks_for(cnt, cap_a), nb = nchunks_for(cnt, cap_b);
     uint32_t ta, tb;
     const uint32_t xa = block_exclusive_scan<WL_THREADS>(na, s_wave, ta);
     const uint32_t xb = block_exclusive_scan<WL_THREADS>(nb, s_wave, tb);
@@ -752,8 +786,8 @@ work_list_kernel(const uint64_t *__restrict__ mt, int64_t n, uint32_t kx, int64_
     __syncthreads();
     if (cnt > 0) {
         const uint32_t icell = cell_key(int(k / kx), int(k % kx));
-        store_chunks(icell, begin, cnt, a.cap, s_base[0] + xa, a.list, a.max_chunks);
-        store_chunks(icell, begin, cnt, b.cap, s_base[1] + xb, b.list, b.max_chunks);
+        store_chunks(icell, b0, cnt, cap_a, s_base[0] + xa, a.list, a.max_chunks);
+        store_chunks(icell, b0, cnt, cap_b, s_base[1] + xb, b.list, b.max_chunks);
     }
 }
 
@@ -943,8 +977,8 @@ __global__ void __launch_bounds__(PREPLAN_SIZE)
 plan_errors_kernel(const uint32_t *__restrict__ in, int n, uint32_t *__restrict__ err_word, uint32_t *__restrict__ counts)
 {
     gather_plan_errors(in, n, err_word, counts);
-    if (threadIdx.x == 0)
-        counts[PC_CHUNKS_M2T] = counts[PC_CHUNKS_T2M] = 0;
+    if (threadIdx.x < PC_TOTAL && threadIdx.x != PC_NMLINES && threadIdx.x != PC_ERROR)
+        counts[threadIdx.x] = 0;
 }
 
 // ------------------------------------------------------------------------------------------
@@ -977,21 +1011,26 @@ __device__ inline Chunk sp_unpack(uint32_t v, const uint64_t *items)
     return c;
 }
 
-// The list of chunks of at most 'cap' entries of the cells that start at start[0 .. ncells). In 'dst' in
-// order when there are at most SP_RANK, else in 'tmp' in any (the host then orders it).
+// The list of chunks of the cells that start at start[0 .. ncells). In 'dst' in order when there are at most SP_RANK, else in 'tmp' in any (the host then orders it).
 __device__ inline void sp_work_list(const uint64_t *items, const uint16_t *start, uint32_t ncells, const WorkListOut &l,
                                     Chunk *__restrict__ dst, uint32_t *s_key, uint32_t *s_wave)
 {
     const uint32_t t = threadIdx.x;
-    uint32_t mine = 0, total;
-    for (uint32_t c = t; c < ncells; c += SP_THREADS)
-        mine += nchunks_for(uint32_t(start[c + 1]) - start[c], l.cap);
-    uint32_t at = block_exclusive_scan<SP_THREADS>(mine, s_wave, total);
+    uint32_t at, total, cap;
+    for (uint32_t j = 0;; j++) {
+        cap = l.caps.cap[j];
+        uint32_t mine = 0;
+        for (uint32_t c = t; c < ncells; c += SP_THREADS)
+            mine += nchunks_for(uint32_t(start[c + 1]) - start[c], cap);
+        at = block_exclusive_scan<SP_THREADS>(mine, s_wave, total);
+        if (j + 1 >= l.caps.n || total <= l.caps.limit[j])
+            break;
+    }
     if (t == 0)
         *l.count = total;
     const bool ordered = total <= SP_RANK;
     for (uint32_t c = t; c < ncells; c += SP_THREADS) {
-        const uint32_t b = start[c], cnt = uint32_t(start[c + 1]) - b, nc = nchunks_for(cnt, l.cap);
+        const uint32_t b = start[c], cnt = uint32_t(start[c + 1]) - b, nc = nchunks_for(cnt, cap);
         for (uint32_t j = 0; j < nc; j++, at++) {
             const uint32_t v = sp_pack(b + cnt * j / nc, b + cnt * (j + 1) / nc, nc > 1);
             if (ordered)
@@ -1278,17 +1317,62 @@ SortLayout sort_layout(int64_t nmt)
     return L;
 }
 
+constexpr int64_t CAP_MIN = 128, CAP_MAX = 8192;         // entries per work unit
+
 // Lists of up to this many chunks are ordered by rank (n^2 comparisons: 16384 take about 40 us).
 constexpr int64_t RANK_MAX = 16384;
 
 WorkListOut m2t_out(const gmm_preplan &pp, const PlanLists &l, uint32_t *counts)
 {
-    return WorkListOut{l.tmp_m2t, l.max_m2t, uint32_t(pp.chunk_cap), counts + PC_CHUNKS_M2T};
+    return WorkListOut{l.tmp_m2t, l.max_m2t, pp.caps_m2t, counts + PC_CAPS_M2T, counts + PC_CHUNKS_M2T};
 }
 
 WorkListOut t2m_out(const gmm_preplan &pp, const PlanLists &l, uint32_t *counts)
 {
-    return WorkListOut{l.tmp_t2m, l.max_t2m, uint32_t(pp.chunk_cap_t2m), counts + PC_CHUNKS_T2M};
+    return WorkListOut{l.tmp_t2m, l.max_t2m, pp.caps_t2m, counts + PC_CAPS_T2M, counts + PC_CHUNKS_T2M};
+}
+
+// Sizes for a plan of nmt entries on 'slots' blocks that run at once: lists of at most k * slots chunks (k
+// full rounds) with chunks up to 5, 15, 30 and 50% above an even share, ordered by the time that the
+// rounds take when a block costs as much as 'fixed' entries; and last 'general', which any list may take.
+ChunkCaps make_caps(int64_t nmt, int64_t slots, int64_t fixed, int kmax, int64_t general)
+{
+    struct Option { int64_t cap, limit, cost; };
+    std::vector<Option> opt;
+    for (int k = 1; k <= kmax; k++)
+        for (int percent : {105, 115, 130, 150}) {
+            const int64_t share = k * slots * 100;
+            const int64_t cap = std::max<int64_t>(CAP_MIN, (nmt * percent + share - 1) / share);
+            if (cap <= CAP_MAX && int(opt.size()) < NCAPS - 1)
+                opt.push_back(Option{cap, k * slots, k * (fixed + cap)});
+        }
+    std::stable_sort(opt.begin(), opt.end(), [](const Option &a, const Option &b) { return a.cost < b.cost; });
+    ChunkCaps c = {};
+    for (const Option &o : opt) {
+        c.cap[c.n] = uint32_t(o.cap);
+        c.limit[c.n++] = uint32_t(o.limit);
+    }
+    c.cap[c.n] = uint32_t(general);
+    c.limit[c.n++] = 0xffffffffu;
+    return c;
+}
+
+int64_t max_chunks(const ChunkCaps &c, int64_t nmt, int64_t nkeys)
+{
+    int64_t n = (nmt + c.cap[c.n - 1] - 1) / c.cap[c.n - 1] + std::min(nmt, nkeys);
+    for (uint32_t j = 0; j + 1 < c.n; j++)
+        n = std::max(n, std::min<int64_t>(c.limit[j], nmt));
+    return n;
+}
+
+void launch_work_lists(const uint64_t *mt, int64_t n, uint32_t kx, int64_t nkeys, uint32_t *begin, const WorkListOut &a,
+                       const WorkListOut &b, hipStream_t stream)
+{
+    const unsigned grid = unsigned(nkeys / WL_THREADS + 1);             // begin[nkeys] too
+    cell_runs_kernel<<<grid, WL_THREADS, 0, stream>>>(mt, n, kx, nkeys, begin, a, b);
+    GMM_HIP(hipGetLastError());
+    work_list_kernel<<<grid, WL_THREADS, 0, stream>>>(begin, kx, nkeys, a, b);
+    GMM_HIP(hipGetLastError());
 }
 
 // Orders the lists, of at most max_m2t and max_t2m chunks (0: leaves that one alone).
@@ -1304,9 +1388,31 @@ void launch_rank(const PlanLists &l, const uint32_t *counts, int64_t max_m2t, in
 
 }  // namespace
 
+// Entries per work unit of the operators. A tod2map block clears and flushes a 116 KiB tile, atomically
+// when its cell is split, and has its CU to itself: lists are cut for one to three full rounds of the 256
+// CUs where their cells allow it (tod2map with chunks of half a CU's share against this, in us: 145 000
+// entries of 64 x 65536 samples 36 / 32; rotated scans of 256 and 1024 x 65536 131 / 92 and 388 / 323; the
+// fast one of 768 x 50004 311 / 275; with one round as the only choice the last two gain nothing; rasters
+// over more cells than that the same). map2tod, two blocks a CU and bound by memory, balances best in many
+// small chunks (263 us on the 768 x 50004; 285 with tod2map's), except when they would not fill a round
+// (64 x 65536 samples 25.8 us in chunks of 512, 22.7 in one round; 8 x 4096 10.9 and 9.5).
+constexpr int64_t TILE_COST = 700, STAGE_COST = 100;     // a block's fixed work, in entries
+
+void plan_chunk_caps(gmm_preplan &pp)
+{
+    const int64_t nmt = pp.plan_nmt, nkeys = pp.nycells_g * pp.nxcells_g, cus = 256;
+    const int64_t m2t = std::min(CAP_MAX, std::max<int64_t>(512, (nmt + 12 * cus - 1) / (12 * cus)));
+    const int64_t t2m = std::min(CAP_MAX, std::max<int64_t>(1024, (nmt + 2 * cus - 1) / (2 * cus)));
+    pp.caps_m2t = make_caps(nmt, 2 * cus, STAGE_COST, (nmt <= 512 * 2 * cus) ? 1 : 0, m2t);
+    pp.caps_t2m = make_caps(nmt, cus, TILE_COST, 3, t2m);
+    pp.max_nchunks = max_chunks(pp.caps_m2t, nmt, nkeys);
+    pp.max_nchunks_t2m = max_chunks(pp.caps_t2m, nmt, nkeys);
+}
+
 int64_t plan_scratch_nbytes(const gmm_preplan &pp)
 {
-    return sort_layout(pp.plan_nmt).total + align128(int64_t(sizeof(Chunk)) * (pp.max_nchunks + pp.max_nchunks_t2m));
+    return sort_layout(pp.plan_nmt).total + align128(int64_t(sizeof(Chunk)) * (pp.max_nchunks + pp.max_nchunks_t2m))
+         + align128(4 * (pp.nycells_g * pp.nxcells_g + 1));
 }
 
 PlanLists plan_lists(const gmm_preplan &pp, Chunk *m2t, Chunk *t2m, void *scratch)
@@ -1318,6 +1424,8 @@ PlanLists plan_lists(const gmm_preplan &pp, Chunk *m2t, Chunk *t2m, void *scratc
     l.max_t2m = pp.max_nchunks_t2m;
     l.tmp_m2t = reinterpret_cast<Chunk *>(static_cast<uint8_t *>(scratch) + sort_layout(pp.plan_nmt).total);
     l.tmp_t2m = l.tmp_m2t + pp.max_nchunks;
+    l.begin = reinterpret_cast<uint32_t *>(static_cast<uint8_t *>(scratch) + plan_scratch_nbytes(pp)
+                                           - align128(4 * (pp.nycells_g * pp.nxcells_g + 1)));
     return l;
 }
 
@@ -1359,9 +1467,8 @@ void plan_schedule(const gmm_preplan &pp, const uint64_t *sorted_mt, const PlanL
 {
     const int64_t n = pp.plan_nmt;
     const int64_t nkeys = pp.nycells_g * pp.nxcells_g;
-    work_list_kernel<<<unsigned((nkeys + WL_THREADS - 1) / WL_THREADS), WL_THREADS, 0, stream>>>(
-        sorted_mt, n, uint32_t(pp.nxcells_g), nkeys, m2t_out(pp, l, counts_gpu), t2m_out(pp, l, counts_gpu));
-    GMM_HIP(hipGetLastError());
+    launch_work_lists(sorted_mt, n, uint32_t(pp.nxcells_g), nkeys, l.begin, m2t_out(pp, l, counts_gpu),
+                      t2m_out(pp, l, counts_gpu), stream);
     if (l.max_m2t <= RANK_MAX && l.max_t2m <= RANK_MAX)
         launch_rank(l, counts_gpu, l.max_m2t, l.max_t2m, stream);
 }
@@ -1369,8 +1476,10 @@ void plan_schedule(const gmm_preplan &pp, const uint64_t *sorted_mt, const PlanL
 void plan_small(const gmm_preplan &pp, const uint64_t *items, uint64_t *out, uint16_t *qmask, const PlanLists &l,
                 const uint32_t *err_in, uint32_t *err_word, uint32_t *counts_gpu, hipStream_t stream)
 {
-    GMM_REQUIRE(pp.plan_nmt <= SP_MAX && pp.chunk_cap < (1 << SP_LEN_BITS) && pp.chunk_cap_t2m < (1 << SP_LEN_BITS),
-                "plan_small: plan too large");
+    uint32_t cap = 0;
+    for (const ChunkCaps *c : {&pp.caps_m2t, &pp.caps_t2m})
+        cap = std::max(cap, *std::max_element(c->cap, c->cap + c->n));
+    GMM_REQUIRE(pp.plan_nmt <= SP_MAX && cap < (1u << SP_LEN_BITS), "plan_small: plan too large");
     small_plan_kernel<<<1, SP_THREADS, 0, stream>>>(items, uint32_t(pp.plan_nmt), uint32_t(pp.nxcells_g), pp.key_bits, out,
                                                     qmask, m2t_out(pp, l, counts_gpu), t2m_out(pp, l, counts_gpu), l.m2t,
                                                     l.t2m, err_in, int(pp.pparams.planner_nblocks), err_word, counts_gpu);
@@ -1433,18 +1542,25 @@ void order_long_lists(const gmm_preplan &pp, const PlanLists &l, int64_t n_m2t, 
     order(l.tmp_t2m, l.t2m, n_t2m);
 }
 
+constexpr int64_t GENERIC_KEYS = int64_t(1) << 20;
+
+int64_t build_chunks_generic_scratch_nbytes() { return align128(4 * (GENERIC_KEYS + 1)) + 128; }
+
 int64_t build_chunks_generic(const uint64_t *plan_mt_gpu, int64_t nmt, int64_t chunk_cap,
-                             Chunk *chunks_gpu, int64_t max_chunks, uint32_t *counts, hipStream_t stream)
+                             Chunk *chunks_gpu, int64_t max_chunks, void *scratch, hipStream_t stream)
 {
-    const int64_t nkeys = int64_t(1) << 20;
-    fill_u32_kernel<<<1, 64, 0, stream>>>(counts, 2, 0u);
-    const WorkListOut a{chunks_gpu, max_chunks, uint32_t(chunk_cap), counts}, b{chunks_gpu, 0, uint32_t(nmt), counts + 1};
-    work_list_kernel<<<unsigned(nkeys / WL_THREADS), WL_THREADS, 0, stream>>>(plan_mt_gpu, nmt, 1024u, nkeys, a, b);
+    uint32_t *begin = static_cast<uint32_t *>(scratch);
+    uint32_t *counts = begin + align128(4 * (GENERIC_KEYS + 1)) / 4;
+    fill_u32_kernel<<<1, 64, 0, stream>>>(counts, PC_TOTAL, 0u);
     GMM_HIP(hipGetLastError());
-    uint32_t h = 0;
-    GMM_HIP(hipMemcpyAsync(&h, counts, 4, hipMemcpyDeviceToHost, stream));
-    GMM_HIP(hipStreamSynchronize(stream));
-    return int64_t(h);
+    ChunkCaps cap = {}, none = {};
+    cap.n = none.n = 1;
+    cap.cap[0] = uint32_t(chunk_cap);
+    none.cap[0] = 1u << 30;
+    const WorkListOut a{chunks_gpu, max_chunks, cap, counts + PC_CAPS_M2T, counts + PC_CHUNKS_M2T};
+    const WorkListOut b{chunks_gpu, 0, none, counts + PC_CAPS_T2M, counts + PC_CHUNKS_T2M};
+    launch_work_lists(plan_mt_gpu, nmt, 1024u, GENERIC_KEYS, begin, a, b, stream);
+    return int64_t(read_word(counts + PC_CHUNKS_M2T, stream));
 }
 
 void launch_fill_u32(uint32_t *p, int64_t n, uint32_t v, hipStream_t stream)

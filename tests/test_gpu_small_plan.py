@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 import torch
 
-from test_gpu_work_lists import CHUNK, align128, check_list, make_pointing
+from test_gpu_work_lists import CHUNK, align128, bound, check_list, make_pointing, sizes
 
 pytestmark = pytest.mark.gpu
 
@@ -28,7 +28,7 @@ def test_small_plan(gmm, orc, dev, kind, n, ny, nx):
     nmt, nkeys = pre.plan_nmt, -(-ny // 64) * -(-nx // 64)
     buf = plan.buf.cpu().numpy()
     end = pre.plan_nbytes - align128(2 * nmt)
-    for cap in (1024, 512):                              # tod2map's list, before it map2tod's
-        nmax = -(-nmt // cap) + min(nmt, nkeys)
+    for opt in sizes(nmt)[::-1]:                         # tod2map's list, before it map2tod's
+        nmax = bound(opt, nmt, nkeys)
         end -= align128(16 * nmax)
-        check_list(buf[end:end + 16 * nmax].view(CHUNK), mt, cap, True)
+        check_list(buf[end:end + 16 * nmax].view(CHUNK), mt, opt, True)

@@ -1,6 +1,6 @@
 """The operators' work lists: every run of a cell's entries is cut into equal chunks of at most the
-list's size, the chunks are marked when they share a cell, and the list goes from the largest to the
-smallest. Lists short enough to be ranked (equal ones then in plan order), possibly long but short in
+list's size (one that fits full rounds of the card's blocks, where there is one), the chunks are marked
+when they share a cell, and the list goes from the largest to the smallest. Lists short enough to be ranked (equal ones then in plan order), possibly long but short in
 fact, and long ones, which a radix sort orders.
 """
 
@@ -28,10 +28,27 @@ def make_pointing(kind, n, ny, nx):
     return np.stack([y, x, 0 * y]).astype(np.float32)
 
 
-def check_list(chunks, mt, cap, ranked):
+def sizes(nmt):
+    """(cap, limit) options of map2tod's and of tod2map's list, in the order of preference."""
+    def options(slots, fixed, kmax, general):
+        opt = [(max(128, -(-nmt * m // (100 * k * slots))), k * slots) for k in range(1, kmax + 1)
+               for m in (105, 115, 130, 150)]
+        opt = [o for o in opt if o[0] <= 8192][:11]
+        opt.sort(key=lambda o: o[1] // slots * (fixed + o[0]))
+        return opt + [(general, 1 << 32)]
+    return (options(512, 100, 1 if nmt <= 512 * 512 else 0, min(8192, max(512, -(-nmt // 3072)))),
+            options(256, 700, 3, min(8192, max(1024, -(-nmt // 512)))))
+
+
+def bound(opt, nmt, nkeys):
+    return max([-(-nmt // opt[-1][0]) + min(nmt, nkeys)] + [min(lim, nmt) for _, lim in opt[:-1]])
+
+
+def check_list(chunks, mt, opt, ranked):
     cell = mt & np.uint64(0xfffff)
     begin = np.flatnonzero(np.r_[True, cell[1:] != cell[:-1]])
     cnt = np.diff(np.r_[begin, len(mt)])
+    cap = next(cap for cap, lim in opt if ((cnt + cap - 1) // cap).sum() <= lim)
     nc = (cnt + cap - 1) // cap
     want = [(int(cell[b]), b + c * j // m, b + c * (j + 1) // m, int(m > 1))
             for b, c, m in zip(begin.tolist(), cnt.tolist(), nc.tolist()) for j in range(m)]
@@ -46,7 +63,8 @@ def check_list(chunks, mt, cap, ranked):
 @pytest.mark.parametrize("kind,n,ny,nx", [
     ("one cell", 1, 200, 330), ("one cell", 32 * 512, 200, 330), ("one cell", 32 * 1024 + 1, 200, 330),
     ("one cell", 32 * 70001, 200, 330), ("lines", 32 * 4096, 640, 1281), ("samples", 20000, 640, 1281),
-    ("lines", 32 * 1000, 8960, 8960), ("samples", 16384, 8960, 8960), ("samples", 60000, 8960, 8960)])
+    ("lines", 32 * 15000, 640, 640), ("lines", 32 * 15000, 300, 300), ("lines", 32 * 70000, 1000, 2000),
+    ("lines", 32 * 70000, 1600, 2000), ("lines", 32 * 1000, 8960, 8960), ("samples", 16384, 8960, 8960), ("samples", 60000, 8960, 8960)])
 def test_work_lists(gmm, dev, kind, n, ny, nx):
     xg = torch.from_numpy(make_pointing(kind, n, ny, nx)).to(dev)
     pre = gmm.PointingPrePlan(xg, ny, nx, periodic_xcoord=False)
@@ -55,9 +73,9 @@ def test_work_lists(gmm, dev, kind, n, ny, nx):
     nkeys = -(-ny // 64) * -(-nx // 64)
     buf = plan.buf.cpu().numpy()
     end = pre.plan_nbytes - align128(2 * nmt)           # the owned-quad masks end the buffer
-    caps = min(8192, max(512, -(-nmt // 3072))), min(8192, max(1024, -(-nmt // 512)))
-    bound = [-(-nmt // cap) + min(nmt, nkeys) for cap in caps]
-    assert pre.max_nchunks == bound[0]
-    for cap, nmax in zip(caps[::-1], bound[::-1]):      # tod2map's list, before it map2tod's
+    opts = sizes(nmt)
+    bounds = [bound(opt, nmt, nkeys) for opt in opts]
+    assert pre.max_nchunks == bounds[0]
+    for opt, nmax in zip(opts[::-1], bounds[::-1]):     # tod2map's list, before it map2tod's
         end -= align128(16 * nmax)
-        check_list(buf[end:end + 16 * nmax].view(CHUNK), mt, cap, max(bound) <= RANK_MAX)
+        check_list(buf[end:end + 16 * nmax].view(CHUNK), mt, opt, max(bounds) <= RANK_MAX)
