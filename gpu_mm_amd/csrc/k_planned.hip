@@ -563,8 +563,11 @@ __device__ inline void m2t_entries(TT *__restrict__ tod, const float *__restrict
 
     for (uint32_t base = wb; base < we; base += 64) {
         const uint32_t cnt = min(64u, we - base);
-        const uint32_t packed = (uint32_t(lane) < cnt) ? pack_entry(plan_mt[base + lane]) : 0u;
-        const uint32_t qmw = (uint32_t(lane) < cnt) ? uint32_t(qmask[base + lane]) : 0u;
+        const uint32_t at = base + min(uint32_t(lane), cnt - 1);           // both loads at once
+        const uint64_t mt_l = plan_mt[at];
+        const uint32_t qm_l = qmask[at];
+        const uint32_t packed = (uint32_t(lane) < cnt) ? pack_entry(mt_l) : 0u;
+        const uint32_t qmw = (uint32_t(lane) < cnt) ? qm_l : 0u;
 
         for (uint32_t j = 0; j < cnt; j += 8) {
             const uint32_t idx = j + li;
@@ -1155,8 +1158,11 @@ __device__ inline void t2m_entries(unsigned long long *__restrict__ acc, float *
     for (uint32_t base = wb; base < we; base += 64) {
         const uint32_t cnt = min(64u, we - base);
         const bool valid = uint32_t(lane) < cnt;
-        const uint32_t packed = valid ? pack_entry(plan_mt[base + lane]) : 0u;
-        const uint32_t qmw = valid ? uint32_t(qmask[base + lane]) : 0u;
+        const uint32_t at = base + min(uint32_t(lane), cnt - 1);           // both loads at once
+        const uint64_t mt_l = plan_mt[at];
+        const uint32_t qm_l = qmask[at];
+        const uint32_t packed = valid ? pack_entry(mt_l) : 0u;
+        const uint32_t qmw = valid ? qm_l : 0u;
         const uint32_t icl_l = packed & ICL_MASK;
         if (valid && icl_l >= ncl)
             err |= ERR_INCONSISTENT_NMT;
