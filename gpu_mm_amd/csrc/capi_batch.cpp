@@ -190,6 +190,8 @@ BatchLaunch launch_of(const gmm_batch &b, const DeviceTables &t, int op)
     bl.grid = t.grid;
     bl.threads = t.threads;
     bl.has_resp = b.has_resp;
+    for (const BatchTod &t : b.tods)
+        bl.whole_rows = bl.whole_rows && (!t.scale || t.scale_div.nper % 4 == 0) && (!t.resp || t.resp_div.nper % 4 == 0);
     return bl;
 }
 

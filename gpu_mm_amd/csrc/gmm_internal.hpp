@@ -278,6 +278,7 @@ struct BatchLaunch
     int64_t grid = 0;
     int threads = 512;
     bool has_resp = false;      // every TOD has per-detector gains (FP32 TODs only)
+    bool whole_rows = true;     // the rows of every TOD's gains and scales are multiples of 4 samples long
 };
 
 void launch_batched_map2tod(const BatchLaunch &bl, const float *lmap, const gmm_lpix &lp, int tod_type, bool partial,

@@ -249,19 +249,13 @@ struct Gains
     RowDiv resp_div, scale_div;
 };
 
-// Row of each of the 4 samples s0..s0+3 (s0 a multiple of 4) for rows of d.nper samples. When
-// nper is a multiple of 4 the quad lies in one row (one multiplication); otherwise it crosses at
-// most one row boundary when nper >= 4. Only the first nv samples exist (nv < 4 for the last
+// Row of each of the 4 samples s0..s0+3 (s0 a multiple of 4) for rows of d.nper samples. The quad
+// crosses at most one row boundary when nper >= 4. Only the first nv samples exist (nv < 4 for the last
 // group of a TOD whose length is not a multiple of 4): the others take the row of the last.
 __device__ inline void quad_rows(uint32_t s0, const RowDiv &d, uint32_t (&r)[4], uint32_t nv = 4)
 {
     const uint32_t r0 = rowdiv(s0, d);
-    if ((d.nper & 3u) == 0) {
-#pragma unroll
-        for (int k = 0; k < 4; k++)
-            r[k] = r0;
-    }
-    else if (d.nper >= 4) {
+    if (d.nper >= 4) {
         const uint32_t b = (r0 + 1) * d.nper - s0;  // samples of the quad in row r0
 #pragma unroll
         for (int k = 0; k < 4; k++)
@@ -274,28 +268,35 @@ __device__ inline void quad_rows(uint32_t s0, const RowDiv &d, uint32_t (&r)[4],
     }
 }
 
-// T and P gain of the 4 samples of a quad (1 without a response array).
-template<bool HasResp>
+// Gains of the 4 samples of a quad (1 without a response array; scales of 16-bit TODs, whose length is a
+// multiple of 4). Whole: the rows are multiples of 4 samples long, so that a quad has one gain. Chosen at
+// run time, the kernels, which have no registers to spare, held four of each: on 768 x 50004 16-bit
+// samples with gains map2tod 260 -> 234 us and tod2map 269 -> 232 with the choice at launch; batched on
+// 4 x 512 x 131072 with gains 1095 -> 967 and 1182 -> 1168.
+template<bool Whole>
+__device__ inline void quad_values(const float *__restrict__ v, uint32_t s0, const RowDiv &d, float (&out)[4], uint32_t nv)
+{
+    if (Whole) {
+        const float x = v[rowdiv(s0, d)];
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            out[k] = x;
+    }
+    else {
+        uint32_t r[4];
+        quad_rows(s0, d, r, nv);
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            out[k] = v[r[k]];
+    }
+}
+
+template<bool HasResp, bool Whole>
 __device__ inline void quad_resp(const Gains &g, uint32_t s0, float (&tr)[4], float (&pr)[4], uint32_t nv = 4)
 {
     if (HasResp) {
-        uint32_t d[4];
-        quad_rows(s0, g.resp_div, d, nv);
-        if ((g.resp_div.nper & 3u) == 0) {
-            const float t = g.resp[d[0]], p = g.resp[g.resp_ndet + d[0]];
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                tr[k] = t;
-                pr[k] = p;
-            }
-        }
-        else {
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                tr[k] = g.resp[d[k]];
-                pr[k] = g.resp[g.resp_ndet + d[k]];
-            }
-        }
+        quad_values<Whole>(g.resp, s0, g.resp_div, tr, nv);
+        quad_values<Whole>(g.resp + g.resp_ndet, s0, g.resp_div, pr, nv);
     }
     else {
 #pragma unroll
@@ -304,8 +305,7 @@ __device__ inline void quad_resp(const Gains &g, uint32_t s0, float (&tr)[4], fl
     }
 }
 
-// Scale of the 4 samples of a quad (16-bit TODs only; their length is a multiple of 4).
-template<typename TT>
+template<typename TT, bool Whole>
 __device__ inline void quad_scale(const Gains &g, uint32_t s0, float (&sc)[4])
 {
     if constexpr (std::is_same<TT, float>::value) {
@@ -313,21 +313,8 @@ __device__ inline void quad_scale(const Gains &g, uint32_t s0, float (&sc)[4])
         for (int k = 0; k < 4; k++)
             sc[k] = 1.0f;
     }
-    else {
-        uint32_t r[4];
-        quad_rows(s0, g.scale_div, r);
-        if ((g.scale_div.nper & 3u) == 0) {
-            const float v = g.scale[r[0]];
-#pragma unroll
-            for (int k = 0; k < 4; k++)
-                sc[k] = v;
-        }
-        else {
-#pragma unroll
-            for (int k = 0; k < 4; k++)
-                sc[k] = g.scale[r[k]];
-        }
-    }
+    else
+        quad_values<Whole>(g.scale, s0, g.scale_div, sc, 4);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -549,7 +536,7 @@ __device__ inline float m2t_sample(const float4 *__restrict__ tile, const float2
 // map2tod of plan entries [wb, we) of one TOD by the calling wave, with the halo tile of the
 // block's cell (whose top-left pixel is (ybase, xbase)) in LDS. Every sample is written once, by
 // the block that owns it: no atomics and no zeroing.
-template<bool Periodic, bool Vec, bool HasResp, typename TT, bool Debug = false>
+template<bool Periodic, bool Vec, bool HasResp, bool Whole, typename TT, bool Debug = false>
 __device__ inline void m2t_entries(TT *__restrict__ tod, const float *__restrict__ xp,
                                    const uint64_t *__restrict__ plan_mt, const uint16_t *__restrict__ qmask,
                                    int64_t nsamp, uint32_t wb, uint32_t we, const float4 *__restrict__ tile,
@@ -592,8 +579,8 @@ __device__ inline void m2t_entries(TT *__restrict__ tod, const float *__restrict
             const float4 x4 = Vec ? load4_nt(xp + nsamp + s0) : load4n<Vec>(xp + nsamp + s0, nv);
             const float4 a4 = Vec ? load4_nt(xp + 2 * nsamp + s0) : load4n<Vec>(xp + 2 * nsamp + s0, nv);
             float tr[4], pr[4], sc[4];
-            quad_resp<HasResp>(gn, uint32_t(s0), tr, pr, nv);
-            quad_scale<TT>(gn, uint32_t(s0), sc);
+            quad_resp<HasResp, Whole>(gn, uint32_t(s0), tr, pr, nv);
+            quad_scale<TT, Whole>(gn, uint32_t(s0), sc);
 
             bool o0, o1, o2, o3;
             float4 v;
@@ -661,7 +648,7 @@ __device__ inline uint32_t claim_batch(uint32_t n, uint32_t nwaves)
     return min(64u, max(8u, (per + 7u) & ~7u));
 }
 
-template<bool Periodic, bool Vec, bool HasResp, typename TT, bool Debug = false>
+template<bool Periodic, bool Vec, bool HasResp, bool Whole, typename TT, bool Debug = false>
 __global__ void __launch_bounds__(M2T_THREADS, 4)
 planned_map2tod_kernel(TT *__restrict__ tod, const float *__restrict__ lmap, const float *__restrict__ xp,
                        const int64_t *__restrict__ cell_offsets, const uint64_t *__restrict__ plan_mt,
@@ -694,7 +681,7 @@ planned_map2tod_kernel(TT *__restrict__ tod, const float *__restrict__ lmap, con
     if (n < M2T_DYNAMIC_MIN) {
         uint32_t wb, we;
         wave_slice(ch, int(threadIdx.x >> 6), M2T_THREADS / WAVE, wb, we);
-        m2t_entries<Periodic, Vec, HasResp, TT, Debug>(tod, xp, plan_mt, qmask, nsamp, wb, we, tile, sct, g, ybase,
+        m2t_entries<Periodic, Vec, HasResp, Whole, TT, Debug>(tod, xp, plan_mt, qmask, nsamp, wb, we, tile, sct, g, ybase,
                                                        xbase, accum, gn, chk, err, dbg);
     }
     else {
@@ -705,7 +692,7 @@ planned_map2tod_kernel(TT *__restrict__ tod, const float *__restrict__ lmap, con
             b = __builtin_amdgcn_readfirstlane(b);
             if (b >= n)
                 break;
-            m2t_entries<Periodic, Vec, HasResp, TT, Debug>(tod, xp, plan_mt, qmask, nsamp, ch.begin + b,
+            m2t_entries<Periodic, Vec, HasResp, Whole, TT, Debug>(tod, xp, plan_mt, qmask, nsamp, ch.begin + b,
                                                            ch.begin + min(b + 64u, n), tile, sct, g, ybase, xbase,
                                                            accum, gn, chk, err, dbg);
         }
@@ -1069,7 +1056,7 @@ __device__ inline void wave_compact_offsets(uint32_t n, uint32_t &excl, uint32_t
 
 // Largest |t| (times the gains) over the first 8 plan entries of [wb, we), for the calling
 // lane (lane 8*li + q reads quad q of entry wb + li); 'act' tells whether the lane read samples.
-template<bool Vec, bool HasResp, typename TT>
+template<bool Vec, bool HasResp, bool Whole, typename TT>
 __device__ inline float t2m_probe(const TT *__restrict__ tod, const uint64_t *__restrict__ plan_mt, int64_t nsamp,
                                   uint32_t wb, uint32_t we, const Gains &gn, bool &act)
 {
@@ -1090,8 +1077,8 @@ __device__ inline float t2m_probe(const TT *__restrict__ tod, const uint64_t *__
             const uint32_t nv = uint32_t(min<int64_t>(4, nsamp - s0));
             const float4 t4 = IO::load_n(tod + s0, nv);
             float tr[4], pr[4], sc[4];
-            quad_resp<HasResp>(gn, uint32_t(s0), tr, pr, nv);
-            quad_scale<TT>(gn, uint32_t(s0), sc);
+            quad_resp<HasResp, Whole>(gn, uint32_t(s0), tr, pr, nv);
+            quad_scale<TT, Whole>(gn, uint32_t(s0), sc);
             const float tv[4] = { t4.x, t4.y, t4.z, t4.w };
 #pragma unroll
             for (int k = 0; k < 4; k++) {
@@ -1129,86 +1116,63 @@ __device__ inline uint32_t wave_probe_bound(float m, bool act)
     return (lo >= 254) ? FINITE_LIMIT : uint32_t(lo + 1) << 23;
 }
 
+constexpr int ITEM_QUAD_SHIFT = 26;                     // above the line index (ICL_MASK)
+constexpr uint32_t ITEM_TAKES_RIGHT = 1u << 29;
+
 // tod2map of plan entries [wb, we) of one TOD by the calling wave into the block's halo tile:
 // fixed point with scale 'scale' when 'finite', else float atomics. In fixed point a group whose
 // largest |t| (times the gains) is below 'limit' takes the 32-bit path, any other group (an
 // outlier) deposits sample by sample in 64-bit fixed point and counts in nwide. Tracks per lane
 // the largest |t| of its outlier groups (mrun) and a sum that is NaN whenever a value it deposits
 // is NaN (tsum; an outlier group adds all of its samples).
-template<bool Periodic, bool Vec, bool HasResp, typename TT, bool Debug = false>
+template<bool Periodic, bool Vec, bool HasResp, bool Whole, typename TT, bool Debug = false>
 __device__ inline void t2m_entries(unsigned long long *__restrict__ acc, float *__restrict__ facc,
                                    const TT *__restrict__ tod, const float *__restrict__ xp,
                                    const uint64_t *__restrict__ plan_mt, const uint16_t *__restrict__ qmask,
                                    int64_t nsamp, uint32_t wb, uint32_t we, const float2 *__restrict__ sct,
                                    const Geom &g, int ybase, int xbase, const Gains &gn, bool finite, float scale,
                                    float limit, float &mrun, float &tsum, uint32_t &nwide, Checks &chk, uint32_t &err,
-                                   uint16_t *__restrict__ wlist, const Dbg &dbg = Dbg{}, bool count = false)
+                                   uint32_t *__restrict__ wlist, const Dbg &dbg = Dbg{}, bool count = false)
 {
     constexpr bool Q16 = !std::is_same<TT, float>::value;
     using IO = TodIO<TT, Vec>;
     const int lane = threadIdx.x & 63;
     const uint32_t ncl = uint32_t((nsamp + 31) >> 5);     // the last line may be partial
-    // When the rows of a gain array (16-bit scales, response) are a multiple of 32 samples long, a
-    // line's samples share one gain: it is loaded once per entry and broadcast with the entry
-    // (FP16 tod2map 1% faster than a lookup per group; map2tod, bound by memory latency, was
-    // slower this way and keeps the lookup per group).
-    const bool line_sc = Q16 && (gn.scale_div.nper & 31u) == 0;
-    const bool line_resp = HasResp && (gn.resp_div.nper & 31u) == 0;
 
     for (uint32_t base = wb; base < we; base += 64) {
         const uint32_t cnt = min(64u, we - base);
         const bool valid = uint32_t(lane) < cnt;
         const uint32_t at = base + min(uint32_t(lane), cnt - 1);           // both loads at once
-        const uint64_t mt_l = plan_mt[at];
-        const uint32_t qm_l = qmask[at];
-        const uint32_t packed = valid ? pack_entry(mt_l) : 0u;
-        const uint32_t qmw = valid ? qm_l : 0u;
-        const uint32_t icl_l = packed & ICL_MASK;
-        if (valid && icl_l >= ncl)
+        const uint32_t icl = uint32_t(plan_mt[at] >> ICL_SHIFT) & ICL_MASK;
+        const uint32_t qm = qmask[at];
+        if (valid && icl >= ncl)
             err |= ERR_INCONSISTENT_NMT;
-        float scl = 1.0f, trl = 1.0f, prl = 1.0f;
-        if ((line_sc || line_resp) && valid && icl_l < ncl) {
-            const uint32_t sl = icl_l * LINE;
-            if (line_sc)
-                scl = gn.scale[rowdiv(sl, gn.scale_div)];
-            if (line_resp) {
-                const uint32_t d = rowdiv(sl, gn.resp_div);
-                trl = gn.resp[d];
-                prl = gn.resp[gn.resp_ndet + d];
-            }
-        }
         if constexpr (Debug) {
             if (count && valid)
                 atomicAdd(dbg.entry_visits + (base + lane), 1u);
         }
         // The batch's evaluated 4-sample groups (the quad bits of the entries' masks), compacted
-        // into the wave's LDS list as items (entry, quad) in entry order, so that every lane of a
-        // step has a group: with one lane per (entry, quad) of 8 entries, the quads that an entry
-        // does not evaluate left lanes idle (13% of them on a raster, 20% on fast rotated scans).
-        const uint32_t qb = (valid && icl_l < ncl) ? (qmw & 0xFFu) : 0u;
+        // into the wave's LDS list in entry order, one word each, so that every lane of a step has a
+        // group: with one lane per (entry, quad) of 8 entries, the quads that an entry does not
+        // evaluate left lanes idle (13% of them on a raster, 20% on fast rotated scans).
+        const uint32_t qb = (valid && icl < ncl) ? (qm & 0xFFu) : 0u;
+        const uint32_t line = icl | ((qm & QM_TAKES_RIGHT) ? ITEM_TAKES_RIGHT : 0u);
         uint32_t pos, total;
         wave_compact_offsets(__popc(qb), pos, total);
         for (uint32_t bits = qb; bits; bits &= bits - 1)
-            wlist[pos++] = uint16_t((uint32_t(lane) << 3) | uint32_t(__builtin_ctz(bits)));
+            wlist[pos++] = line | (uint32_t(__builtin_ctz(bits)) << ITEM_QUAD_SHIFT);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 
         for (uint32_t r = 0; r < total; r += 64) {
             const uint32_t item = r + uint32_t(lane);
-            const uint32_t code = (item < total) ? uint32_t(wlist[item]) : 0u;
-            const int li = int(code >> 3), q = int(code & 7u);
-            const uint32_t e2 = __shfl(packed, li, WAVE);
-            const uint32_t qm = __shfl(qmw, li, WAVE);
-            const float sce = line_sc ? __shfl(scl, li, WAVE) : 1.0f;
-            const float tre = line_resp ? __shfl(trl, li, WAVE) : 1.0f;
-            const float pre = line_resp ? __shfl(prl, li, WAVE) : 1.0f;
+            const uint32_t code = wlist[min(item, total - 1)];
             // Columns of the right-hand cell that this entry evaluates (ownership rule at HALO_X).
-            const unsigned lxlim = (qm & QM_TAKES_RIGHT) ? unsigned(64 + HALO_X - 1) : 64u;
-            const uint32_t icl = e2 & ICL_MASK;
+            const unsigned lxlim = (code & ITEM_TAKES_RIGHT) ? unsigned(64 + HALO_X - 1) : 64u;
             if (item >= total)
                 continue;
-            const int64_t s0 = int64_t(icl) * LINE + 4 * q;
+            const int64_t s0 = int64_t(code & ICL_MASK) * LINE + 4 * ((code >> ITEM_QUAD_SHIFT) & 7u);
             // Past the end of the TOD (nv < 4) the samples read as zeros: they deposit nothing.
             const uint32_t nv = uint32_t(min<int64_t>(4, nsamp - s0));
             // Non-temporal: the pointing and TOD stream through once, while the cell's map lines
@@ -1222,22 +1186,8 @@ __device__ inline void t2m_entries(unsigned long long *__restrict__ acc, float *
             else
                 t4 = IO::load_n(tod + s0, nv);
             float tr[4], pr[4], sc[4];
-            if (line_resp) {
-#pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    tr[k] = tre;
-                    pr[k] = pre;
-                }
-            }
-            else
-                quad_resp<HasResp>(gn, uint32_t(s0), tr, pr, nv);
-            if (line_sc) {
-#pragma unroll
-                for (int k = 0; k < 4; k++)
-                    sc[k] = sce;
-            }
-            else
-                quad_scale<TT>(gn, uint32_t(s0), sc);
+            quad_resp<HasResp, Whole>(gn, uint32_t(s0), tr, pr, nv);
+            quad_scale<TT, Whole>(gn, uint32_t(s0), sc);
             if (Q16) {
                 t4.x *= sc[0];
                 t4.y *= sc[1];
@@ -1570,7 +1520,7 @@ __device__ inline bool t2m_accumulate(unsigned long long *__restrict__ acc, uint
     return finite;
 }
 
-template<bool Periodic, bool Vec, bool HasResp, typename TT, bool Debug = false>
+template<bool Periodic, bool Vec, bool HasResp, bool Whole, typename TT, bool Debug = false>
 __global__ void __launch_bounds__(T2M_THREADS)
 planned_tod2map_kernel(float *__restrict__ lmap, const TT *__restrict__ tod, const float *__restrict__ xp,
                        const int64_t *__restrict__ cell_offsets, const uint64_t *__restrict__ plan_mt,
@@ -1581,7 +1531,7 @@ planned_tod2map_kernel(float *__restrict__ lmap, const TT *__restrict__ tod, con
     __shared__ __align__(16) unsigned long long acc[3 * HPLANE];       // 116 KiB
     __shared__ float2 sct[SCT];
     __shared__ uint32_t s_words[T2M_WORDS];
-    __shared__ uint16_t s_list[T2M_THREADS / WAVE][T2M_LIST];            // 16 KiB
+    __shared__ uint32_t s_list[T2M_THREADS / WAVE][T2M_LIST];            // 32 KiB
     float *facc = reinterpret_cast<float *>(acc);         // float tile for the non-finite fallback
 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1606,7 +1556,7 @@ planned_tod2map_kernel(float *__restrict__ lmap, const TT *__restrict__ tod, con
     __syncthreads();
     {
         bool act;
-        const float m = t2m_probe<Vec, HasResp, TT>(tod, plan_mt, nsamp, wb, we, gn, act);
+        const float m = t2m_probe<Vec, HasResp, Whole, TT>(tod, plan_mt, nsamp, wb, we, gn, act);
         const uint32_t mw = wave_probe_bound(m, act);
         if (lane == 0)
             atomicMax(&s_words[W_MAX], mw);
@@ -1633,7 +1583,7 @@ planned_tod2map_kernel(float *__restrict__ lmap, const TT *__restrict__ tod, con
                 b = __builtin_amdgcn_readfirstlane(b);
                 if (b >= n)
                     break;
-                t2m_entries<Periodic, Vec, HasResp, TT, Debug>(acc, facc, tod, xp, plan_mt, qmask, nsamp, ch.begin + b,
+                t2m_entries<Periodic, Vec, HasResp, Whole, TT, Debug>(acc, facc, tod, xp, plan_mt, qmask, nsamp, ch.begin + b,
                                                                ch.begin + min(b + bs, n), sct, g, ybase, xbase, gn,
                                                                fin, scale, limit, mrun, tsum, nwide, chk, err,
                                                                s_list[wave], dbg, first);
@@ -1726,7 +1676,7 @@ __device__ inline Gains batch_gains(const BatchTod &td)
     return Gains{ td.resp, td.scale, td.resp_ndet, td.resp_div, td.scale_div };
 }
 
-template<bool Periodic, typename TT, int NT, bool HasResp = false>
+template<bool Periodic, typename TT, int NT, bool HasResp, bool Whole>
 __global__ void __launch_bounds__(NT, 4)
 batched_map2tod_kernel(const float *__restrict__ lmap, const BatchTod *__restrict__ tods,
                        const BatchSeg *__restrict__ segs, const BatchItem *__restrict__ items,
@@ -1758,7 +1708,7 @@ batched_map2tod_kernel(const float *__restrict__ lmap, const BatchTod *__restric
         const uint32_t we = uint32_t((uint64_t(it.nent) * (wave + 1)) / (NT / WAVE));
         batch_wave_segments(segs, it, wb, we, [&](const BatchSeg &sg, uint32_t b, uint32_t e) {
             const BatchTod td = tods[sg.tod];
-            m2t_entries<Periodic, true, HasResp, TT>(static_cast<TT *>(td.tod), td.xp, td.plan_mt, td.qmask, td.nsamp,
+            m2t_entries<Periodic, true, HasResp, Whole, TT>(static_cast<TT *>(td.tod), td.xp, td.plan_mt, td.qmask, td.nsamp,
                                                    b, e, tile, sct, g, ybase, xbase, ba.accum, batch_gains(td), chk,
                                                    err);
         });
@@ -1770,7 +1720,7 @@ batched_map2tod_kernel(const float *__restrict__ lmap, const BatchTod *__restric
     report_err(err | chk.bits(g), ba.err_word);
 }
 
-template<bool Periodic, typename TT, bool HasResp = false>
+template<bool Periodic, typename TT, bool HasResp, bool Whole>
 __global__ void __launch_bounds__(T2M_THREADS)
 batched_tod2map_kernel(float *__restrict__ lmap, const BatchTod *__restrict__ tods,
                        const BatchSeg *__restrict__ segs, const BatchItem *__restrict__ items,
@@ -1779,7 +1729,7 @@ batched_tod2map_kernel(float *__restrict__ lmap, const BatchTod *__restrict__ to
     __shared__ __align__(16) unsigned long long acc[3 * HPLANE];       // 116 KiB
     __shared__ float2 sct[SCT];
     __shared__ uint32_t s_words[T2M_WORDS], s_item;
-    __shared__ uint16_t s_list[T2M_THREADS / WAVE][T2M_LIST];            // 16 KiB
+    __shared__ uint32_t s_list[T2M_THREADS / WAVE][T2M_LIST];            // 32 KiB
     float *facc = reinterpret_cast<float *>(acc);
 
     fill_sincos_table(sct, T2M_THREADS);
@@ -1811,7 +1761,7 @@ batched_tod2map_kernel(float *__restrict__ lmap, const BatchTod *__restrict__ to
             batch_wave_segments(segs, it, wb, we, [&](const BatchSeg &sg, uint32_t b, uint32_t e) {
                 if (first) {
                     const BatchTod td = tods[sg.tod];
-                    m = t2m_probe<true, HasResp, TT>(static_cast<const TT *>(td.tod), td.plan_mt, td.nsamp, b, e,
+                    m = t2m_probe<true, HasResp, Whole, TT>(static_cast<const TT *>(td.tod), td.plan_mt, td.nsamp, b, e,
                                                    batch_gains(td), act);
                     first = false;
                 }
@@ -1843,7 +1793,7 @@ batched_tod2map_kernel(float *__restrict__ lmap, const BatchTod *__restrict__ to
                     batch_wave_segments(segs, it, b0, min(b0 + bs, it.nent),
                                         [&](const BatchSeg &sg, uint32_t b, uint32_t e) {
                         const BatchTod td = tods[sg.tod];
-                        t2m_entries<Periodic, true, HasResp, TT>(acc, facc, static_cast<const TT *>(td.tod), td.xp,
+                        t2m_entries<Periodic, true, HasResp, Whole, TT>(acc, facc, static_cast<const TT *>(td.tod), td.xp,
                                                                td.plan_mt, td.qmask, td.nsamp, b, e, sct, g, ybase,
                                                                xbase, batch_gains(td), fin, scale, limit, mrun, tsum,
                                                                nwide, chk, err, s_list[wave]);
@@ -1861,6 +1811,12 @@ batched_tod2map_kernel(float *__restrict__ lmap, const BatchTod *__restrict__ to
     report_err(err, ba.err_word);
 }
 
+// Every gain array has rows of a multiple of 4 samples.
+bool whole_rows(const Gains &gn)
+{
+    return (!gn.resp || gn.resp_div.nper % 4 == 0) && (!gn.scale || gn.scale_div.nper % 4 == 0);
+}
+
 template<bool HasResp, typename TT>
 void launch_m2t(TT *tod, const float *lmap, const float *xp, const OpArgs &a, const gmm_plan &plan,
                 bool accum, const Gains &gn, hipStream_t stream)
@@ -1869,15 +1825,23 @@ void launch_m2t(TT *tod, const float *lmap, const float *xp, const OpArgs &a, co
     uint32_t *err_word = plan.err + (plan.pp.n_err - 1);
     dim3 grid(unsigned(plan.nchunks)), block(M2T_THREADS);
     const bool vec = (((reinterpret_cast<uintptr_t>(tod) | reinterpret_cast<uintptr_t>(xp)) & 15) == 0) && (a.nsamp % 4 == 0);
-    auto k = lp.periodic_xcoord ? (vec ? planned_map2tod_kernel<true, true, HasResp, TT> : planned_map2tod_kernel<true, false, HasResp, TT>)
-                                : (vec ? planned_map2tod_kernel<false, true, HasResp, TT> : planned_map2tod_kernel<false, false, HasResp, TT>);
+    auto pick = [&](auto whole) {
+        constexpr bool W = decltype(whole)::value;
+        return lp.periodic_xcoord ? (vec ? planned_map2tod_kernel<true, true, HasResp, W, TT> : planned_map2tod_kernel<true, false, HasResp, W, TT>)
+                                  : (vec ? planned_map2tod_kernel<false, true, HasResp, W, TT> : planned_map2tod_kernel<false, false, HasResp, W, TT>);
+    };
+    auto k = pick(std::true_type{});
+    if constexpr (HasResp || !std::is_same<TT, float>::value) {
+        if (!whole_rows(gn))
+            k = pick(std::false_type{});
+    }
     Dbg dbg{ nullptr, nullptr, nullptr };
     if constexpr (std::is_same<TT, float>::value) {
         // debug=True: the instrumented instantiation (float32 TODs).
         if (a.debug) {
             dbg = Dbg{ a.debug->entry_visits, a.debug->sample_evals, a.debug->tile_bad };
-            k = lp.periodic_xcoord ? (vec ? planned_map2tod_kernel<true, true, HasResp, TT, true> : planned_map2tod_kernel<true, false, HasResp, TT, true>)
-                                   : (vec ? planned_map2tod_kernel<false, true, HasResp, TT, true> : planned_map2tod_kernel<false, false, HasResp, TT, true>);
+            k = lp.periodic_xcoord ? (vec ? planned_map2tod_kernel<true, true, HasResp, false, TT, true> : planned_map2tod_kernel<true, false, HasResp, false, TT, true>)
+                                   : (vec ? planned_map2tod_kernel<false, true, HasResp, false, TT, true> : planned_map2tod_kernel<false, false, HasResp, false, TT, true>);
         }
     }
     kernel_timer_mark(TK_MAP2TOD, false, stream);
@@ -1896,14 +1860,22 @@ void launch_t2m(float *lmap, const TT *tod, const float *xp, const OpArgs &a, co
     uint32_t *err_word = plan.err + (plan.pp.n_err - 1);
     dim3 grid(unsigned(plan.nchunks_t2m)), block(T2M_THREADS);
     const bool vec = (((reinterpret_cast<uintptr_t>(tod) | reinterpret_cast<uintptr_t>(xp)) & 15) == 0) && (a.nsamp % 4 == 0);
-    auto k = lp.periodic_xcoord ? (vec ? planned_tod2map_kernel<true, true, HasResp, TT> : planned_tod2map_kernel<true, false, HasResp, TT>)
-                                : (vec ? planned_tod2map_kernel<false, true, HasResp, TT> : planned_tod2map_kernel<false, false, HasResp, TT>);
+    auto pick = [&](auto whole) {
+        constexpr bool W = decltype(whole)::value;
+        return lp.periodic_xcoord ? (vec ? planned_tod2map_kernel<true, true, HasResp, W, TT> : planned_tod2map_kernel<true, false, HasResp, W, TT>)
+                                  : (vec ? planned_tod2map_kernel<false, true, HasResp, W, TT> : planned_tod2map_kernel<false, false, HasResp, W, TT>);
+    };
+    auto k = pick(std::true_type{});
+    if constexpr (HasResp || !std::is_same<TT, float>::value) {
+        if (!whole_rows(gn))
+            k = pick(std::false_type{});
+    }
     Dbg dbg{ nullptr, nullptr, nullptr };
     if constexpr (std::is_same<TT, float>::value) {
         if (a.debug) {
             dbg = Dbg{ a.debug->entry_visits, a.debug->sample_evals, a.debug->tile_bad };
-            k = lp.periodic_xcoord ? (vec ? planned_tod2map_kernel<true, true, HasResp, TT, true> : planned_tod2map_kernel<true, false, HasResp, TT, true>)
-                                   : (vec ? planned_tod2map_kernel<false, true, HasResp, TT, true> : planned_tod2map_kernel<false, false, HasResp, TT, true>);
+            k = lp.periodic_xcoord ? (vec ? planned_tod2map_kernel<true, true, HasResp, false, TT, true> : planned_tod2map_kernel<true, false, HasResp, false, TT, true>)
+                                   : (vec ? planned_tod2map_kernel<false, true, HasResp, false, TT, true> : planned_tod2map_kernel<false, false, HasResp, false, TT, true>);
         }
     }
     kernel_timer_mark(TK_TOD2MAP, false, stream);
@@ -1975,53 +1947,52 @@ unsigned batch_grid(const BatchLaunch &bl)
     return unsigned((bl.grid > 0) ? std::min<int64_t>(bl.grid, bl.nitems) : bl.nitems);
 }
 
-template<typename TT>
+template<typename TT, bool HasResp, bool Whole>
+void batched_m2t_launch(const BatchLaunch &bl, const float *lmap, const int64_t *cell_offsets, const BatchArgs &ba,
+                        bool periodic, hipStream_t stream)
+{
+    const unsigned grid = batch_grid(bl);
+    if (bl.threads == 256) {
+        auto k = periodic ? batched_map2tod_kernel<true, TT, 256, HasResp, Whole> : batched_map2tod_kernel<false, TT, 256, HasResp, Whole>;
+        k<<<grid, 256, 0, stream>>>(lmap, bl.tods, bl.segs, bl.items, cell_offsets, ba);
+    }
+    else {
+        auto k = periodic ? batched_map2tod_kernel<true, TT, 512, HasResp, Whole> : batched_map2tod_kernel<false, TT, 512, HasResp, Whole>;
+        k<<<grid, 512, 0, stream>>>(lmap, bl.tods, bl.segs, bl.items, cell_offsets, ba);
+    }
+    GMM_HIP(hipGetLastError());
+}
+
+template<typename TT, bool HasResp, bool Whole>
+void batched_t2m_launch(const BatchLaunch &bl, float *lmap, const int64_t *cell_offsets, const BatchArgs &ba,
+                        bool periodic, hipStream_t stream)
+{
+    auto k = periodic ? batched_tod2map_kernel<true, TT, HasResp, Whole> : batched_tod2map_kernel<false, TT, HasResp, Whole>;
+    k<<<batch_grid(bl), T2M_THREADS, 0, stream>>>(lmap, bl.tods, bl.segs, bl.items, cell_offsets, ba);
+    GMM_HIP(hipGetLastError());
+}
+
+// Gains of any kind come with rows of whole groups (in every TOD) or of any length.
+template<typename TT, bool HasResp>
 void batched_m2t_typed(const BatchLaunch &bl, const float *lmap, const int64_t *cell_offsets, const BatchArgs &ba,
                        bool periodic, hipStream_t stream)
 {
-    const unsigned grid = batch_grid(bl);
-    if (bl.threads == 256) {
-        auto k = periodic ? batched_map2tod_kernel<true, TT, 256> : batched_map2tod_kernel<false, TT, 256>;
-        k<<<grid, 256, 0, stream>>>(lmap, bl.tods, bl.segs, bl.items, cell_offsets, ba);
+    if constexpr (HasResp || !std::is_same<TT, float>::value) {
+        if (!bl.whole_rows)
+            return batched_m2t_launch<TT, HasResp, false>(bl, lmap, cell_offsets, ba, periodic, stream);
     }
-    else {
-        auto k = periodic ? batched_map2tod_kernel<true, TT, 512> : batched_map2tod_kernel<false, TT, 512>;
-        k<<<grid, 512, 0, stream>>>(lmap, bl.tods, bl.segs, bl.items, cell_offsets, ba);
-    }
-    GMM_HIP(hipGetLastError());
+    batched_m2t_launch<TT, HasResp, true>(bl, lmap, cell_offsets, ba, periodic, stream);
 }
 
-template<typename TT>
+template<typename TT, bool HasResp>
 void batched_t2m_typed(const BatchLaunch &bl, float *lmap, const int64_t *cell_offsets, const BatchArgs &ba,
                        bool periodic, hipStream_t stream)
 {
-    auto k = periodic ? batched_tod2map_kernel<true, TT> : batched_tod2map_kernel<false, TT>;
-    k<<<batch_grid(bl), T2M_THREADS, 0, stream>>>(lmap, bl.tods, bl.segs, bl.items, cell_offsets, ba);
-    GMM_HIP(hipGetLastError());
-}
-
-// Batched operators with per-detector gains (float32 TODs).
-void batched_m2t_resp(const BatchLaunch &bl, const float *lmap, const int64_t *cell_offsets, const BatchArgs &ba,
-                      bool periodic, hipStream_t stream)
-{
-    const unsigned grid = batch_grid(bl);
-    if (bl.threads == 256) {
-        auto k = periodic ? batched_map2tod_kernel<true, float, 256, true> : batched_map2tod_kernel<false, float, 256, true>;
-        k<<<grid, 256, 0, stream>>>(lmap, bl.tods, bl.segs, bl.items, cell_offsets, ba);
+    if constexpr (HasResp || !std::is_same<TT, float>::value) {
+        if (!bl.whole_rows)
+            return batched_t2m_launch<TT, HasResp, false>(bl, lmap, cell_offsets, ba, periodic, stream);
     }
-    else {
-        auto k = periodic ? batched_map2tod_kernel<true, float, 512, true> : batched_map2tod_kernel<false, float, 512, true>;
-        k<<<grid, 512, 0, stream>>>(lmap, bl.tods, bl.segs, bl.items, cell_offsets, ba);
-    }
-    GMM_HIP(hipGetLastError());
-}
-
-void batched_t2m_resp(const BatchLaunch &bl, float *lmap, const int64_t *cell_offsets, const BatchArgs &ba,
-                      bool periodic, hipStream_t stream)
-{
-    auto k = periodic ? batched_tod2map_kernel<true, float, true> : batched_tod2map_kernel<false, float, true>;
-    k<<<batch_grid(bl), T2M_THREADS, 0, stream>>>(lmap, bl.tods, bl.segs, bl.items, cell_offsets, ba);
-    GMM_HIP(hipGetLastError());
+    batched_t2m_launch<TT, HasResp, true>(bl, lmap, cell_offsets, ba, periodic, stream);
 }
 
 }  // namespace
@@ -2061,12 +2032,12 @@ void launch_batched_map2tod(const BatchLaunch &bl, const float *lmap, const gmm_
     switch (tod_type) {
     case TOD_F32:
         if (bl.has_resp)
-            batched_m2t_resp(bl, lmap, lp.offsets_gpu, ba, lp.periodic_xcoord, stream);
+            batched_m2t_typed<float, true>(bl, lmap, lp.offsets_gpu, ba, lp.periodic_xcoord, stream);
         else
-            batched_m2t_typed<float>(bl, lmap, lp.offsets_gpu, ba, lp.periodic_xcoord, stream);
+            batched_m2t_typed<float, false>(bl, lmap, lp.offsets_gpu, ba, lp.periodic_xcoord, stream);
         break;
-    case TOD_F16: batched_m2t_typed<_Float16>(bl, lmap, lp.offsets_gpu, ba, lp.periodic_xcoord, stream); break;
-    case TOD_BF16: batched_m2t_typed<__bf16>(bl, lmap, lp.offsets_gpu, ba, lp.periodic_xcoord, stream); break;
+    case TOD_F16: batched_m2t_typed<_Float16, false>(bl, lmap, lp.offsets_gpu, ba, lp.periodic_xcoord, stream); break;
+    case TOD_BF16: batched_m2t_typed<__bf16, false>(bl, lmap, lp.offsets_gpu, ba, lp.periodic_xcoord, stream); break;
     default: fail("batched map2tod: unknown TOD element type");
     }
 }
@@ -2081,12 +2052,12 @@ void launch_batched_tod2map(const BatchLaunch &bl, float *lmap, const gmm_lpix &
     switch (tod_type) {
     case TOD_F32:
         if (bl.has_resp)
-            batched_t2m_resp(bl, lmap, lp.offsets_gpu, ba, lp.periodic_xcoord, stream);
+            batched_t2m_typed<float, true>(bl, lmap, lp.offsets_gpu, ba, lp.periodic_xcoord, stream);
         else
-            batched_t2m_typed<float>(bl, lmap, lp.offsets_gpu, ba, lp.periodic_xcoord, stream);
+            batched_t2m_typed<float, false>(bl, lmap, lp.offsets_gpu, ba, lp.periodic_xcoord, stream);
         break;
-    case TOD_F16: batched_t2m_typed<_Float16>(bl, lmap, lp.offsets_gpu, ba, lp.periodic_xcoord, stream); break;
-    case TOD_BF16: batched_t2m_typed<__bf16>(bl, lmap, lp.offsets_gpu, ba, lp.periodic_xcoord, stream); break;
+    case TOD_F16: batched_t2m_typed<_Float16, false>(bl, lmap, lp.offsets_gpu, ba, lp.periodic_xcoord, stream); break;
+    case TOD_BF16: batched_t2m_typed<__bf16, false>(bl, lmap, lp.offsets_gpu, ba, lp.periodic_xcoord, stream); break;
     default: fail("batched tod2map: unknown TOD element type");
     }
 }
