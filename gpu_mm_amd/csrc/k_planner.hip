@@ -1324,7 +1324,7 @@ SortLayout sort_layout(int64_t nmt)
     return L;
 }
 
-constexpr int64_t CAP_MIN = 128, CAP_MAX = 8192;         // entries per work unit
+constexpr int64_t CAP_MAX = 8192;                        // entries per work unit
 
 // Lists of up to this many chunks are ordered by rank (n^2 comparisons: 16384 take about 40 us).
 constexpr int64_t RANK_MAX = 16384;
@@ -1341,15 +1341,16 @@ WorkListOut t2m_out(const gmm_preplan &pp, const PlanLists &l, uint32_t *counts)
 
 // Sizes for a plan of nmt entries on 'slots' blocks that run at once: lists of at most k * slots chunks (k
 // full rounds) with chunks up to 5, 15, 30 and 50% above an even share, ordered by the time that the
-// rounds take when a block costs as much as 'fixed' entries; and last 'general', which any list may take.
-ChunkCaps make_caps(int64_t nmt, int64_t slots, int64_t fixed, int kmax, int64_t general)
+// rounds take when a block costs as much as 'fixed' entries; no chunk is smaller than 'least' for the sake
+// of a round. Last comes 'general', which any list may take.
+ChunkCaps make_caps(int64_t nmt, int64_t slots, int64_t fixed, int kmax, int64_t least, int64_t general)
 {
     struct Option { int64_t cap, limit, cost; };
     std::vector<Option> opt;
     for (int k = 1; k <= kmax; k++)
         for (int percent : {105, 115, 130, 150}) {
             const int64_t share = k * slots * 100;
-            const int64_t cap = std::max<int64_t>(CAP_MIN, (nmt * percent + share - 1) / share);
+            const int64_t cap = std::max<int64_t>(least, (nmt * percent + share - 1) / share);
             if (cap <= CAP_MAX && int(opt.size()) < NCAPS - 1)
                 opt.push_back(Option{cap, k * slots, k * (fixed + cap)});
         }
@@ -1402,7 +1403,8 @@ void launch_rank(const PlanLists &l, const uint32_t *counts, int64_t max_m2t, in
 // fast one of 768 x 50004 311 / 275; with one round as the only choice the last two gain nothing; rasters
 // over more cells than that the same). map2tod, two blocks a CU and bound by memory, balances best in many
 // small chunks (263 us on the 768 x 50004; 285 with tod2map's), except when they would not fill a round
-// (64 x 65536 samples 25.8 us in chunks of 512, 22.7 in one round; 8 x 4096 10.9 and 9.5).
+// (64 x 65536 samples 25.8 us in chunks of 512, 22.7 in one round; 8 x 4096 10.9 and 9.5). Each chunk of a
+// split cell adds to the map with a rounding of its own, so that tod2map's stay at 512 entries or more.
 constexpr int64_t TILE_COST = 700, STAGE_COST = 100;     // a block's fixed work, in entries
 
 void plan_chunk_caps(gmm_preplan &pp)
@@ -1410,8 +1412,8 @@ void plan_chunk_caps(gmm_preplan &pp)
     const int64_t nmt = pp.plan_nmt, nkeys = pp.nycells_g * pp.nxcells_g, cus = 256;
     const int64_t m2t = std::min(CAP_MAX, std::max<int64_t>(512, (nmt + 12 * cus - 1) / (12 * cus)));
     const int64_t t2m = std::min(CAP_MAX, std::max<int64_t>(1024, (nmt + 2 * cus - 1) / (2 * cus)));
-    pp.caps_m2t = make_caps(nmt, 2 * cus, STAGE_COST, (nmt <= 512 * 2 * cus) ? 1 : 0, m2t);
-    pp.caps_t2m = make_caps(nmt, cus, TILE_COST, 3, t2m);
+    pp.caps_m2t = make_caps(nmt, 2 * cus, STAGE_COST, (nmt <= 512 * 2 * cus) ? 1 : 0, 128, m2t);
+    pp.caps_t2m = make_caps(nmt, cus, TILE_COST, 3, 512, t2m);
     pp.max_nchunks = max_chunks(pp.caps_m2t, nmt, nkeys);
     pp.max_nchunks_t2m = max_chunks(pp.caps_t2m, nmt, nkeys);
 }

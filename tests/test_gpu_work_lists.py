@@ -30,14 +30,14 @@ def make_pointing(kind, n, ny, nx):
 
 def sizes(nmt):
     """(cap, limit) options of map2tod's and of tod2map's list, in the order of preference."""
-    def options(slots, fixed, kmax, general):
-        opt = [(max(128, -(-nmt * m // (100 * k * slots))), k * slots) for k in range(1, kmax + 1)
+    def options(slots, fixed, kmax, least, general):
+        opt = [(max(least, -(-nmt * m // (100 * k * slots))), k * slots) for k in range(1, kmax + 1)
                for m in (105, 115, 130, 150)]
         opt = [o for o in opt if o[0] <= 8192][:11]
         opt.sort(key=lambda o: o[1] // slots * (fixed + o[0]))
         return opt + [(general, 1 << 32)]
-    return (options(512, 100, 1 if nmt <= 512 * 512 else 0, min(8192, max(512, -(-nmt // 3072)))),
-            options(256, 700, 3, min(8192, max(1024, -(-nmt // 512)))))
+    return (options(512, 100, 1 if nmt <= 512 * 512 else 0, 128, min(8192, max(512, -(-nmt // 3072)))),
+            options(256, 700, 3, 512, min(8192, max(1024, -(-nmt // 512)))))
 
 
 def bound(opt, nmt, nkeys):
