@@ -1175,6 +1175,10 @@ __device__ inline void t2m_entries(unsigned long long *__restrict__ acc, float *
             const int64_t s0 = int64_t(code & ICL_MASK) * LINE + 4 * ((code >> ITEM_QUAD_SHIFT) & 7u);
             // Past the end of the TOD (nv < 4) the samples read as zeros: they deposit nothing.
             const uint32_t nv = uint32_t(min<int64_t>(4, nsamp - s0));
+            // The gains before the samples (batched, 16-bit, 24 TODs: 12.59 -> 11.97 ms).
+            float tr[4], pr[4], sc[4];
+            quad_resp<HasResp, Whole>(gn, uint32_t(s0), tr, pr, nv);
+            quad_scale<TT, Whole>(gn, uint32_t(s0), sc);
             // Non-temporal: the pointing and TOD stream through once, while the cell's map lines
             // (touched at block start by t2m_warm_cell) should stay cached for the flush.
             const float4 y4 = Vec ? load4_nt(xp + s0) : load4n<Vec>(xp + s0, nv);
@@ -1185,9 +1189,6 @@ __device__ inline void t2m_entries(unsigned long long *__restrict__ acc, float *
                 t4 = Vec ? load4_nt(tod + s0) : IO::load_n(tod + s0, nv);
             else
                 t4 = IO::load_n(tod + s0, nv);
-            float tr[4], pr[4], sc[4];
-            quad_resp<HasResp, Whole>(gn, uint32_t(s0), tr, pr, nv);
-            quad_scale<TT, Whole>(gn, uint32_t(s0), sc);
             if (Q16) {
                 t4.x *= sc[0];
                 t4.y *= sc[1];
