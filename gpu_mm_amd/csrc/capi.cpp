@@ -595,7 +595,9 @@ int gmm_plan_create(gmm_plan **out, const gmm_preplan *pp, const float *xpointin
             plan->nmlines = h[PC_NMLINES];
             GMM_REQUIRE(plan->nchunks <= pp->max_nchunks && plan->nchunks_t2m <= pp->max_nchunks_t2m,
                         "PointingPlan constructor: work list larger than its bound (internal error)");
-            order_long_lists(*pp, lists, plan->nchunks, plan->nchunks_t2m, counts, a, b, scratch, stream);
+            // The plan may be used on any stream once this returns.
+            if (order_long_lists(*pp, lists, plan->nchunks, plan->nchunks_t2m, counts, a, b, scratch, stream))
+                GMM_HIP(hipStreamSynchronize(stream));
             if (debug)
                 check_plan_invariants(*plan, where, stream);
         }

@@ -1508,18 +1508,19 @@ void plan_masks(const gmm_preplan &pp, const uint64_t *sorted_mt, const float *x
     GMM_HIP(hipGetLastError());
 }
 
-void order_long_lists(const gmm_preplan &pp, const PlanLists &l, int64_t n_m2t, int64_t n_t2m, const uint32_t *counts_gpu,
+bool order_long_lists(const gmm_preplan &pp, const PlanLists &l, int64_t n_m2t, int64_t n_t2m, const uint32_t *counts_gpu,
                       uint64_t *a, uint64_t *b, void *scratch, hipStream_t stream)
 {
     if (pp.plan_nmt <= SP_MAX) {                                     // plan_small() did the short ones
-        launch_rank(l, counts_gpu, (n_m2t > SP_RANK) ? n_m2t : 0, (n_t2m > SP_RANK) ? n_t2m : 0, stream);
-        return;
+        const int64_t r_m2t = (n_m2t > SP_RANK) ? n_m2t : 0, r_t2m = (n_t2m > SP_RANK) ? n_t2m : 0;
+        launch_rank(l, counts_gpu, r_m2t, r_t2m, stream);
+        return r_m2t > 0 || r_t2m > 0;
     }
     if (l.max_m2t <= RANK_MAX && l.max_t2m <= RANK_MAX)
-        return;                                                      // plan_schedule() did it
+        return false;                                                // plan_schedule() did it
     if (n_m2t <= RANK_MAX && n_t2m <= RANK_MAX) {
         launch_rank(l, counts_gpu, n_m2t, n_t2m, stream);
-        return;
+        return true;
     }
     // a and b hold plan_nmt items each, a list at most as many. 13-bit keys: kx = 1024 makes the sort's
     // key the item's low 20 bits.
@@ -1549,6 +1550,7 @@ void order_long_lists(const gmm_preplan &pp, const PlanLists &l, int64_t n_m2t, 
     };
     order(l.tmp_m2t, l.m2t, n_m2t);
     order(l.tmp_t2m, l.t2m, n_t2m);
+    return true;
 }
 
 constexpr int64_t GENERIC_KEYS = int64_t(1) << 20;
