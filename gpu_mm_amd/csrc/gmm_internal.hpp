@@ -159,6 +159,7 @@ struct PlanLists
 {
     Chunk *m2t, *t2m;
     Chunk *tmp_m2t, *tmp_t2m;
+    uint32_t *block_counts;                // chunks made by the cells of each block, for each size of each list
     uint32_t *begin;                       // first entry of each cell of the global map
     int64_t max_m2t, max_t2m;
 };

@@ -674,7 +674,7 @@ __global__ void split_items_kernel(const uint64_t *__restrict__ in, uint64_t *__
 
 // ------------------------------------------------------------------------------------------
 // Work lists: per-cell [begin, end) in the sorted plan, cut into chunks of <= cap entries, one list per
-// operator. The chunks of a list come in no fixed order; rank_chunks_kernel puts them in theirs.
+// operator, in plan order; rank_chunks_kernel or a stable sort by size then puts them in theirs.
 
 __global__ void fill_u32_kernel(uint32_t *p, int64_t n, uint32_t v)
 {
@@ -714,14 +714,15 @@ __device__ inline void store_chunks(uint32_t icell, uint32_t b, uint32_t cnt, ui
     }
 }
 
-// One list as the kernels see it: the sizes to choose from, how many chunks each of them makes, and the
-// number of chunks of the list.
+// One list as the kernels see it: the sizes to choose from, how many chunks each of them makes (in all,
+// and [size][block of cell_runs_kernel]), and the number of chunks of the list.
 struct WorkListOut
 {
     Chunk *list;
     int64_t max_chunks;
     ChunkCaps caps;
     uint32_t *cap_counts;
+    uint32_t *block_counts;
     uint32_t *count;
 };
 
@@ -755,39 +756,59 @@ cell_runs_kernel(const uint64_t *__restrict__ mt, int64_t n, uint32_t kx, int64_
         }
     }
     __syncthreads();
-    if (threadIdx.x < 2 * NCAPS && s_counts[threadIdx.x])
-        atomicAdd((threadIdx.x < NCAPS) ? a.cap_counts + threadIdx.x : b.cap_counts + threadIdx.x - NCAPS,
-                  s_counts[threadIdx.x]);
+    if (threadIdx.x < 2 * NCAPS) {
+        const bool ina = threadIdx.x < NCAPS;
+        const uint32_t j = threadIdx.x % NCAPS, c = s_counts[threadIdx.x];
+        (ina ? a.block_counts : b.block_counts)[j * gridDim.x + blockIdx.x] = c;
+        if (c)
+            atomicAdd((ina ? a.cap_counts : b.cap_counts) + j, c);
+    }
 }
 
 __device__ inline uint32_t chosen_cap(const WorkListOut &l)
 {
     for (uint32_t j = 0; j + 1 < l.caps.n; j++)
         if (l.cap_counts[j] <= l.caps.limit[j])
-            return l.caps.cap[j];
-    return l.caps.cap[l.caps.n - 1];
+            return j;
+    return l.caps.n - 1;
 }
 
 __global__ void __launch_bounds__(WL_THREADS)
 work_list_kernel(const uint32_t *__restrict__ begin, uint32_t kx, int64_t nkeys, WorkListOut a, WorkListOut b)
 {
-    __shared__ uint32_t s_wave[WL_THREADS / WAVE], s_base[2];
+    // The grid is cell_runs_kernel's. Each block adds up the chunks of the blocks before it (at most 4096
+    // words a list), so that the lists come in plan order, the same in every run.
+    __shared__ uint32_t s_wave[WL_THREADS / WAVE], s_before[2][WL_THREADS / WAVE];
     const int64_t k = int64_t(blockIdx.x) * WL_THREADS + threadIdx.x;
     const uint32_t b0 = (k < nkeys) ? begin[k] : 0u, cnt = (k < nkeys) ? max(begin[k + 1], b0) - b0 : 0u;
-    const uint32_t cap_a = chosen_cap(a), cap_b = chosen_cap(b);
-    const uint32_t na = nchunks_for(cnt, cap_a), nb = nchunks_for(cnt, cap_b);
-    uint32_t ta, tb;
-    const uint32_t xa = block_exclusive_scan<WL_THREADS>(na, s_wave, ta);
-    const uint32_t xb = block_exclusive_scan<WL_THREADS>(nb, s_wave, tb);
-    if (threadIdx.x == 0) {
-        s_base[0] = ta ? atomicAdd(a.count, ta) : 0u;
-        s_base[1] = tb ? atomicAdd(b.count, tb) : 0u;
+    const uint32_t ja = chosen_cap(a), jb = chosen_cap(b), cap_a = a.caps.cap[ja], cap_b = b.caps.cap[jb];
+    uint32_t xa = 0, xb = 0;
+    for (uint32_t i = threadIdx.x; i < blockIdx.x; i += WL_THREADS) {
+        xa += a.block_counts[ja * gridDim.x + i];
+        xb += b.block_counts[jb * gridDim.x + i];
     }
-    __syncthreads();
+    xa = wave_reduce_add(xa);
+    xb = wave_reduce_add(xb);
+    if (lane_id() == 0) {
+        s_before[0][threadIdx.x / WAVE] = xa;
+        s_before[1][threadIdx.x / WAVE] = xb;
+    }
+    uint32_t ta, tb;
+    xa = block_exclusive_scan<WL_THREADS>(nchunks_for(cnt, cap_a), s_wave, ta);     // synchronizes
+    xb = block_exclusive_scan<WL_THREADS>(nchunks_for(cnt, cap_b), s_wave, tb);
+#pragma unroll
+    for (int w = 0; w < WL_THREADS / WAVE; w++) {
+        xa += s_before[0][w];
+        xb += s_before[1][w];
+    }
+    if (threadIdx.x == 0 && blockIdx.x == gridDim.x - 1) {
+        *a.count = xa + ta;
+        *b.count = xb + tb;
+    }
     if (cnt > 0) {
         const uint32_t icell = cell_key(int(k / kx), int(k % kx));
-        store_chunks(icell, b0, cnt, cap_a, s_base[0] + xa, a.list, a.max_chunks);
-        store_chunks(icell, b0, cnt, cap_b, s_base[1] + xb, b.list, b.max_chunks);
+        store_chunks(icell, b0, cnt, cap_a, xa, a.list, a.max_chunks);
+        store_chunks(icell, b0, cnt, cap_b, xb, b.list, b.max_chunks);
     }
 }
 
@@ -1329,14 +1350,19 @@ constexpr int64_t CAP_MAX = 8192;                        // entries per work uni
 // Lists of up to this many chunks are ordered by rank (n^2 comparisons: 16384 take about 40 us).
 constexpr int64_t RANK_MAX = 16384;
 
+// Blocks of the work list kernels, and the words that cell_runs_kernel leaves for each list.
+int64_t work_list_blocks(int64_t nkeys) { return nkeys / WL_THREADS + 1; }            // begin[nkeys] too
+int64_t block_count_words(int64_t nkeys) { return NCAPS * work_list_blocks(nkeys); }
+
 WorkListOut m2t_out(const gmm_preplan &pp, const PlanLists &l, uint32_t *counts)
 {
-    return WorkListOut{l.tmp_m2t, l.max_m2t, pp.caps_m2t, counts + PC_CAPS_M2T, counts + PC_CHUNKS_M2T};
+    return WorkListOut{l.tmp_m2t, l.max_m2t, pp.caps_m2t, counts + PC_CAPS_M2T, l.block_counts, counts + PC_CHUNKS_M2T};
 }
 
 WorkListOut t2m_out(const gmm_preplan &pp, const PlanLists &l, uint32_t *counts)
 {
-    return WorkListOut{l.tmp_t2m, l.max_t2m, pp.caps_t2m, counts + PC_CAPS_T2M, counts + PC_CHUNKS_T2M};
+    return WorkListOut{l.tmp_t2m, l.max_t2m, pp.caps_t2m, counts + PC_CAPS_T2M,
+                       l.block_counts + block_count_words(pp.nycells_g * pp.nxcells_g), counts + PC_CHUNKS_T2M};
 }
 
 // Sizes for a plan of nmt entries on 'slots' blocks that run at once: lists of at most k * slots chunks (k
@@ -1376,7 +1402,7 @@ int64_t max_chunks(const ChunkCaps &c, int64_t nmt, int64_t nkeys)
 void launch_work_lists(const uint64_t *mt, int64_t n, uint32_t kx, int64_t nkeys, uint32_t *begin, const WorkListOut &a,
                        const WorkListOut &b, hipStream_t stream)
 {
-    const unsigned grid = unsigned(nkeys / WL_THREADS + 1);             // begin[nkeys] too
+    const unsigned grid = unsigned(work_list_blocks(nkeys));
     cell_runs_kernel<<<grid, WL_THREADS, 0, stream>>>(mt, n, kx, nkeys, begin, a, b);
     GMM_HIP(hipGetLastError());
     work_list_kernel<<<grid, WL_THREADS, 0, stream>>>(begin, kx, nkeys, a, b);
@@ -1420,8 +1446,9 @@ void plan_chunk_caps(gmm_preplan &pp)
 
 int64_t plan_scratch_nbytes(const gmm_preplan &pp)
 {
+    const int64_t nkeys = pp.nycells_g * pp.nxcells_g;
     return sort_layout(pp.plan_nmt).total + align128(int64_t(sizeof(Chunk)) * (pp.max_nchunks + pp.max_nchunks_t2m))
-         + align128(4 * (pp.nycells_g * pp.nxcells_g + 1));
+         + align128(8 * block_count_words(nkeys)) + align128(4 * (nkeys + 1));
 }
 
 PlanLists plan_lists(const gmm_preplan &pp, Chunk *m2t, Chunk *t2m, void *scratch)
@@ -1433,8 +1460,10 @@ PlanLists plan_lists(const gmm_preplan &pp, Chunk *m2t, Chunk *t2m, void *scratc
     l.max_t2m = pp.max_nchunks_t2m;
     l.tmp_m2t = reinterpret_cast<Chunk *>(static_cast<uint8_t *>(scratch) + sort_layout(pp.plan_nmt).total);
     l.tmp_t2m = l.tmp_m2t + pp.max_nchunks;
-    l.begin = reinterpret_cast<uint32_t *>(static_cast<uint8_t *>(scratch) + plan_scratch_nbytes(pp)
-                                           - align128(4 * (pp.nycells_g * pp.nxcells_g + 1)));
+    const int64_t nkeys = pp.nycells_g * pp.nxcells_g;
+    uint8_t *begin = static_cast<uint8_t *>(scratch) + plan_scratch_nbytes(pp) - align128(4 * (nkeys + 1));
+    l.begin = reinterpret_cast<uint32_t *>(begin);
+    l.block_counts = reinterpret_cast<uint32_t *>(begin - align128(8 * block_count_words(nkeys)));
     return l;
 }
 
@@ -1555,21 +1584,26 @@ bool order_long_lists(const gmm_preplan &pp, const PlanLists &l, int64_t n_m2t, 
 
 constexpr int64_t GENERIC_KEYS = int64_t(1) << 20;
 
-int64_t build_chunks_generic_scratch_nbytes() { return align128(4 * (GENERIC_KEYS + 1)) + 128; }
+int64_t build_chunks_generic_scratch_nbytes()
+{
+    return align128(4 * (GENERIC_KEYS + 1)) + 128 + 8 * block_count_words(GENERIC_KEYS);
+}
 
 int64_t build_chunks_generic(const uint64_t *plan_mt_gpu, int64_t nmt, int64_t chunk_cap,
                              Chunk *chunks_gpu, int64_t max_chunks, void *scratch, hipStream_t stream)
 {
     uint32_t *begin = static_cast<uint32_t *>(scratch);
     uint32_t *counts = begin + align128(4 * (GENERIC_KEYS + 1)) / 4;
+    uint32_t *block_counts = counts + 128 / 4;
     fill_u32_kernel<<<1, 64, 0, stream>>>(counts, PC_TOTAL, 0u);
     GMM_HIP(hipGetLastError());
     ChunkCaps cap = {}, none = {};
     cap.n = none.n = 1;
     cap.cap[0] = uint32_t(chunk_cap);
     none.cap[0] = 1u << 30;
-    const WorkListOut a{chunks_gpu, max_chunks, cap, counts + PC_CAPS_M2T, counts + PC_CHUNKS_M2T};
-    const WorkListOut b{chunks_gpu, 0, none, counts + PC_CAPS_T2M, counts + PC_CHUNKS_T2M};
+    const WorkListOut a{chunks_gpu, max_chunks, cap, counts + PC_CAPS_M2T, block_counts, counts + PC_CHUNKS_M2T};
+    const WorkListOut b{chunks_gpu, 0, none, counts + PC_CAPS_T2M, block_counts + block_count_words(GENERIC_KEYS),
+                        counts + PC_CHUNKS_T2M};
     launch_work_lists(plan_mt_gpu, nmt, 1024u, GENERIC_KEYS, begin, a, b, stream);
     return int64_t(read_word(counts + PC_CHUNKS_M2T, stream));
 }

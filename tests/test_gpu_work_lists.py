@@ -79,3 +79,20 @@ def test_work_lists(gmm, dev, kind, n, ny, nx):
     for opt, nmax in zip(opts[::-1], bounds[::-1]):     # tod2map's list, before it map2tod's
         end -= align128(16 * nmax)
         check_list(buf[end:end + 16 * nmax].view(CHUNK), mt, opt, max(bounds) <= RANK_MAX)
+
+
+@pytest.mark.parametrize("kind,n,ny,nx", [("samples", 60000, 8960, 8960), ("lines", 32 * 25000, 12800, 12800),
+                                          ("samples", 20000, 65536, 65536)])
+def test_long_list_ties(gmm, dev, kind, n, ny, nx):
+    """Lists that the radix sort orders: equal chunks in plan order, so that a plan has one list."""
+    xg = torch.from_numpy(make_pointing(kind, n, ny, nx)).to(dev)
+    pre = gmm.PointingPrePlan(xg, ny, nx, periodic_xcoord=False)
+    plan = gmm.PointingPlan(pre, xg)
+    nmt, mt = pre.plan_nmt, plan.get_plan_mt()
+    buf = plan.buf.cpu().numpy()
+    end = pre.plan_nbytes - align128(2 * nmt)
+    for opt in sizes(nmt)[::-1]:
+        nmax = bound(opt, nmt, -(-ny // 64) * -(-nx // 64))
+        end -= align128(16 * nmax)
+        check_list(buf[end:end + 16 * nmax].view(CHUNK), mt, opt, True)
+    assert plan.nchunks > RANK_MAX
