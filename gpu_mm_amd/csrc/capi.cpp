@@ -145,15 +145,22 @@ void init_npix(gmm_lpix &lp, const char *where)
         fail(std::string(where) + ": something is wrong with the cell_offsets -- the cells do not fit together contiguously");
 }
 
+uint32_t *plan_error_word(const gmm_plan &plan) { return plan.err + (plan.pp.n_err - 1); }
+
+// Raises the errors 'e' that 'word' held, and clears it.
+void raise_errors(uint32_t e, uint32_t *word, const char *where, hipStream_t stream)
+{
+    if (e) {
+        clear_word(word, stream);
+        throw_errflags(e, where);
+    }
+}
+
 // Synchronous check of the plan's accumulated error word; clears it when set.
 void check_plan_errors(const gmm_plan &plan, const char *where, hipStream_t stream)
 {
-    uint32_t *w = plan.err + (plan.pp.n_err - 1);
-    uint32_t e = read_word(w, stream);
-    if (e) {
-        clear_word(w, stream);
-        throw_errflags(e, where);
-    }
+    uint32_t *w = plan_error_word(plan);
+    raise_errors(read_word(w, stream), w, where, stream);
 }
 
 void check_op_common(const gmm_lpix *lpix, const gmm_plan *plan, int64_t tod_nsamp,
@@ -644,7 +651,8 @@ int gmm_plan_check_errflags(const gmm_plan *plan, const char *where)
 {
     return guarded([&] {
         require_ptr(plan, "check_errflags", "plan");
-        check_plan_errors(*plan, where ? where : "PointingPlan", nullptr);
+        uint32_t *w = plan_error_word(*plan);
+        raise_errors(read_word_of_any_device(w), w, where ? where : "PointingPlan", nullptr);
     });
 }
 

@@ -212,13 +212,17 @@ void run_op(gmm_batch &b, int op, float *lmap, bool partial, bool accum, hipStre
         launch_batched_tod2map(launch_of(b, b.t2m, op), lmap, *b.lpix, b.tod_type, partial, stream);
 }
 
-void check_batch_errors(gmm_batch &b, const char *where, hipStream_t stream)
+void raise_batch_errors(gmm_batch &b, uint32_t e, const char *where, hipStream_t stream)
 {
-    const uint32_t e = read_word(b.words + 4, stream);
     if (e) {
         clear_word(b.words + 4, stream);
         throw_errflags(e, where);
     }
+}
+
+void check_batch_errors(gmm_batch &b, const char *where, hipStream_t stream)
+{
+    raise_batch_errors(b, read_word(b.words + 4, stream), where, stream);
 }
 
 // Median time of 'reps' launches of one operator (after one untimed launch), in ms. The launches
@@ -475,7 +479,7 @@ int gmm_batch_check_errflags(gmm_batch *b, const char *where)
 {
     return guarded([&] {
         require_ptr(b, "batch check_errflags", "batch");
-        check_batch_errors(*b, where ? where : "batch", nullptr);
+        raise_batch_errors(*b, read_word_of_any_device(b->words + 4), where ? where : "batch", nullptr);
     });
 }
 

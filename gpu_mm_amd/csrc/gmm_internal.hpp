@@ -95,12 +95,16 @@ int guarded(F &&f)
 
 inline hipStream_t as_stream(void *s) { return reinterpret_cast<hipStream_t>(s); }
 void require_ptr(const void *p, const char *where, const char *name);
-// Synchronous read / clear of one device word on 'stream'.
 // Device words as they are after the work enqueued on 'stream' so far, for which they wait: one, n (a few,
-// below 16), or the OR of n.
+// below 16), or the OR of n. The words are read by a kernel of the current device, on the stream of a call
+// that has launched others there.
 uint32_t read_word(const uint32_t *p, hipStream_t stream);
 void read_words(uint32_t *out, const uint32_t *src, int n, hipStream_t stream);
 uint32_t read_word_or(const uint32_t *p, int64_t n, hipStream_t stream);
+// For calls that launch nothing: a word that may be of another device than the current one, on the null
+// stream of the current one.
+uint32_t read_word_of_any_device(const uint32_t *p);
+// Clears one device word and waits for it.
 void clear_word(uint32_t *p, hipStream_t stream);
 
 // Converts a set of error bits into the exception the reference raises

@@ -161,6 +161,19 @@ uint32_t read_word(const uint32_t *p, hipStream_t stream)
     return h;
 }
 
+uint32_t read_word_of_any_device(const uint32_t *p)
+{
+    // A kernel of the current device may not be able to read another device's memory; a copy can.
+    int dev = 0;
+    hipPointerAttribute_t attr = {};
+    if (hipGetDevice(&dev) == hipSuccess && hipPointerGetAttributes(&attr, p) == hipSuccess && attr.device == dev)
+        return read_word(p, nullptr);
+    (void)hipGetLastError();
+    uint32_t h = 0;
+    copy_words(&h, p, 1, false, nullptr);
+    return h;
+}
+
 uint32_t read_word_or(const uint32_t *p, int64_t n, hipStream_t stream)
 {
     uint32_t h = 0;
