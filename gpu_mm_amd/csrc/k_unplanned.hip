@@ -166,8 +166,9 @@ struct Window
     int slope;             // 65536 * minor pixels per major pixel, at most 3 * 65536 in magnitude
 
     __device__ int place(int major) const { return major - major0 + WIN_LEAD; }
-    // First minor pixel held at place j.
-    __device__ int line(int j) const { return minor0 + ((slope * (j - WIN_LEAD)) >> 16); }
+    // First minor pixel held at place j. (Far outside the window, on maps of more than 10922 pixels, the
+    // product wraps, and the place is refused for its j.)
+    __device__ int line(int j) const { return minor0 + (int(uint32_t(slope) * uint32_t(j - WIN_LEAD)) >> 16); }
 
     // Element of a pixel, or -1.
     __device__ int find(int iy, int ix) const

@@ -112,3 +112,32 @@ def test_planfree_tod2map_nonfinite(gmm, dev, bad):
     hit[:, iy:iy + 2, ix:ix + 2] = True
     assert np.all(np.isfinite(got[~hit]))
     assert not np.any(np.isfinite(got[hit]))
+
+
+@pytest.mark.parametrize("kind", ["corners", "scattered", "jumps"])
+@pytest.mark.parametrize("periodic", [False, True])
+def test_planfree_tod2map_large_map(gmm, orc, dev, kind, periodic):
+    # Positions up to the largest map (16 bits a coordinate), and samples of one block that lie tens of
+    # thousands of pixels apart, in a map of a few cells.
+    ny = nx = 65536
+    n = 5000
+    rng = np.random.default_rng(n)
+    cells = [(0, 0), (0, 1023), (1023, 0), (1023, 1023), (511, 512), (512, 511)]
+    k = {"corners": np.arange(n) // 1024, "scattered": rng.integers(0, 6, n), "jumps": np.arange(n) // 300}[kind] % 6
+    c = np.array(cells)[k]
+    t = np.arange(n)
+    step = rng.uniform(0, 62, (2, n)) if kind == "scattered" else np.stack([0.02 * t % 60, 0.2 * t % 60])
+    xp = np.stack([64 * c[:, 0] + step[0] + 0.5, 64 * c[:, 1] + step[1] + 0.5, 0.001 * t]).astype(F32)
+    xp[0] = np.minimum(xp[0], ny - 2)
+    xp[1] = np.minimum(xp[1], nx - 2.5)
+    tod = rng.standard_normal(n).astype(F32)
+    lp = gmm.LocalPixelization.make_cells(ny, nx, cells, periodic_xcoord=periodic)
+    pix = orc.Pix(ny, nx, lp.cell_offsets_cpu, 64, 4096, periodic)
+    ref, err = orc.tod2map(tod.astype(np.float64), xp, pix, f64=True)
+    assert err == 0
+    got = run(gmm, dev, lp, xp, tod).astype(np.float64)
+    mag, _ = orc.tod2map(np.abs(tod).astype(np.float64), np.stack([xp[0], xp[1], 0 * xp[2]]), pix, f64=True)
+    mag = np.repeat(mag.reshape(len(cells), 3, 4096)[:, :1], 3, axis=1).reshape(-1)
+    # The bound of the smaller maps: roundings of the weights (exact differences of coordinates here too).
+    assert np.all(np.abs(got - ref) <= 2e-6 * mag + 1e-6 * np.abs(tod).max())
+    assert np.sum(np.abs(got - ref)) <= 1e-5 * np.sum(np.abs(ref))
