@@ -26,14 +26,21 @@ struct LocalMapView
     int nycells, nxcells;
     int64_t ystride, polstride;
 
-    // Offset of the T value of pixel (iy, ix), or -1 if its cell is not in the local map.
-    __device__ inline int64_t offset(int iy, int ix) const
+    // Offset of the cell of pixel (iy, ix), negative if it is not in the local map; of the pixel in it.
+    __device__ inline int64_t cell(int iy, int ix) const
     {
         const int cy = iy >> 6, cx = ix >> 6;
         if (unsigned(cy) >= unsigned(nycells) || unsigned(cx) >= unsigned(nxcells))
             return -1;
-        const int64_t o = cell_offsets[int64_t(cy) * nxcells + cx];
-        return (o < 0) ? int64_t(-1) : (o + int64_t(iy & 63) * ystride + (ix & 63));
+        return cell_offsets[int64_t(cy) * nxcells + cx];
+    }
+    __device__ inline int64_t inside(int iy, int ix) const { return int64_t(iy & 63) * ystride + (ix & 63); }
+
+    // Offset of the T value of pixel (iy, ix), or -1 if its cell is not in the local map.
+    __device__ inline int64_t offset(int iy, int ix) const
+    {
+        const int64_t o = cell(iy, ix);
+        return (o < 0) ? int64_t(-1) : o + inside(iy, ix);
     }
 };
 
@@ -142,14 +149,22 @@ unplanned_map2tod_kernel(float *__restrict__ tod, const float *__restrict__ lmap
 // before they go to the map (34 us; VALU issue is 25 of them), in a window along the straight line that
 // the samples follow: at each place j of the window's major axis it holds the few pixels around the
 // line, so that a scan in any direction fits (45 degrees: 69 us, the map rows it crosses are that many
-// more atomic requests; 0.73 pixel per sample: 105 us). What falls outside (scattered pointing) goes to
-// the map sample by sample.
+// more atomic requests; 0.73 pixel per sample: 105 us). What falls outside goes to the map: samples that
+// lie together summed in registers first (16 samples a detector at 0.1 pixel per sample 2370 -> 505 us of
+// the call), others with consecutive samples in consecutive lanes, as without windows (with a lane's four
+// one after the other, and their blocks' waves in turn, 3 pixels per sample along x took 1590 us, 667
+// without windows, 600 now; random pointing 2460 us).
 // The sums are float64: ds_add_f64 takes 9 clocks a wave, ds_add_f32 194 (measured). An element that
 // was never added to holds -0.0 in its T plane, which no sum of values other than -0.0 gives.
 
 constexpr int WIN_THREADS = 256, WIN_WAVES = WIN_THREADS / 64;
 constexpr int WIN_SAMPLES = 4 * WIN_THREADS;
 constexpr int WIN_N = 1024;                // pixels of the window (24 KiB of sums: 6 blocks per CU)
+// Least number of a wave's 256 samples that are worth a round of their own (from a few detectors' turns to
+// 5 pixels per sample 16, 32 and 64 are the same; 128 takes 2400 us for 4.2e6 samples at 1 pixel per
+// sample along y, 32 takes 1610), and of blocks: a small call waits for its rounds (1000 samples 54 us, 49
+// straight to the map).
+constexpr int WIN_SHARE = 32, WIN_SHARE_BLOCKS = 64;
 constexpr int WIN_LEAD = 4;                // places before the least one seen (lanes show one of their 4 samples)
 typedef double WindowSums[3][WIN_N];
 
@@ -170,11 +185,15 @@ struct Window
     // product wraps, and the place is refused for its j.)
     __device__ int line(int j) const { return minor0 + (int(uint32_t(slope) * uint32_t(j - WIN_LEAD)) >> 16); }
 
-    // Element of a pixel, or -1.
-    __device__ int find(int iy, int ix) const
+    // Element of the footprint's first pixel (and, in 'next', of the one beside it along the major axis)
+    // if all of a footprint that starts at (iy0, ix0) is held, else -1.
+    __device__ int find(int iy0, int ix0, int &next) const
     {
-        const int j = place(xmajor ? ix : iy), k = (xmajor ? iy : ix) - line(j);
-        return (unsigned(j) < unsigned(length) && unsigned(k) < unsigned(width)) ? j * jstride + k * kstride : -1;
+        const int j = place(xmajor ? ix0 : iy0), minor = xmajor ? iy0 : ix0;
+        const int k0 = minor - line(j), k1 = minor - line(j + 1);
+        const bool in = j >= 0 && j + 1 < length && min(k0, k1) >= 0 && max(k0, k1) + 1 < width;
+        next = (j + 1) * jstride + k1 * kstride;
+        return in ? j * jstride + k0 * kstride : -1;
     }
 };
 
@@ -289,24 +308,103 @@ struct Place
     float dy, dx;
 };
 
-// The four corners of one sample: to the window or, outside it, to the map.
+// Element of a sample's footprint in the window, or -1. x0 = nx - 1 of periodic x has its second column at
+// x = 0, outside.
 template<bool Periodic>
-__device__ inline void deposit_sample(const Place &p, float t, float q, float u, const Window &win, WindowSums &acc,
-                                      float *__restrict__ lmap, const LocalMapView &mv, int nx, bool partial, uint32_t &err)
+__device__ inline int find_sample(const Place &p, const Window &win, int nx, int &next)
 {
+    const int e = win.find(p.iy0, p.ix0, next);
+    return (Periodic && p.ix0 + 1 >= nx) ? -1 : e;
+}
+
+// The four corners of one sample that the window holds.
+template<bool Periodic>
+__device__ inline void deposit_sample(const Place &p, float t, float q, float u, const Window &win, WindowSums &acc, int nx)
+{
+    int next;
+    const int e = find_sample<Periodic>(p, win, nx, next);
+    const float dj = win.xmajor ? p.dx : p.dy, dn = win.xmajor ? p.dy : p.dx;
 #pragma unroll 1
     for (int i = 0; i < 4; i++) {
-        const int iy = p.iy0 + (i >> 1);
-        int ix = p.ix0 + (i & 1);
-        if (Periodic)
-            ix = (ix < nx) ? ix : 0;
-        const float w = ((i & 2) ? p.dy : 1.0f - p.dy) * ((i & 1) ? p.dx : 1.0f - p.dx);
-        const int e = win.find(iy, ix);
-        if (e >= 0)
-            window_add(acc, e, w * t, w * q, w * u);
-        else {
-            const int64_t o = mv.offset(iy, ix);
+        const float w = ((i & 2) ? dj : 1.0f - dj) * ((i & 1) ? dn : 1.0f - dn);
+        window_add(acc, ((i & 2) ? next : e) + ((i & 1) ? win.kstride : 0), w * t, w * q, w * u);
+    }
+}
+
+// Samples that no window holds go straight to the map. Four of a lane whose footprints are within 3 x 3
+// pixels are summed in registers before ...
+template<bool Periodic>
+__device__ inline void deposit_near(const Place (&p)[4], const float (&t)[4], const float (&q)[4], const float (&u)[4],
+                                    float *__restrict__ lmap, const LocalMapView &mv, int nx, bool partial, uint32_t &err)
+{
+    const int iy = min(min(p[0].iy0, p[1].iy0), min(p[2].iy0, p[3].iy0));
+    const int ix = min(min(p[0].ix0, p[1].ix0), min(p[2].ix0, p[3].ix0));
+    // The pixels' cells are those of the first and the last row and column: four lookups at once.
+    const int ix2 = (Periodic && ix + 2 >= nx) ? ix + 2 - nx : ix + 2;
+    const int64_t o00 = mv.cell(iy, ix), o01 = mv.cell(iy, ix2), o10 = mv.cell(iy + 2, ix), o11 = mv.cell(iy + 2, ix2);
+#pragma unroll 1
+    for (int i = 0; i < 9; i++) {
+        const int y = iy + i / 3, x = ix + i % 3;
+        float a = 0.0f, b = 0.0f, c = 0.0f;
+        bool any = false;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int r = y - p[k].iy0, l = x - p[k].ix0;
+            if (unsigned(r) <= 1u && unsigned(l) <= 1u) {
+                const float w = (r ? p[k].dy : 1.0f - p[k].dy) * (l ? p[k].dx : 1.0f - p[k].dx);
+                a = fmaf(w, t[k], a);
+                b = fmaf(w, q[k], b);
+                c = fmaf(w, u[k], c);
+                any = true;
+            }
+        }
+        if (any) {
+            const int xw = (Periodic && x >= nx) ? x - nx : x;
+            const bool row = (y ^ iy) >> 6, col = (xw ^ ix) >> 6;
+            int64_t o = row ? (col ? o11 : o10) : (col ? o01 : o00);
             if (o >= 0) {
+                o += mv.inside(y, xw);
+                unsafeAtomicAdd(lmap + o, a);
+                unsafeAtomicAdd(lmap + o + mv.polstride, b);
+                unsafeAtomicAdd(lmap + o + 2 * mv.polstride, c);
+            }
+            else if (!partial)
+                err |= ERR_NOT_IN_PIXELIZATION;
+        }
+    }
+}
+
+// ... and others, those of a wave's 256 samples from s on that are not done (sample i: bit i / 4 of
+// 'done' in lanes i % 4, i % 4 + 4 ...), one per lane and consecutive lanes consecutive samples: their atomics share cache lines
+// where the scan runs along a map row.
+template<bool Periodic>
+__device__ inline void deposit_far(float *__restrict__ lmap, const float *__restrict__ tod, const float *__restrict__ xp,
+                                   int64_t nsamp, int64_t s, int64_t s1, uint64_t done, const Geom &g,
+                                   const LocalMapView &mv, bool partial, uint32_t &err)
+{
+    Checks checked;                            // with the tile's samples
+    const int lane = threadIdx.x & 63;
+#pragma unroll 1
+    for (int r = 0; r < 4; r++) {
+        const int64_t i = s + 64 * r + lane;
+        if (i >= s1 || ((done >> (16 * r + (lane >> 2))) & 1u))
+            continue;
+        const float y = xp[i], x = xp[nsamp + i], alpha = xp[2 * nsamp + i], t = tod[i];
+        Place p;
+        locate_op<Periodic>(y, x, g, checked, p.iy0, p.ix0, p.dy, p.dx);
+        // The corners' cells are looked up at once.
+        const int iy1 = p.iy0 + 1, ix1 = (Periodic && p.ix0 + 1 >= g.nx) ? 0 : p.ix0 + 1;
+        const int64_t o00 = mv.cell(p.iy0, p.ix0), o01 = mv.cell(p.iy0, ix1), o10 = mv.cell(iy1, p.ix0), o11 = mv.cell(iy1, ix1);
+        float sn, cs;
+        sincos_angle(2.0f * alpha, sn, cs);
+        const float q = t * cs, u = t * sn;
+#pragma unroll 1
+        for (int c = 0; c < 4; c++) {
+            const bool row = c & 2, col = c & 1;
+            int64_t o = row ? (col ? o11 : o10) : (col ? o01 : o00);
+            const float w = (row ? p.dy : 1.0f - p.dy) * (col ? p.dx : 1.0f - p.dx);
+            if (o >= 0) {
+                o += mv.inside(row ? iy1 : p.iy0, col ? ix1 : p.ix0);
                 unsafeAtomicAdd(lmap + o, w * t);
                 unsafeAtomicAdd(lmap + o + mv.polstride, w * q);
                 unsafeAtomicAdd(lmap + o + 2 * mv.polstride, w * u);
@@ -324,7 +422,8 @@ struct QuadPlace
     int mj, mn;            // smallest corner on the major and minor axis
     uint32_t at;           // bit 2 * a + b: some sample's corner is at (mj + a, mn + b)
     int base[3];           // elements of (mj + m, mn)
-    bool fits;
+    bool near;             // the footprints are within 3 x 3 pixels,
+    bool fits;             // which the window holds
 };
 
 template<bool Periodic>
@@ -357,7 +456,8 @@ __device__ inline QuadPlace place_quad(const Place (&p)[4], const Window &win, i
         }
     }
     // x0 = nx - 1 of periodic x has its second column at x = 0.
-    z.fits = ej - z.mj <= 1 && en - z.mn <= 1 && j >= 0 && j + (j2 ? 2 : 1) < win.length && lo >= 0
+    z.near = ej - z.mj <= 1 && en - z.mn <= 1;
+    z.fits = z.near && j >= 0 && j + (j2 ? 2 : 1) < win.length && lo >= 0
              && hi + (n2 ? 2 : 1) < win.width && !(Periodic && (win.xmajor ? ej : en) + 1 >= nx);
     return z;
 }
@@ -417,7 +517,7 @@ unplanned_tod2map_kernel(float *__restrict__ lmap, const float *__restrict__ tod
 {
     __shared__ __align__(16) WindowSums acc;
     __shared__ Extremes s_ext[WIN_WAVES];
-    __shared__ uint32_t s_err, s_split;
+    __shared__ uint32_t s_err, s_split, s_use;
     if (threadIdx.x == 0)
         s_err = s_split = 0;
     window_clear(acc);
@@ -479,31 +579,69 @@ unplanned_tod2map_kernel(float *__restrict__ lmap, const float *__restrict__ tod
         bool fits = !__any(n > 0 && !(z.fits && finite));
         if (!fits && (threadIdx.x & 63) == 0)
             s_split = 1;
+        if (threadIdx.x == 0)
+            s_use = 0;
         __syncthreads();
-        const int part = s_split ? 1 : WIN_WAVES;
-#pragma unroll 1
-        for (int w0 = 0; w0 < WIN_WAVES; w0 += part) {
-            if (part == 1) {
-                win = make_window(s_ext[w0]);
-                z = place_quad<Periodic>(p, win, nx);
-                fits = !__any(n > 0 && !(z.fits && finite));
+        // A wave whose lanes' samples do not fit (faster than half a pixel per sample, a few of many
+        // detectors, scattered) adds those that its window holds one by one, if they are enough to be worth
+        // a round; the rest go to the map.
+        const bool split = s_split;
+        uint32_t held = 0, rounds = 1;
+        bool use = __any(n > 0);
+        if (split) {
+            win = make_window(s_ext[wave]);
+            z = place_quad<Periodic>(p, win, nx);
+            fits = !__any(n > 0 && !(z.fits && finite));
+            if (!fits) {
+                int nheld = 0;
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    int next;
+                    const bool in = k < n && find_sample<Periodic>(p[k], win, nx, next) >= 0;
+                    held |= in ? 1u << k : 0u;
+                    nheld += __popcll(__ballot(in));
+                }
+                use = nheld >= WIN_SHARE && gridDim.x >= WIN_SHARE_BLOCKS;
+                held = use ? held : 0u;
             }
-            if (n > 0 && wave >= w0 && wave < w0 + part) {
+            if (use && (threadIdx.x & 63) == 0)
+                atomicOr(&s_use, 1u << wave);
+            __syncthreads();
+            rounds = s_use;
+            if (threadIdx.x == 0)
+                s_split = 0;                              // every wave has read it
+        }
+#pragma unroll 1
+        for (; rounds; rounds &= rounds - 1) {
+            const int w0 = __builtin_ctz(rounds);
+            if (split)
+                win = make_window(s_ext[w0]);
+            if (n > 0 && (!split || wave == w0)) {
                 if (fits)
                     deposit_quad(p, t, q, u, z, win, acc);
                 else {
 #pragma unroll
                     for (int k = 0; k < 4; k++)
-                        if (k < n)
-                            deposit_sample<Periodic>(p[k], t[k], q[k], u[k], win, acc, lmap, mv, nx, partial, err);
+                        if ((held >> k) & 1u)
+                            deposit_sample<Periodic>(p[k], t[k], q[k], u[k], win, acc, nx);
                 }
             }
             __syncthreads();
             window_flush(win, acc, lmap, mv, partial, err);
             __syncthreads();
         }
-        if (threadIdx.x == 0)
-            s_split = 0;                                  // every wave has read it; the next tile synchronizes first
+        if (!fits) {
+            const bool near = held == 0 && z.near;
+            uint64_t done = 0;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const uint64_t b = __ballot(near || ((held >> k) & 1u));
+                done = ((threadIdx.x & 3) == k) ? b : done;
+            }
+            if (near && n > 0)
+                deposit_near<Periodic>(p, t, q, u, lmap, mv, nx, partial, err);
+            deposit_far<Periodic>(lmap, tod, xp, nsamp, base + 256 * wave, s1, done, g, mv, partial, err);
+        }
     }
 
     err = wave_or_u(err | chk.bits(g));

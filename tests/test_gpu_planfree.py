@@ -141,3 +141,59 @@ def test_planfree_tod2map_large_map(gmm, orc, dev, kind, periodic):
     # The bound of the smaller maps: roundings of the weights (exact differences of coordinates here too).
     assert np.all(np.abs(got - ref) <= 2e-6 * mag + 1e-6 * np.abs(tod).max())
     assert np.sum(np.abs(got - ref)) <= 1e-5 * np.sum(np.abs(ref))
+
+
+def make_runs(kind, n, periodic, seed):
+    """Samples of which a window holds some or none: detectors of 16 samples at places of their own, short
+    turns, and scans too fast for four samples in 3 x 3 pixels."""
+    rng = np.random.default_rng(seed)
+    t = np.arange(n, dtype=np.float64)
+    hi = NX - (0 if periodic else 2)
+    if kind == "detectors":
+        run = np.arange(n) // 16
+        y, x = rng.uniform(0, NY - 4, run[-1] + 1)[run] + 0.1 * (t % 16), rng.uniform(0, hi, run[-1] + 1)[run] + 0.13 * (t % 16)
+    elif kind == "turns":
+        y, x = 100 + 60 * np.sin(t / 700), 300 + 90 * np.abs((t / 150) % 2 - 1)
+    elif kind == "fast_x":
+        y, x = 40 + 0.02 * t % 200, 1.3 * t % hi
+    else:                                # "fast_y"
+        y, x = NY / 2 + (NY / 2 - 3) * (2 * np.abs((t / 250) % 2 - 1) - 1), 50 + 0.011 * t % 600
+    x = x % hi if periodic else np.clip(x, 0, hi)
+    xp = np.stack([np.clip(y, 0, NY - 1), x, 0.3 + 0.001 * t]).astype(F32)
+    xp[1] = np.minimum(xp[1], np.nextafter(F32(NX), F32(0)) if periodic else F32(hi))
+    return np.ascontiguousarray(xp)
+
+
+@pytest.mark.parametrize("kind", ["detectors", "turns", "fast_x", "fast_y"])
+@pytest.mark.parametrize("n", [33, 3001, 70002])                # one block, a few, and more than 64
+@pytest.mark.parametrize("periodic", [False, True])
+def test_planfree_tod2map_outside(gmm, orc, dev, kind, n, periodic):
+    xp = make_runs(kind, n, periodic, n)
+    tod = np.random.default_rng(n).standard_normal(n).astype(F32)
+    # Every third cell is absent.
+    cells = [(cy, cx) for cy in range(5) for cx in range(11) if (cy + cx) % 3]
+    lp = gmm.LocalPixelization.make_cells(NY, NX, cells, periodic_xcoord=periodic)
+    pix = orc.Pix(NY, NX, lp.cell_offsets_cpu, 64, 4096, periodic)
+    for lmap, opix, partial in [(lp, pix, True), (gmm.LocalPixelization.make_rectangle(NY, NX, periodic_xcoord=periodic),
+                                                  orc.Pix.rectangle(NY, NX, periodic), False)]:
+        ref, err = orc.tod2map(tod.astype(np.float64), xp, opix, partial=partial, f64=True)
+        assert err == 0
+        got = run(gmm, dev, lmap, xp, tod, partial).astype(np.float64)
+        mag, _ = orc.tod2map(np.abs(tod).astype(np.float64), np.stack([xp[0], xp[1], 0 * xp[2]]), opix, partial=partial,
+                             f64=True)
+        if partial:
+            mag = np.repeat(mag.reshape(-1, 3, 4096)[:, :1], 3, axis=1).reshape(-1)
+        else:
+            mag = np.tile(mag.reshape(3, -1)[0], 3)
+        assert np.all(np.abs(got - ref) <= 2e-6 * mag + 1e-6 * np.abs(tod).max())
+    if n > 100:
+        with pytest.raises(RuntimeError, match="not in LocalPixelization"):
+            run(gmm, dev, lp, xp, tod)
+    # A value that is not finite reaches its own four pixels alone.
+    k = n // 2
+    tod[k] = np.nan
+    got = run(gmm, dev, lmap, xp, tod).reshape(3, lmap.nycells * 64, lmap.nxcells * 64)
+    iy, ix = min(int(xp[0, k]), NY - 2), int(xp[1, k]) if periodic else min(int(xp[1, k]), NX - 2)
+    hit = np.zeros(got.shape, bool)
+    hit[:, iy:iy + 2, [ix, (ix + 1) % NX]] = True
+    assert np.all(np.isnan(got[hit])) and not np.any(np.isnan(got[~hit]))
