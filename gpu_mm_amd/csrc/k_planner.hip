@@ -87,7 +87,10 @@ __device__ inline void sample_cells(float y, float x, const Geom &g, Checks &chk
 // line, and when they are the same or neighbours along one axis, the line's cells are exactly these
 // (the lowest sample touches the one, the highest the other). A line that spans two cells along both
 // axes takes the union of its samples' corners in these 2 x 2 cells. Anything else (longer lines, the
-// wrap of periodic x) is found sample by sample, by repeated extraction.
+// wrap of periodic x) is found sample by sample, by repeated extraction, two such lines at a time: 4.2e6
+// scattered samples take 154 us to count and 597 us in all to plan (one line at a time, loaded again for
+// the count and the emit's two passes, 202 and 760; sample by sample throughout 159 and 629); 6.7e7 at 3
+// pixels per sample 223 and 840 us (266 and 1010; 321 and 1024).
 // Working through every sample's four corners, with ballots over them, took 68 and 101 instructions
 // per sample, 0.93 and 1.38 ms of VALU issue in the 1.01 and 1.62 ms of the passes on 2048x262144
 // samples. By ranges the count takes 0.63 ms (6.8 TB/s: the 4.3 GB it reads) and the emit 0.87 ms (at
@@ -132,6 +135,13 @@ __device__ inline void load_quad(const float *__restrict__ p, int64_t nsamp, int
 __device__ inline int samples_left(int64_t line, int64_t l1, int64_t nsamp, int cap)
 {
     return int(max<int64_t>(0, min<int64_t>(cap, min(nsamp, l1 * LINE) - line * LINE)));
+}
+
+// Lines a wave takes at a time: fewer than eight where the block has not as many for each wave, for the sake
+// of slow ones, which a wave does in pairs (preplan of 32768 scattered samples 59 us, 45 so).
+__device__ inline int lines_per_wave(int64_t nlines, int nwaves)
+{
+    return int(min<int64_t>(SCAN_LINES, (nlines + nwaves - 1) / nwaves));
 }
 
 // x after the wrap of locate_op: in [0, nx] for every valid x.
@@ -229,22 +239,40 @@ __device__ inline LineCells line_cells(const QuadRange &q, const float (&y)[4], 
     return l;
 }
 
-// Number of cells of a slow line of n samples from s0, by the whole wave: one sample per lane.
-template<bool Periodic, typename F>
-__device__ inline uint32_t slow_line(const float *__restrict__ xp, int64_t nsamp, int64_t s0, const Geom &g, F &&each)
+// The samples of a wave's eight lines in LDS, for those of its lines that are slow.
+struct __align__(16) WaveSamples
 {
-    const int lane = lane_id();
-    const bool act = lane < 32 && s0 + lane < nsamp;
-    uint32_t k[4];
-    Checks unchecked;                          // the line's ranges were checked already
-    sample_cells<Periodic>(act ? xp[s0 + lane] : 0.0f, act ? xp[nsamp + s0 + lane] : 0.0f, g, unchecked, act, k);
-    uint32_t c, n = 0;
-    bool lo, hi;
-    while (extract_one(k, c, lo, hi)) {
-        each(n, __builtin_amdgcn_readfirstlane(c));
-        n++;
+    float y[SCAN_LINES * LINE], x[SCAN_LINES * LINE];
+
+    __device__ void put(const float (&yq)[4], const float (&xq)[4])
+    {
+        const int lane = lane_id();
+        *reinterpret_cast<float4 *>(y + 4 * lane) = make_float4(yq[0], yq[1], yq[2], yq[3]);
+        *reinterpret_cast<float4 *>(x + 4 * lane) = make_float4(xq[0], xq[1], xq[2], xq[3]);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
-    return n;
+};
+
+// Two slow lines at a time, la in lanes 0..31 and lb in 32..63 (lb = la: one line only), a sample per lane:
+// their footprint cells go to k for extract_one(). s0: first sample of the wave's lines.
+template<bool Periodic>
+__device__ inline void slow_pair(const WaveSamples &w, int la, int lb, int64_t s0, int64_t nsamp, const Geom &g, uint32_t k[4])
+{
+    const int lane = lane_id(), i = LINE * ((lane < 32) ? la : lb) + (lane & 31);
+    Checks unchecked;                          // the line's ranges were checked already
+    const bool act = (lane < 32 || lb != la) && s0 + i < nsamp;
+    sample_cells<Periodic>(w.y[i], w.x[i], g, unchecked, act, k);
+}
+
+// The next pair of the slow lines in m, a bit for the first lane of each.
+__device__ inline void next_pair(uint64_t &m, int &la, int &lb)
+{
+    la = __builtin_ctzll(m) >> 3;
+    m &= m - 1;
+    lb = m ? __builtin_ctzll(m) >> 3 : la;
+    m &= m - 1;
 }
 
 // ------------------------------------------------------------------------------------------
@@ -260,6 +288,7 @@ preplan_count_kernel(const float *__restrict__ xp, int64_t nsamp, int64_t ncl, i
                      int ny, int nx, uint32_t *__restrict__ nmt_out, uint32_t *__restrict__ err_out)
 {
     __shared__ uint32_t s_cnt[PP_THREADS / WAVE], s_err[PP_THREADS / WAVE];
+    __shared__ WaveSamples s_samples[PP_THREADS / WAVE];
     const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     constexpr int NW = PP_THREADS / WAVE;
     const int q = lane & 7;
@@ -271,13 +300,14 @@ preplan_count_kernel(const float *__restrict__ xp, int64_t nsamp, int64_t ncl, i
     const Geom g = make_geom(ny, nx, Periodic);
     Checks chk;
 
-    for (int64_t lb = l0 + SCAN_LINES * wave; lb < l1; lb += SCAN_LINES * NW * PP_UNROLL) {
+    const int lpw = lines_per_wave(l1 - l0, NW);
+    for (int64_t lb = l0 + lpw * wave; lb < l1; lb += lpw * NW * PP_UNROLL) {
         float y[PP_UNROLL][4], x[PP_UNROLL][4];
         int n[PP_UNROLL];
 #pragma unroll
         for (int u = 0; u < PP_UNROLL; u++) {
-            const int64_t line = lb + SCAN_LINES * NW * u;         // the wave's first line of the group
-            n[u] = min(max(samples_left(line, l1, nsamp, SCAN_LINES * LINE) - 4 * lane, 0), 4);
+            const int64_t line = lb + lpw * NW * u;                // the wave's first line of the group
+            n[u] = min(max(samples_left(line, l1, nsamp, lpw * LINE) - 4 * lane, 0), 4);
             load_quad<Vec>(xp + line * LINE + 4 * lane, nsamp, n[u], y[u], x[u]);
         }
 #pragma unroll
@@ -286,9 +316,17 @@ preplan_count_kernel(const float *__restrict__ xp, int64_t nsamp, int64_t ncl, i
             const LineCells l = line_cells<Periodic>(r, y[u], x[u], n[u] > 0, g);
             const bool lead = (q == 0) && n[u] > 0;
             cnt += lead ? uint32_t(__popc(l.at)) : 0u;
-            for (uint64_t m = __ballot(lead && l.slow); m; m &= m - 1) {
-                const int64_t line = lb + SCAN_LINES * NW * u + (__builtin_ctzll(m) >> 3);
-                slow_cnt += slow_line<Periodic>(xp, nsamp, line * LINE, g, [](uint32_t, uint32_t) {});
+            uint64_t m = __ballot(lead && l.slow);
+            if (m)
+                s_samples[wave].put(y[u], x[u]);
+            while (m) {
+                int la, lb2;
+                next_pair(m, la, lb2);
+                uint32_t k[4], c;
+                slow_pair<Periodic>(s_samples[wave], la, lb2, (lb + lpw * NW * u) * LINE, nsamp, g, k);
+                bool lo, hi;
+                while (extract_one(k, c, lo, hi))
+                    slow_cnt += uint32_t(lo) + uint32_t(hi);
             }
         }
     }
@@ -354,8 +392,7 @@ preplan_finish_kernel(uint32_t *nmt, uint32_t *err, int nblocks)
 // marked QM_PENDING and done by qmask_kernel afterwards.
 
 constexpr int EM_THREADS = 512;
-constexpr int EM_NW = EM_THREADS / WAVE;
-constexpr int EM_LINES = SCAN_LINES * EM_NW;           // lines per block step (64; 128 measure the same)
+constexpr int EM_NW = EM_THREADS / WAVE;               // 64 lines per block step (128 measure the same)
 constexpr uint16_t QM_PENDING = 0x8000;
 constexpr int QM_SHIFT = 48;
 constexpr int NML_SHIFT = 8;
@@ -370,6 +407,8 @@ plan_emit_kernel(const float *__restrict__ xp, int64_t nsamp, int64_t ncl, int64
 {
     __shared__ uint32_t s_total[2][EM_NW];
     __shared__ uint32_t s_err[EM_NW], s_nml[EM_NW];
+    __shared__ WaveSamples s_samples[EM_NW];
+    __shared__ uint32_t s_cells[EM_NW][SCAN_LINES][LINE];      // cells of the wave's slow lines
     const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const int li = lane >> 3, q = lane & 7;
     const int b = blockIdx.x;
@@ -387,9 +426,10 @@ plan_emit_kernel(const float *__restrict__ xp, int64_t nsamp, int64_t ncl, int64
     Checks chk;
     int parity = 0;
 
-    for (int64_t ls = l0; ls < l1; ls += EM_LINES) {
-        const int64_t lw = ls + SCAN_LINES * wave;         // the wave's first line
-        const int n = min(max(samples_left(lw, l1, nsamp, SCAN_LINES * LINE) - 4 * lane, 0), 4);
+    const int lpw = lines_per_wave(l1 - l0, EM_NW);
+    for (int64_t ls = l0; ls < l1; ls += lpw * EM_NW) {
+        const int64_t lw = ls + lpw * wave;                // the wave's first line
+        const int n = min(max(samples_left(lw, l1, nsamp, lpw * LINE) - 4 * lane, 0), 4);
         float y[4], x[4];
         load_quad<Vec>(xp + lw * LINE + 4 * lane, nsamp, n, y, x);
 
@@ -427,11 +467,23 @@ plan_emit_kernel(const float *__restrict__ xp, int64_t nsamp, int64_t ncl, int64
             z = (at > 1u) ? (uint32_t(MFLAG >> 32) | (zf ? uint32_t(ZFLAG >> 32) : 0u)) : 0u;
             nml += uint32_t(__popcll(__ballot(lead && at > 1u)));
         }
-        for (uint64_t sm = slow; sm; sm &= sm - 1) {
-            const int src = __builtin_ctzll(sm);
-            const uint32_t c = slow_line<Periodic>(xp, nsamp, (lw + (src >> 3)) * LINE, g, [](uint32_t, uint32_t) {});
-            cnt = (lane == src) ? c : cnt;
-            nml += (c > 1) ? 1u : 0u;
+        if (slow)
+            s_samples[wave].put(y, x);
+        for (uint64_t sm = slow; sm;) {
+            int la, lb;
+            next_pair(sm, la, lb);
+            uint32_t k[4], c, nlo = 0, nhi = 0, mine = NO_CELL;
+            slow_pair<Periodic>(s_samples[wave], la, lb, lw * LINE, nsamp, g, k);
+            bool lo, hi;
+            while (extract_one(k, c, lo, hi)) {
+                mine = (uint32_t(lane & 31) == ((lane < 32) ? nlo : nhi)) ? c : mine;
+                nlo += lo;
+                nhi += hi;
+            }
+            if (mine != NO_CELL)
+                s_cells[wave][(lane < 32) ? la : lb][lane & 31] = mine;
+            cnt = (lane == 8 * la) ? nlo : ((lane == 8 * lb) ? nhi : cnt);
+            nml += uint32_t(nlo > 1) + uint32_t(nhi > 1);
         }
 
         // Offsets of the wave's lines, then of the step's waves, in line order.
@@ -458,21 +510,34 @@ plan_emit_kernel(const float *__restrict__ xp, int64_t nsamp, int64_t ncl, int64
             else
                 err |= ERR_INCONSISTENT_NMT;
         }
-        for (uint64_t sm = slow; sm; sm &= sm - 1) {
-            const int src = __builtin_ctzll(sm);
-            const int64_t line = lw + (src >> 3);
-            const uint32_t soff = __builtin_amdgcn_readlane(off, src), c = __builtin_amdgcn_readlane(cnt, src);
-            slow_line<Periodic>(xp, nsamp, line * LINE, g, [&](uint32_t i, uint32_t key) {
-                // The first cell extracted is the first sample's.
-                const uint64_t mt = uint64_t(key) | (uint64_t(line) << ICL_SHIFT) | (uint64_t(QM_PENDING) << QM_SHIFT)
+        for (uint64_t sm = slow; sm;) {
+            int la, lb;
+            next_pair(sm, la, lb);
+            const int ln = (lane < 32) ? la : lb, sub = lane & 31;
+            const uint32_t soff = __shfl(off, 8 * ln, WAVE), c = __shfl(cnt, 8 * ln, WAVE);
+            const bool mine = lane < 32 || lb != la;
+            // The first cell extracted is the first sample's.
+            auto store = [&](uint32_t i, uint32_t key) {
+                const uint64_t mt = uint64_t(key) | (uint64_t(lw + ln) << ICL_SHIFT) | (uint64_t(QM_PENDING) << QM_SHIFT)
                                   | ((c > 1) ? MFLAG : 0ull) | ((c > 1 && i == 0) ? ZFLAG : 0ull);
-                if (lane == 0) {
-                    if (soff + i < limit)
-                        out[soff + i] = mt;
-                    else
-                        err |= ERR_INCONSISTENT_NMT;
+                if (soff + i < limit)
+                    out[soff + i] = mt;
+                else
+                    err |= ERR_INCONSISTENT_NMT;
+            };
+            if (mine && uint32_t(sub) < c)
+                store(uint32_t(sub), s_cells[wave][ln][sub]);
+            // Cells beyond 32 of a line (not reachable by ordinary scans) are extracted again.
+            if (__any(mine && c > 32)) {
+                uint32_t k[4], key, i = 0;
+                slow_pair<Periodic>(s_samples[wave], la, lb, lw * LINE, nsamp, g, k);
+                bool lo, hi;
+                while (extract_one(k, key, lo, hi)) {
+                    if (sub == 0 && i >= 32 && key != NO_CELL)
+                        store(i, key);
+                    i += ((lane < 32) ? lo : hi) ? 1u : 0u;
                 }
-            });
+            }
         }
 
         running += step_total;

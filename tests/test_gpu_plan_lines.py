@@ -88,3 +88,35 @@ def test_plan_lines(gmm, orc, dev, kind, n, offset):
     nb = (2 * nmt + 127) // 128 * 128
     got = plan.buf[pre.plan_nbytes - nb:pre.plan_nbytes - nb + 2 * nmt].cpu().numpy().view(np.uint16)
     assert np.array_equal(got, masks(orc, ref, xp, ny, nx, periodic))
+
+
+@pytest.mark.parametrize("periodic", [False, True])
+@pytest.mark.parametrize("n", [31, 500, 32 * 40 + 7, 32 * 16 * 70, 32 * 1024 * 20 + 65])
+@pytest.mark.parametrize("share", [0.1, 0.5, 1.0])
+def test_scattered_lines(gmm, orc, dev, n, share, periodic):
+    """Lines of many cells among ordinary ones, one, several or all of a wave's, of up to 128 cells (every
+    sample at a corner of four) and with few lines to a block or many."""
+    ny, nx = 1000, 2000
+    rng = np.random.default_rng(n + int(10 * share))
+    line = np.arange(n) // 32
+    nl = line[-1] + 1
+    kind = rng.choice([0, 1, 2], nl, p=[1 - share, share / 2, share / 2])[line]
+    t = np.arange(n) % 32
+    y, x = rng.uniform(0, ny - 20, nl)[line] + 0.1 * t, rng.uniform(0, nx - 20, nl)[line] + 0.3 * t
+    ys, xs = rng.uniform(0, ny - 1.5, n), rng.uniform(0, nx - 2.5, n)
+    corner = lambda m, k: 64.0 * rng.integers(1, (m - 2) // 64, k) - 0.5
+    y = np.choose(kind, [y, ys, corner(ny, n)])
+    x = np.choose(kind, [x, xs, corner(nx, n)])
+    if periodic:
+        x = np.where(kind == 1, x + rng.choice([-nx, 0, nx], n), x)
+    xp = np.stack([y, x, 0 * y]).astype(F32)
+    xp[1] = np.clip(xp[1], -nx, 2 * nx) if periodic else xp[1]
+    ref, err = orc.plan_build(xp, ny, nx, periodic)
+    assert err == 0
+    xg = torch.from_numpy(xp).to(dev)
+    pre = gmm.PointingPrePlan(xg, ny, nx, periodic_xcoord=periodic)
+    cum, nmt, _ = orc.plan_count(xp, ny, nx, periodic)
+    assert pre.plan_nmt == nmt and np.array_equal(pre.get_nmt_cumsum(), cum)
+    plan = gmm.PointingPlan(pre, xg, debug=True)
+    assert np.array_equal(plan.get_plan_mt(), ref)
+    assert plan.nmlines == int(np.sum(ref >> np.uint64(47) & np.uint64(1)))
