@@ -181,8 +181,8 @@ void plan_small(const gmm_preplan &pp, const uint64_t *items, uint64_t *out, uin
 // The owned-quad masks that the emit pass left pending.
 void plan_masks(const gmm_preplan &pp, const uint64_t *sorted_mt, const float *xp, uint16_t *qmask, hipStream_t stream);
 
-// Lists that were too long to be put in order on the way are in the scratch; this orders them, their
-// lengths known on the host. Returns whether it launched anything.
+// Lists that were too long to be put in order on the way are in the scratch, in plan order; this orders
+// them, their lengths known on the host. Returns whether it launched anything.
 bool order_long_lists(const gmm_preplan &pp, const PlanLists &l, int64_t n_m2t, int64_t n_t2m, const uint32_t *counts_gpu,
                       uint64_t *a, uint64_t *b, void *scratch, hipStream_t stream);
 

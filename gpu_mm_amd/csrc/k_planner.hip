@@ -879,9 +879,12 @@ work_list_kernel(const uint32_t *__restrict__ begin, uint32_t kx, int64_t nkeys,
 
 // Largest-first order of a list (entries equal in size in plan order), so that the operators' last
 // blocks are short ones (tod2map 1.4% faster on the 2048x262144 raster): each wave counts the chunks
-// that go before its four. blockIdx.y tells the list.
+// that go before its four. blockIdx.y tells the list. Lists of more than RANK_MAX chunks are left to the
+// radix sort: n^2 comparisons cross its time near 9000 chunks (plans of as many cells with 30 entries each,
+// ranked / sorted, in us: 4096 chunks 150 / 197, 8192 203 / 216, 11264 256 / 223, 15872 334 / 233).
+constexpr uint32_t RANK_MAX = 9000;
 constexpr int RK_PER_WAVE = 4;
-constexpr int RK_LOADS = 8;                              // in flight (11000 chunks: 42 us one by one, 30 so)
+constexpr int RK_LOADS = 8;                              // in flight (4947 chunks: 42 us one by one, 30 so)
 constexpr int RK_PER_BLOCK = RK_PER_WAVE * (WL_THREADS / WAVE);
 
 struct RankList
@@ -893,13 +896,13 @@ struct RankList
 };
 
 __global__ void __launch_bounds__(WL_THREADS)
-rank_chunks_kernel(RankList a, RankList b)
+rank_chunks_kernel(RankList a, RankList b, uint32_t least)
 {
     const RankList l = blockIdx.y ? b : a;
     const int lane = lane_id(), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
-    const uint32_t n = uint32_t(min<int64_t>(*l.count, l.max_chunks));
+    const uint32_t n = *l.count;
     const uint32_t i0 = blockIdx.x * RK_PER_BLOCK + wave * RK_PER_WAVE;
-    if (i0 >= n)
+    if (i0 >= n || n <= least || n > min<int64_t>(RANK_MAX, l.max_chunks))
         return;
     Chunk own[RK_PER_WAVE];
     uint32_t rank[RK_PER_WAVE] = {};
@@ -1412,9 +1415,6 @@ SortLayout sort_layout(int64_t nmt)
 
 constexpr int64_t CAP_MAX = 8192;                        // entries per work unit
 
-// Lists of up to this many chunks are ordered by rank (n^2 comparisons: 16384 take about 40 us).
-constexpr int64_t RANK_MAX = 16384;
-
 // Blocks of the work list kernels, and the words that cell_runs_kernel leaves for each list.
 int64_t work_list_blocks(int64_t nkeys) { return nkeys / WL_THREADS + 1; }            // begin[nkeys] too
 int64_t block_count_words(int64_t nkeys) { return NCAPS * work_list_blocks(nkeys); }
@@ -1474,14 +1474,12 @@ void launch_work_lists(const uint64_t *mt, int64_t n, uint32_t kx, int64_t nkeys
     GMM_HIP(hipGetLastError());
 }
 
-// Orders the lists, of at most max_m2t and max_t2m chunks (0: leaves that one alone).
-void launch_rank(const PlanLists &l, const uint32_t *counts, int64_t max_m2t, int64_t max_t2m, hipStream_t stream)
+// Orders the lists of more than 'least' and up to RANK_MAX chunks, which have at most nmax.
+void launch_rank(const PlanLists &l, const uint32_t *counts, int64_t nmax, uint32_t least, hipStream_t stream)
 {
-    const RankList a{l.tmp_m2t, l.m2t, counts + PC_CHUNKS_M2T, max_m2t}, b{l.tmp_t2m, l.t2m, counts + PC_CHUNKS_T2M, max_t2m};
-    const int64_t n = std::max(max_m2t, max_t2m);
-    if (n <= 0)
-        return;
-    rank_chunks_kernel<<<dim3(unsigned((n + RK_PER_BLOCK - 1) / RK_PER_BLOCK), 2), WL_THREADS, 0, stream>>>(a, b);
+    const RankList a{l.tmp_m2t, l.m2t, counts + PC_CHUNKS_M2T, l.max_m2t}, b{l.tmp_t2m, l.t2m, counts + PC_CHUNKS_T2M, l.max_t2m};
+    const int64_t n = std::min<int64_t>(nmax, RANK_MAX);
+    rank_chunks_kernel<<<dim3(unsigned((n + RK_PER_BLOCK - 1) / RK_PER_BLOCK), 2), WL_THREADS, 0, stream>>>(a, b, least);
     GMM_HIP(hipGetLastError());
 }
 
@@ -1572,8 +1570,7 @@ void plan_schedule(const gmm_preplan &pp, const uint64_t *sorted_mt, const PlanL
     const int64_t nkeys = pp.nycells_g * pp.nxcells_g;
     launch_work_lists(sorted_mt, n, uint32_t(pp.nxcells_g), nkeys, l.begin, m2t_out(pp, l, counts_gpu),
                       t2m_out(pp, l, counts_gpu), stream);
-    if (l.max_m2t <= RANK_MAX && l.max_t2m <= RANK_MAX)
-        launch_rank(l, counts_gpu, l.max_m2t, l.max_t2m, stream);
+    launch_rank(l, counts_gpu, std::max(l.max_m2t, l.max_t2m), 0, stream);
 }
 
 void plan_small(const gmm_preplan &pp, const uint64_t *items, uint64_t *out, uint16_t *qmask, const PlanLists &l,
@@ -1606,21 +1603,18 @@ bool order_long_lists(const gmm_preplan &pp, const PlanLists &l, int64_t n_m2t, 
                       uint64_t *a, uint64_t *b, void *scratch, hipStream_t stream)
 {
     if (pp.plan_nmt <= SP_MAX) {                                     // plan_small() did the short ones
-        const int64_t r_m2t = (n_m2t > SP_RANK) ? n_m2t : 0, r_t2m = (n_t2m > SP_RANK) ? n_t2m : 0;
-        launch_rank(l, counts_gpu, r_m2t, r_t2m, stream);
-        return r_m2t > 0 || r_t2m > 0;
-    }
-    if (l.max_m2t <= RANK_MAX && l.max_t2m <= RANK_MAX)
-        return false;                                                // plan_schedule() did it
-    if (n_m2t <= RANK_MAX && n_t2m <= RANK_MAX) {
-        launch_rank(l, counts_gpu, n_m2t, n_t2m, stream);
+        static_assert(SP_MAX <= RANK_MAX, "small plans' lists are ranked");
+        if (n_m2t <= SP_RANK && n_t2m <= SP_RANK)
+            return false;
+        launch_rank(l, counts_gpu, std::max(n_m2t, n_t2m), SP_RANK, stream);
         return true;
     }
+    // plan_schedule() did lists of up to RANK_MAX.
     // a and b hold plan_nmt items each, a list at most as many. 13-bit keys: kx = 1024 makes the sort's
     // key the item's low 20 bits.
     uint8_t *sc = reinterpret_cast<uint8_t *>(scratch);
     auto order = [&](const Chunk *src, Chunk *dst, int64_t nch) {
-        if (nch <= 0)
+        if (nch <= RANK_MAX)
             return;
         SortLayout L = sort_layout(nch);
         uint32_t *hist = reinterpret_cast<uint32_t *>(sc + L.hist_off);
@@ -1644,7 +1638,7 @@ bool order_long_lists(const gmm_preplan &pp, const PlanLists &l, int64_t n_m2t, 
     };
     order(l.tmp_m2t, l.m2t, n_m2t);
     order(l.tmp_t2m, l.t2m, n_t2m);
-    return true;
+    return std::max(n_m2t, n_t2m) > RANK_MAX;
 }
 
 constexpr int64_t GENERIC_KEYS = int64_t(1) << 20;

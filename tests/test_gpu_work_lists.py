@@ -96,3 +96,19 @@ def test_long_list_ties(gmm, dev, kind, n, ny, nx):
         end -= align128(16 * nmax)
         check_list(buf[end:end + 16 * nmax].view(CHUNK), mt, opt, True)
     assert plan.nchunks > RANK_MAX
+
+
+@pytest.mark.parametrize("rows", [88, 90, 91, 112])              # x 100 cells: ranked up to 9000, sorted above
+def test_list_order_limit(gmm, dev, rows):
+    ny, nx, n = 64 * rows, 6400, 32 * 1500 * rows
+    xg = torch.from_numpy(make_pointing("lines", n, ny, nx)).to(dev)
+    pre = gmm.PointingPrePlan(xg, ny, nx, periodic_xcoord=False)
+    plan = gmm.PointingPlan(pre, xg, debug=True)
+    assert plan.nchunks == 100 * rows
+    nmt, mt = pre.plan_nmt, plan.get_plan_mt()
+    buf = plan.buf.cpu().numpy()
+    end = pre.plan_nbytes - align128(2 * nmt)
+    for opt in sizes(nmt)[::-1]:
+        nmax = bound(opt, nmt, 100 * rows)
+        end -= align128(16 * nmax)
+        check_list(buf[end:end + 16 * nmax].view(CHUNK), mt, opt, True)
