@@ -17,6 +17,7 @@ namespace {
 constexpr int SLOT_WORDS = 16;                // 64 bytes
 constexpr int NSLOTS = 64;                    // one page; each is in use by one call at a time
 constexpr int PB_THREADS = 256;
+constexpr int PB_LOADS = 16;                  // in flight per thread (a call with 262144 error words 907 -> 620 us)
 
 // Stores n words of src (their OR, when 'any') and then the ticket, where the host sees them. One block;
 // it runs after everything that was enqueued on its stream before it.
@@ -29,8 +30,17 @@ publish_words_kernel(const uint32_t *__restrict__ src, int64_t n, bool any, uint
         if (threadIdx.x == 0)
             s_or = 0;
         __syncthreads();
-        for (int64_t i = threadIdx.x; i < n; i += PB_THREADS)
-            v |= src[i];
+        for (int64_t i0 = 0; i0 < n; i0 += PB_THREADS * PB_LOADS) {
+            uint32_t w[PB_LOADS];
+#pragma unroll
+            for (int k = 0; k < PB_LOADS; k++) {
+                const int64_t i = i0 + k * PB_THREADS + threadIdx.x;
+                w[k] = (i < n) ? src[i] : 0u;
+            }
+#pragma unroll
+            for (int k = 0; k < PB_LOADS; k++)
+                v |= w[k];
+        }
         if (v)
             atomicOr(&s_or, v);
         __syncthreads();

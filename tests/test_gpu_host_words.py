@@ -71,3 +71,24 @@ def test_threads(gmm, dev):
     for t in ts:
         t.join(60)
     assert not failures and not any(t.is_alive() for t in ts)
+
+
+@pytest.mark.parametrize("bad", [None, 0, 4095 * 256, 4096 * 256, 5000 * 256 - 1])
+def test_many_words(gmm, dev, bad):
+    """A word of 5000 blocks, more than the reading block takes at a time."""
+    n = 5000 * 256
+    xg = make_pointing(n, 3, dev)
+    if bad is not None:
+        xg[0, bad] = -1.0
+    lp = gmm.LocalPixelization.make_rectangle(NY, NX, periodic_xcoord=False)
+    m = torch.ones(3 * lp.npix, dtype=torch.float32, device=dev)
+    tod = torch.zeros(n, dtype=torch.float32, device=dev)
+    words = torch.empty(8192, dtype=torch.uint32, device=dev)
+    ext = gmm.gpu_mm._ext
+    call = lambda: ext.unplanned_map2tod(tod, m, xg, lp, words, False, False, check_errors=True, stream=0)
+    torch.cuda.synchronize()
+    if bad is None:
+        call()
+    else:
+        with pytest.raises(RuntimeError, match="y-value"):
+            call()
