@@ -67,6 +67,7 @@ __global__ void dyn_count_kernel(const uint32_t *__restrict__ pos, int64_t n, ui
 // call: three timestreams of 300 x 16421 samples into a map that grows 441 -> 261 us.
 constexpr int DC_THREADS = 1024;
 constexpr int DC_MAX_WORDS = 1024 * 1024 / 32;
+constexpr int DC_LOADS = 8;                   // in flight per thread
 constexpr int64_t DC_MAX_CHUNKS = 32768;      // half a MiB for the one block to read, a few us
 
 __global__ void __launch_bounds__(DC_THREADS)
@@ -80,13 +81,29 @@ dyn_chunks_kernel(const Chunk *__restrict__ chunks, int nchunks, int64_t *__rest
     for (int i = t; i < nwords; i += DC_THREADS)
         s_bits[i] = 0;
     __syncthreads();
-    for (int i = t; i < nchunks; i += DC_THREADS) {
-        const uint32_t icell = chunks[i].icell, cy = icell >> 10, cx = icell & 1023u;
-        const uint32_t ioff = cy * nxcells + cx;
-        if (cy < nycells && cx < nxcells && cell_offsets[ioff] == -1)
-            atomicOr(&s_bits[ioff >> 5], 1u << (ioff & 31));
+    bool fresh = false;
+    for (int i0 = t; i0 < nchunks; i0 += DC_THREADS * DC_LOADS) {
+        uint32_t ioff[DC_LOADS];
+        bool absent[DC_LOADS];
+#pragma unroll
+        for (int k = 0; k < DC_LOADS; k++)
+            ioff[k] = chunks[min(i0 + k * DC_THREADS, nchunks - 1)].icell;
+#pragma unroll
+        for (int k = 0; k < DC_LOADS; k++) {
+            const uint32_t cy = ioff[k] >> 10, cx = ioff[k] & 1023u;
+            const bool in = i0 + k * DC_THREADS < nchunks && cy < nycells && cx < nxcells;
+            ioff[k] = in ? cy * nxcells + cx : 0u;
+            absent[k] = in && cell_offsets[ioff[k]] == -1;
+        }
+#pragma unroll
+        for (int k = 0; k < DC_LOADS; k++)
+            if (absent[k]) {
+                atomicOr(&s_bits[ioff[k] >> 5], 1u << (ioff[k] & 31));
+                fresh = true;
+            }
     }
-    __syncthreads();
+    if (!__syncthreads_or(fresh))
+        return;                                // as on every call but the first few of a loop
     // Thread t numbers the cells of words [per * t, per * t + per).
     const int w0 = per * t, w1 = min(w0 + per, nwords);
     uint32_t n = 0, total;
