@@ -486,7 +486,7 @@ int gmm_preplan_create(gmm_preplan **out, const float *xpointing_gpu, int64_t ns
         pp.off_qmask = pp.off_chunks_t2m + align128(int64_t(sizeof(Chunk)) * pp.max_nchunks_t2m);
         pp.plan_nbytes = pp.off_qmask + align128(2 * nmt);
 
-        pp.sort_nbytes = plan_scratch_nbytes(pp) + 128;
+        pp.sort_nbytes = plan_scratch_nbytes(pp) + PC_NBYTES;
         pp.tmp_nbytes = 2 * align128(8 * nmt) + pp.sort_nbytes;
 
         *out = new gmm_preplan(pp);
@@ -576,7 +576,7 @@ int gmm_plan_create(gmm_plan **out, const gmm_preplan *pp, const float *xpointin
             uint64_t *a = reinterpret_cast<uint64_t *>(tmp);
             uint64_t *b = reinterpret_cast<uint64_t *>(tmp + mt_bytes);
             uint8_t *scratch = tmp + 2 * mt_bytes;
-            const int64_t scratch_nbytes = pp->sort_nbytes - 128;
+            const int64_t scratch_nbytes = pp->sort_nbytes - PC_NBYTES;
             uint32_t *counts = reinterpret_cast<uint32_t *>(scratch + scratch_nbytes);
 
             uint32_t *err_word = plan->err + (pp->n_err - 1);

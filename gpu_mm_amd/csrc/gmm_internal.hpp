@@ -153,6 +153,8 @@ void plan_sort(const gmm_preplan &pp, uint64_t *a, uint64_t *b, uint64_t *out, u
 // Counts that plan construction keeps on the device; the first PC_WORDS are brought back to the host.
 enum PlanCount { PC_CHUNKS_M2T = 0, PC_NMLINES = 1, PC_ERROR = 2, PC_CHUNKS_T2M = 3, PC_WORDS = 4,
                  PC_CAPS_M2T = PC_WORDS, PC_CAPS_T2M = PC_CAPS_M2T + NCAPS, PC_TOTAL = PC_CAPS_T2M + NCAPS };
+constexpr int64_t PC_NBYTES = 128;             // kept for them in the scratch of plan construction
+static_assert(4 * PC_TOTAL <= PC_NBYTES, "the counts fit");
 
 // The sizes that the operators' work lists of a plan of pp.plan_nmt entries may be cut by, and the bounds
 // on the lists' lengths.

@@ -1433,7 +1433,8 @@ WorkListOut t2m_out(const gmm_preplan &pp, const PlanLists &l, uint32_t *counts)
 // Sizes for a plan of nmt entries on 'slots' blocks that run at once: lists of at most k * slots chunks (k
 // full rounds) with chunks up to 5, 15, 30 and 50% above an even share, ordered by the time that the
 // rounds take when a block costs as much as 'fixed' entries; no chunk is smaller than 'least' for the sake
-// of a round. Last comes 'general', which any list may take.
+// of a round. Three rounds 50% above, the costliest of the twelve, are not tried (NCAPS). Last comes
+// 'general', which any list may take.
 ChunkCaps make_caps(int64_t nmt, int64_t slots, int64_t fixed, int kmax, int64_t least, int64_t general)
 {
     struct Option { int64_t cap, limit, cost; };
@@ -1645,7 +1646,7 @@ constexpr int64_t GENERIC_KEYS = int64_t(1) << 20;
 
 int64_t build_chunks_generic_scratch_nbytes()
 {
-    return align128(4 * (GENERIC_KEYS + 1)) + 128 + 8 * block_count_words(GENERIC_KEYS);
+    return align128(4 * (GENERIC_KEYS + 1)) + PC_NBYTES + 8 * block_count_words(GENERIC_KEYS);
 }
 
 int64_t build_chunks_generic(const uint64_t *plan_mt_gpu, int64_t nmt, int64_t chunk_cap,
@@ -1653,7 +1654,7 @@ int64_t build_chunks_generic(const uint64_t *plan_mt_gpu, int64_t nmt, int64_t c
 {
     uint32_t *begin = static_cast<uint32_t *>(scratch);
     uint32_t *counts = begin + align128(4 * (GENERIC_KEYS + 1)) / 4;
-    uint32_t *block_counts = counts + 128 / 4;
+    uint32_t *block_counts = counts + PC_NBYTES / 4;
     fill_u32_kernel<<<1, 64, 0, stream>>>(counts, PC_TOTAL, 0u);
     GMM_HIP(hipGetLastError());
     ChunkCaps cap = {}, none = {};
