@@ -92,3 +92,45 @@ def test_many_words(gmm, dev, bad):
     else:
         with pytest.raises(RuntimeError, match="y-value"):
             call()
+
+
+def test_more_callers_than_slots(gmm, dev):
+    """80 calls that wait at once, behind work on one stream: those that find no slot of pinned memory
+    (there are 64) take a copy."""
+    nthreads = 80
+    good, bad = make_pointing(3000, 5, dev), make_pointing(3000, 5, dev)
+    bad[0, 1234] = NY + 1.0
+    nmt = gmm.PointingPrePlan(good, NY, NX, periodic_xcoord=False).plan_nmt
+    lp = gmm.LocalPixelization.make_rectangle(NY, NX, periodic_xcoord=False)
+    m = gmm.LocalMap(lp, torch.ones(3 * lp.npix, dtype=torch.float32, device=dev))
+    tods = torch.zeros((nthreads, 3000), dtype=torch.float32, device=dev)
+    torch.cuda.synchronize()
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        torch.cuda._sleep(40000000)
+    failures = []
+
+    def work(i):
+        try:
+            with torch.cuda.stream(s):
+                if i % 4 == 0:
+                    assert gmm.PointingPrePlan(good, NY, NX, periodic_xcoord=False).plan_nmt == nmt
+                elif i % 4 == 1:
+                    with pytest.raises(RuntimeError, match="y-value"):
+                        gmm.PointingPrePlan(bad, NY, NX, periodic_xcoord=False)
+                elif i % 4 == 2:
+                    gmm.map2tod(tods[i], m, good, None)
+                else:
+                    with pytest.raises(RuntimeError, match="y-value"):
+                        gmm.map2tod(tods[i], m, bad, None)
+        except BaseException as e:
+            failures.append((i, repr(e)))
+
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(nthreads)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join(60)
+    assert not failures and not any(t.is_alive() for t in ts)
+    want = 1 + torch.cos(2 * good[2]) + torch.sin(2 * good[2])
+    assert torch.allclose(tods[2::4], want.expand(20, 3000), atol=1e-5)

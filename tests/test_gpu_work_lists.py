@@ -112,3 +112,32 @@ def test_list_order_limit(gmm, dev, rows):
         nmax = bound(opt, nmt, 100 * rows)
         end -= align128(16 * nmax)
         check_list(buf[end:end + 16 * nmax].view(CHUNK), mt, opt, True)
+
+
+@pytest.mark.parametrize("kind,n", [("samples", 60000), ("lines", 32 * 90000)])
+def test_plan_on_another_stream(gmm, dev, kind, n):
+    """A plan may be used on any stream once its constructor returns, also where a list is sorted after
+    the counts have come back: operators started at once on a second stream against the same later."""
+    ny = nx = 6400                                       # 10000 cells
+    xg = torch.from_numpy(make_pointing(kind, n, ny, nx)).to(dev)
+    lp = gmm.LocalPixelization.make_rectangle(ny, nx, periodic_xcoord=False)
+    m = gmm.LocalMap(lp, torch.randn(3 * lp.npix, device=dev))
+    tod = torch.randn(n, device=dev)
+    made, used = torch.cuda.Stream(), torch.cuda.Stream()
+    out = torch.zeros(n, device=dev)
+    acc = gmm.LocalMap(lp, torch.zeros(3 * lp.npix, device=dev))
+    torch.cuda.synchronize()
+    with torch.cuda.stream(made):
+        pre = gmm.PointingPrePlan(xg, ny, nx, periodic_xcoord=False)
+        plan = gmm.PointingPlan(pre, xg)
+    with torch.cuda.stream(used):
+        gmm.map2tod(out, m, xg, plan)
+        gmm.tod2map(acc, tod, xg, plan)
+    torch.cuda.synchronize()
+    assert plan.nchunks > 9000
+    out2, acc2 = torch.zeros(n, device=dev), gmm.LocalMap(lp, torch.zeros(3 * lp.npix, device=dev))
+    gmm.map2tod(out2, m, xg, plan)
+    gmm.tod2map(acc2, tod, xg, plan)
+    assert torch.equal(out, out2)
+    # Blocks add to a pixel in any order: float32 rounding of a few deposits.
+    assert torch.allclose(acc.arr, acc2.arr, rtol=1e-5, atol=1e-5)
