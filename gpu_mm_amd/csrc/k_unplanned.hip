@@ -162,9 +162,17 @@ constexpr int WIN_SAMPLES = 4 * WIN_THREADS;
 constexpr int WIN_N = 1024;                // pixels of the window (24 KiB of sums: 6 blocks per CU)
 // Least number of a wave's 256 samples that are worth a round of their own (from a few detectors' turns to
 // 5 pixels per sample 16, 32 and 64 are the same; 128 takes 2400 us for 4.2e6 samples at 1 pixel per
-// sample along y, 32 takes 1610), and of blocks: a small call waits for its rounds (1000 samples 54 us, 49
-// straight to the map).
-constexpr int WIN_SHARE = 32, WIN_SHARE_BLOCKS = 64;
+// sample along y, 32 takes 1610). Calls of a few blocks could do without rounds (1000 samples 54 us, 49
+// straight to the map), but their sums would carry more float32 roundings.
+constexpr int WIN_SHARE = 32;
+// Lanes of a wave: with so many whose four samples step by a pixel or so, what its window does not hold is
+// left for deposit_far(), where consecutive lanes then meet in cache lines. In slower waves they would meet
+// in pixels and wait for each other (one detector's 2^21 samples at 0.58 pixel per sample, back and forth
+// over the same rows, 250 us; 178 when the lanes' samples follow one after the other): there all but those
+// for deposit_near(), if they are WIN_NEAR lanes or more, take the round together, and a few held ones are
+// enough for it when most are not near. Calls without a block for each CU wait for each pass: their slow
+// waves make one only (8 x 16384 samples 66 us, 70 with deposit_near()).
+constexpr int WIN_SOME = 32, WIN_NEAR = 24, WIN_BLOCKS = 256;
 constexpr int WIN_LEAD = 4;                // places before the least one seen (lanes show one of their 4 samples)
 typedef double WindowSums[3][WIN_N];
 
@@ -185,15 +193,11 @@ struct Window
     // product wraps, and the place is refused for its j.)
     __device__ int line(int j) const { return minor0 + (int(uint32_t(slope) * uint32_t(j - WIN_LEAD)) >> 16); }
 
-    // Element of the footprint's first pixel (and, in 'next', of the one beside it along the major axis)
-    // if all of a footprint that starts at (iy0, ix0) is held, else -1.
-    __device__ int find(int iy0, int ix0, int &next) const
+    // Element of a pixel, or -1.
+    __device__ int find(int iy, int ix) const
     {
-        const int j = place(xmajor ? ix0 : iy0), minor = xmajor ? iy0 : ix0;
-        const int k0 = minor - line(j), k1 = minor - line(j + 1);
-        const bool in = j >= 0 && j + 1 < length && min(k0, k1) >= 0 && max(k0, k1) + 1 < width;
-        next = (j + 1) * jstride + k1 * kstride;
-        return in ? j * jstride + k0 * kstride : -1;
+        const int j = place(xmajor ? ix : iy), k = (xmajor ? iy : ix) - line(j);
+        return (unsigned(j) < unsigned(length) && unsigned(k) < unsigned(width)) ? j * jstride + k * kstride : -1;
     }
 };
 
@@ -308,26 +312,31 @@ struct Place
     float dy, dx;
 };
 
-// Element of a sample's footprint in the window, or -1. x0 = nx - 1 of periodic x has its second column at
-// x = 0, outside.
+// The four corners of one sample: to the window or, outside it, to the map.
 template<bool Periodic>
-__device__ inline int find_sample(const Place &p, const Window &win, int nx, int &next)
+__device__ inline void deposit_sample(const Place &p, float t, float q, float u, const Window &win, WindowSums &acc,
+                                      float *__restrict__ lmap, const LocalMapView &mv, int nx, bool partial, uint32_t &err)
 {
-    const int e = win.find(p.iy0, p.ix0, next);
-    return (Periodic && p.ix0 + 1 >= nx) ? -1 : e;
-}
-
-// The four corners of one sample that the window holds.
-template<bool Periodic>
-__device__ inline void deposit_sample(const Place &p, float t, float q, float u, const Window &win, WindowSums &acc, int nx)
-{
-    int next;
-    const int e = find_sample<Periodic>(p, win, nx, next);
-    const float dj = win.xmajor ? p.dx : p.dy, dn = win.xmajor ? p.dy : p.dx;
 #pragma unroll 1
     for (int i = 0; i < 4; i++) {
-        const float w = ((i & 2) ? dj : 1.0f - dj) * ((i & 1) ? dn : 1.0f - dn);
-        window_add(acc, ((i & 2) ? next : e) + ((i & 1) ? win.kstride : 0), w * t, w * q, w * u);
+        const int iy = p.iy0 + (i >> 1);
+        int ix = p.ix0 + (i & 1);
+        if (Periodic)
+            ix = (ix < nx) ? ix : 0;
+        const float w = ((i & 2) ? p.dy : 1.0f - p.dy) * ((i & 1) ? p.dx : 1.0f - p.dx);
+        const int e = win.find(iy, ix);
+        if (e >= 0)
+            window_add(acc, e, w * t, w * q, w * u);
+        else {
+            const int64_t o = mv.offset(iy, ix);
+            if (o >= 0) {
+                unsafeAtomicAdd(lmap + o, w * t);
+                unsafeAtomicAdd(lmap + o + mv.polstride, w * q);
+                unsafeAtomicAdd(lmap + o + 2 * mv.polstride, w * u);
+            }
+            else if (!partial)
+                err |= ERR_NOT_IN_PIXELIZATION;
+        }
     }
 }
 
@@ -422,6 +431,7 @@ struct QuadPlace
     int mj, mn;            // smallest corner on the major and minor axis
     uint32_t at;           // bit 2 * a + b: some sample's corner is at (mj + a, mn + b)
     int base[3];           // elements of (mj + m, mn)
+    bool fast;             // the samples span more than three pixels along an axis
     bool near;             // the footprints are within 3 x 3 pixels,
     bool fits;             // which the window holds
 };
@@ -456,6 +466,7 @@ __device__ inline QuadPlace place_quad(const Place (&p)[4], const Window &win, i
         }
     }
     // x0 = nx - 1 of periodic x has its second column at x = 0.
+    z.fast = max(ej - z.mj, en - z.mn) > 2;
     z.near = ej - z.mj <= 1 && en - z.mn <= 1;
     z.fits = z.near && j >= 0 && j + (j2 ? 2 : 1) < win.length && lo >= 0
              && hi + (n2 ? 2 : 1) < win.width && !(Periodic && (win.xmajor ? ej : en) + 1 >= nx);
@@ -596,13 +607,20 @@ unplanned_tod2map_kernel(float *__restrict__ lmap, const float *__restrict__ tod
                 int nheld = 0;
 #pragma unroll
                 for (int k = 0; k < 4; k++) {
-                    int next;
-                    const bool in = k < n && find_sample<Periodic>(p[k], win, nx, next) >= 0;
+                    // (Of its four corners two opposite ones are looked at.)
+                    const bool in = k < n && max(win.find(p[k].iy0, p[k].ix0), win.find(p[k].iy0 + 1, p[k].ix0 + 1)) >= 0;
                     held |= in ? 1u << k : 0u;
                     nheld += __popcll(__ballot(in));
                 }
-                use = nheld >= WIN_SHARE && gridDim.x >= WIN_SHARE_BLOCKS;
-                held = use ? held : 0u;
+                const bool slow = __popcll(__ballot(n > 0 && z.fast)) < WIN_SOME, small = gridDim.x < WIN_BLOCKS;
+                const int nmid = __popcll(__ballot(n > 0 && !z.fast && !z.near));
+                const int napart = __popcll(__ballot(n > 0 && held == 0 && z.near));
+                use = (slow && small) || nheld >= ((nmid >= WIN_SOME) ? 1 : WIN_SHARE);
+                const bool apart = held == 0 && z.near && napart >= WIN_NEAR && !small;
+                if (!use)
+                    held = 0;
+                else if (slow && !apart)
+                    held = (1u << n) - 1u;
             }
             if (use && (threadIdx.x & 63) == 0)
                 atomicOr(&s_use, 1u << wave);
@@ -623,7 +641,7 @@ unplanned_tod2map_kernel(float *__restrict__ lmap, const float *__restrict__ tod
 #pragma unroll
                     for (int k = 0; k < 4; k++)
                         if ((held >> k) & 1u)
-                            deposit_sample<Periodic>(p[k], t[k], q[k], u[k], win, acc, nx);
+                            deposit_sample<Periodic>(p[k], t[k], q[k], u[k], win, acc, lmap, mv, nx, partial, err);
                 }
             }
             __syncthreads();
