@@ -137,11 +137,12 @@ __device__ inline int samples_left(int64_t line, int64_t l1, int64_t nsamp, int 
     return int(max<int64_t>(0, min<int64_t>(cap, min(nsamp, l1 * LINE) - line * LINE)));
 }
 
-// Lines a wave takes at a time: fewer than eight where the block has not as many for each wave, for the sake
-// of slow ones, which a wave does in pairs (preplan of 32768 scattered samples 59 us, 45 so).
+// Lines a wave takes at a time: eight, or fewer where the blocks don't fill the GPU and have not as many for
+// each wave, for the sake of slow ones, which a wave does in pairs (preplan of 32768 scattered samples 59 us,
+// 45 so; with the GPU full it costs the count of ordinary lines 1.6 us).
 __device__ inline int lines_per_wave(int64_t nlines, int nwaves)
 {
-    return int(min<int64_t>(SCAN_LINES, (nlines + nwaves - 1) / nwaves));
+    return (gridDim.x < 256) ? int(min<int64_t>(SCAN_LINES, (nlines + nwaves - 1) / nwaves)) : SCAN_LINES;
 }
 
 // x after the wrap of locate_op: in [0, nx] for every valid x.
