@@ -93,8 +93,8 @@ __device__ inline void sample_cells(float y, float x, const Geom &g, Checks &chk
 // pixels per sample 223 and 840 us (266 and 1010; 321 and 1024).
 // Working through every sample's four corners, with ballots over them, took 68 and 101 instructions
 // per sample, 0.93 and 1.38 ms of VALU issue in the 1.01 and 1.62 ms of the passes on 2048x262144
-// samples. By ranges the count takes 0.63 ms (6.8 TB/s: the 4.3 GB it reads) and the emit 0.87 ms (at
-// most 50 instructions per sample, 0.68 ms; loading a step ahead spills and takes 0.98).
+// samples. By ranges the count takes 0.65 ms (6.7 TB/s: the 4.3 GB it reads) and the emit 0.89 ms (41
+// instructions per sample, 0.56 ms; loading a step ahead spills and takes 0.98).
 
 constexpr int SCAN_LINES = 8;                 // lines per wave and load
 

@@ -609,15 +609,15 @@ class PointingPrePlan(_ext.PointingPrePlan):
 
 class PointingPlan(_ext.PointingPlan):
     """
-    Second planning step: the sorted list of (line, cell) entries plus the work list of the
-    planned kernels.
+    Second planning step: the sorted list of (line, cell) entries plus the work lists of the
+    planned kernels (one each).
 
     Arguments: preplan, xpointing_gpu (the same pointing as the preplan), buf (uint8, at least
     preplan.plan_nbytes; kept by the plan), tmp_buf (uint8, at least
     preplan.plan_constructor_tmp_nbytes; used only during construction), debug.
 
-    Attributes: nsamp, nypix_global, nxpix_global, periodic_xcoord, plan_nmt, nchunks,
-    nmlines; get_plan_mt() returns the entries (uint64, bit layout of the reference).
+    Attributes: nsamp, nypix_global, nxpix_global, periodic_xcoord, plan_nmt, nchunks (of
+    map2tod's list), nmlines; get_plan_mt() returns the entries (uint64, bit layout of the reference).
 
     With debug=True the constructor also checks the plan's invariants on the device
     (check_invariants()), and raises RuntimeError if one is broken.

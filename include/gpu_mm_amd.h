@@ -94,7 +94,7 @@ typedef struct {
     int64_t nmt_per_threadblock, pointing_nblocks; /* reference launch formulas, informational */
     int64_t plan_nmt;
     int64_t cub_nbytes;                  /* bytes of radix-sort scratch inside tmp_buf */
-    int64_t max_nchunks;                 /* upper bound on operator work units */
+    int64_t max_nchunks;                 /* upper bound on map2tod's work units (gmm_plan_info) */
 } gmm_preplan_info;
 
 int gmm_preplan_create(gmm_preplan **out, const float *xpointing_gpu, int64_t nsamp,
@@ -112,16 +112,19 @@ int gmm_preplan_get_nmt_cumsum(const gmm_preplan *pp, uint32_t *out_cpu, int64_t
  * bound at gpu_mm_pybind11.cu:133-153). 'buf' (>= plan_nbytes, 128-byte aligned) is kept by
  * the plan and must not be shared; 'tmp_buf' (>= plan_constructor_tmp_nbytes) is used only
  * during construction. Layout of buf: uint64 plan_mt[nmt] at offset 0, then uint32 err[...]
- * at align128(8*nmt), then the operator work list. Blocks on the stream once. debug=1 also
- * checks the plan's invariants on the device (gmm_plan_check_invariants) and fails if one is
- * broken (PointingPlan.cu:272-283 launches its Debug planner kernel instead).
+ * at align128(8*nmt), then the work lists of map2tod and of tod2map, then uint16 masks[nmt] (the
+ * groups of 4 samples that each entry evaluates), each from a multiple of 128 bytes on. Blocks on
+ * the stream once, and a second time where a work list is too long to be ordered before its
+ * length is known (more than some thousand work units). debug=1 also checks the plan's invariants
+ * on the device (gmm_plan_check_invariants) and fails if one is broken (PointingPlan.cu:272-283
+ * launches its Debug planner kernel instead).
  * --------------------------------------------------------------------------------------- */
 
 typedef struct {
     int64_t nsamp, nypix_global, nxpix_global;
     int32_t periodic_xcoord;
     int64_t plan_nmt;
-    int64_t nchunks;       /* operator work units (blocks per map2tod/tod2map launch) */
+    int64_t nchunks;       /* work units of map2tod (blocks per launch); tod2map has a list of its own */
     int64_t nmlines;       /* number of 32-sample lines that touch more than one cell */
 } gmm_plan_info;
 
@@ -137,7 +140,7 @@ int gmm_plan_get_plan_mt(const gmm_plan *plan, uint64_t *out, int64_t n, int out
 int gmm_plan_check_errflags(const gmm_plan *plan, const char *where);
 /* The plan invariants that a debug=1 gmm_plan_create checks after construction, on demand:
  * entries in (cell, line) order with each pair once, line indices in range, every line present,
- * the mflag/zflag rule, and a work list covering every entry once within one cell per chunk.
+ * the mflag/zflag rule, and work lists that each cover every entry once, one cell per chunk.
  * Returns nonzero with a message counting each kind of violation. The reference asserts its
  * iterator and enumerator invariants on the device under Debug (plan_iterator.hpp:64-68, 91-103,
  * 137-141; gpu_mm_internals.hpp:224-235); this is the same role as a check that never traps. */
@@ -432,7 +435,7 @@ int gmm_plan_tester_run(const gmm_preplan *pp, const float *xpointing_gpu, int64
                         uint32_t *nmt_cumsum_cpu, uint64_t *sorted_mt_cpu, void *stream);
 
 /* test_plan_iterator, include/plan_iterator.hpp:14; src_lib/test_plan_iterator.cu:120-166.
- * Builds the operator work list for an arbitrary cell-sorted plan_mt (chunks of at most
+ * Builds a work list as the operators' are built for an arbitrary cell-sorted plan_mt (chunks of at most
  * nmt_per_block entries), walks it on the GPU with 'waves_per_block' waves per block and
  * checks that every entry is visited exactly once by a block working on its cell. */
 int gmm_test_plan_iterator(const uint64_t *plan_mt_cpu, int64_t nmt, int64_t nmt_per_block,
