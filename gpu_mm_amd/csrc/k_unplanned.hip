@@ -342,15 +342,14 @@ __device__ inline void deposit_sample(const Place &p, float t, float q, float u,
 
 // Samples that no window holds go straight to the map. Four of a lane whose footprints are within 3 x 3
 // pixels are summed in registers before ...
-template<bool Periodic>
 __device__ inline void deposit_near(const Place (&p)[4], const float (&t)[4], const float (&q)[4], const float (&u)[4],
-                                    float *__restrict__ lmap, const LocalMapView &mv, int nx, bool partial, uint32_t &err)
+                                    float *__restrict__ lmap, const LocalMapView &mv, bool partial, uint32_t &err)
 {
     const int iy = min(min(p[0].iy0, p[1].iy0), min(p[2].iy0, p[3].iy0));
     const int ix = min(min(p[0].ix0, p[1].ix0), min(p[2].ix0, p[3].ix0));
-    // The pixels' cells are those of the first and the last row and column: four lookups at once.
-    const int ix2 = (Periodic && ix + 2 >= nx) ? ix + 2 - nx : ix + 2;
-    const int64_t o00 = mv.cell(iy, ix), o01 = mv.cell(iy, ix2), o10 = mv.cell(iy + 2, ix), o11 = mv.cell(iy + 2, ix2);
+    // The pixels' cells are those of the first and the last row and column: four lookups at once. (They do not
+    // wrap: the three columns of nx - 2, nx - 1 and 0 can lie in three cells.)
+    const int64_t o00 = mv.cell(iy, ix), o01 = mv.cell(iy, ix + 2), o10 = mv.cell(iy + 2, ix), o11 = mv.cell(iy + 2, ix + 2);
 #pragma unroll 1
     for (int i = 0; i < 9; i++) {
         const int y = iy + i / 3, x = ix + i % 3;
@@ -368,11 +367,10 @@ __device__ inline void deposit_near(const Place (&p)[4], const float (&t)[4], co
             }
         }
         if (any) {
-            const int xw = (Periodic && x >= nx) ? x - nx : x;
-            const bool row = (y ^ iy) >> 6, col = (xw ^ ix) >> 6;
+            const bool row = (y ^ iy) >> 6, col = (x ^ ix) >> 6;
             int64_t o = row ? (col ? o11 : o10) : (col ? o01 : o00);
             if (o >= 0) {
-                o += mv.inside(y, xw);
+                o += mv.inside(y, x);
                 unsafeAtomicAdd(lmap + o, a);
                 unsafeAtomicAdd(lmap + o + mv.polstride, b);
                 unsafeAtomicAdd(lmap + o + 2 * mv.polstride, c);
@@ -432,7 +430,7 @@ struct QuadPlace
     uint32_t at;           // bit 2 * a + b: some sample's corner is at (mj + a, mn + b)
     int base[3];           // elements of (mj + m, mn)
     bool fast;             // the samples span more than three pixels along an axis
-    bool near;             // the footprints are within 3 x 3 pixels,
+    bool near;             // the footprints are within 3 x 3 pixels and don't wrap,
     bool fits;             // which the window holds
 };
 
@@ -465,11 +463,10 @@ __device__ inline QuadPlace place_quad(const Place (&p)[4], const Window &win, i
             hi = max(hi, k);
         }
     }
-    // x0 = nx - 1 of periodic x has its second column at x = 0.
     z.fast = max(ej - z.mj, en - z.mn) > 2;
-    z.near = ej - z.mj <= 1 && en - z.mn <= 1;
-    z.fits = z.near && j >= 0 && j + (j2 ? 2 : 1) < win.length && lo >= 0
-             && hi + (n2 ? 2 : 1) < win.width && !(Periodic && (win.xmajor ? ej : en) + 1 >= nx);
+    // x0 = nx - 1 of periodic x has its second column at x = 0.
+    z.near = ej - z.mj <= 1 && en - z.mn <= 1 && !(Periodic && (win.xmajor ? ej : en) + 1 >= nx);
+    z.fits = z.near && j >= 0 && j + (j2 ? 2 : 1) < win.length && lo >= 0 && hi + (n2 ? 2 : 1) < win.width;
     return z;
 }
 
@@ -657,7 +654,7 @@ unplanned_tod2map_kernel(float *__restrict__ lmap, const float *__restrict__ tod
                 done = ((threadIdx.x & 3) == k) ? b : done;
             }
             if (near && n > 0)
-                deposit_near<Periodic>(p, t, q, u, lmap, mv, nx, partial, err);
+                deposit_near(p, t, q, u, lmap, mv, partial, err);
             deposit_far<Periodic>(lmap, tod, xp, nsamp, base + 256 * wave, s1, done, g, mv, partial, err);
         }
     }

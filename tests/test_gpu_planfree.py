@@ -197,3 +197,24 @@ def test_planfree_tod2map_outside(gmm, orc, dev, kind, n, periodic):
     hit = np.zeros(got.shape, bool)
     hit[:, iy:iy + 2, [ix, (ix + 1) % NX]] = True
     assert np.all(np.isnan(got[hit])) and not np.any(np.isnan(got[~hit]))
+
+
+@pytest.mark.parametrize("nx", [64, 65, 66, 128, 129, 130])
+def test_planfree_tod2map_last_column(gmm, orc, dev, nx):
+    # Detectors of 16 slow samples around the column where periodic x wraps, at rows of their own, so that
+    # windows hold few of them: the last cell column may be one or two pixels wide.
+    ny, n = 2000, 300000
+    rng = np.random.default_rng(nx)
+    t, run_ = np.arange(n), np.arange(n) // 16
+    y = rng.uniform(0, ny - 4, run_[-1] + 1)[run_] + 0.1 * (t % 16)
+    x = (rng.uniform(nx - 4, nx + 2, run_[-1] + 1)[run_] + 0.07 * (t % 16)) % nx
+    xp = np.ascontiguousarray(np.stack([y, np.minimum(x, np.nextafter(F32(nx), F32(0))), 0.3 + 0.001 * t]).astype(F32))
+    tod = rng.standard_normal(n).astype(F32)
+    lp, pix = gmm.LocalPixelization.make_rectangle(ny, nx, periodic_xcoord=True), orc.Pix.rectangle(ny, nx, True)
+    ref, err = orc.tod2map(tod.astype(np.float64), xp, pix, f64=True)
+    assert err == 0
+    got = run(gmm, dev, lp, xp, tod).astype(np.float64)
+    mag, _ = orc.tod2map(np.abs(tod).astype(np.float64), np.stack([xp[0], xp[1], 0 * xp[2]]), pix, f64=True)
+    mag = np.tile(mag.reshape(3, -1)[0], 3)
+    # A pixel takes some 100 (at most 200) roundings of 6e-8 of its sum, sine, cosine and weights a few more.
+    assert np.all(np.abs(got - ref) <= 2e-5 * mag + 1e-6 * np.abs(tod).max())
